@@ -400,6 +400,113 @@ __device__ __attribute__((noinline)) void flush_own(int n, int K, int KP, int c,
   __syncthreads();   // the next chunk reads these rows
 }
 
+// Sherman-Morrison update of a walker's inverse after an accepted move (DelayedUpdate.h:166-173),
+// in one pass over its rows:
+//   Ainv[m] -= ((Ainv[m].psiV - [m == row]) / ratio) * Ainv_old[row]
+// A wave holds R rows per G-lane group in registers (a lane: Q 16-byte vectors of each row, stride
+// G), takes their dot products with psiV, and stores the updated rows, so the inverse is read and
+// written once per accept with up to R * Q vectors per lane in flight.
+// Bound: the walker's inverse travels between its one CU and L2 / the last-level cache, 2 n^2
+// elements per accept.  NiO-64 in FP64 (n = 384, 48 walkers, Metropolis): 11.9 ms per sweep; the
+// dot products and the update as two passes, one row per wave in the second, took 53.3 ms.  Eight
+// rows per group instead of four spill and take 13.3 ms.
+template <typename T, int G, int Q, int R>
+__device__ __forceinline__ void sm_update_rows(int n, int row, double rdet, const T* sPsi, const T* sInv, T* Ainv) {
+  using VT = typename V16<T>::type;
+  constexpr int VW = V16<T>::n, RG = 64 / G;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int lg = lane & (G - 1), rg = lane / G, nv = n / VW;
+  const double rinv = 1.0 / rdet;
+  VT ps[Q], iv[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int jv = lg + G * q;
+    const bool in = jv < nv;
+    ps[q] = reinterpret_cast<const VT*>(sPsi)[in ? jv : 0];
+    iv[q] = reinterpret_cast<const VT*>(sInv)[in ? jv : 0];
+#pragma unroll
+    for (int v = 0; v < VW; ++v) ps[q][v] = in ? ps[q][v] : T(0);
+  }
+  for (int m0 = wid * R * RG; m0 < n; m0 += nw * R * RG) {
+    VT a[R][Q];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const T* ar = Ainv + (size_t)min(m0 + r * RG + rg, n - 1) * n;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) a[r][q] = reinterpret_cast<const VT*>(ar)[min(lg + G * q, nv - 1)];
+    }
+    double s[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      s[r] = 0.0;
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int v = 0; v < VW; ++v) s[r] += (double)a[r][q][v] * (double)ps[q][v];
+    }
+    if constexpr (G == 64) {
+      // value i + r R/4 ends in row r of the wave (16 lanes); broadcast through scalar registers
+      wave_sums_rows<R>(s);
+      double t[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const long long b = __double_as_longlong(s[r % (R / 4)]);
+        const int src = (r / (R / 4)) * 16;
+        const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffff), src);
+        const int hi = __builtin_amdgcn_readlane((int)(b >> 32), src);
+        t[r] = __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) s[r] = t[r];
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        s[r] = dpp_add<0xB1, 0xf>(s[r]);    // sum of the lane's row of 16
+        s[r] = dpp_add<0x4E, 0xf>(s[r]);
+        s[r] = dpp_add<0x141, 0xf>(s[r]);
+        s[r] = dpp_add<0x140, 0xf>(s[r]);
+        if constexpr (G == 32) {
+          double x = s[r], y = s[r];
+          swap_rows(x, y);
+          s[r] = x + y;
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int m = m0 + r * RG + rg;
+      const T t = (T)((s[r] - (m == row ? 1.0 : 0.0)) * rinv);
+      if (m < n) {
+        VT* am = reinterpret_cast<VT*>(Ainv + (size_t)m * n);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          const int jv = lg + G * q;
+          if (jv < nv) {
+            VT x = a[r][q];
+#pragma unroll
+            for (int v = 0; v < VW; ++v) x[v] -= t * iv[q][v];
+            am[jv] = x;
+          }
+        }
+      }
+    }
+  }
+}
+// The row group: the fewest lanes that hold a row in at most four vectors each (n <= 512, the
+// workgroup's limit, always fits 64).  False when rows are not whole 16-byte vectors.
+template <typename T>
+__device__ __forceinline__ bool sm_update(int n, int row, double rdet, const T* sPsi, const T* sInv, T* Ainv) {
+  constexpr int VW = V16<T>::n;
+  if (n % VW != 0 || n / VW > 256) return false;
+  const int nv = n / VW;
+  if (nv <= 32) sm_update_rows<T, 16, 2, 4>(n, row, rdet, sPsi, sInv, Ainv);
+  else if (nv <= 48) sm_update_rows<T, 16, 3, 4>(n, row, rdet, sPsi, sInv, Ainv);
+  else if (nv <= 96) sm_update_rows<T, 32, 3, 4>(n, row, rdet, sPsi, sInv, Ainv);
+  else if (nv <= 192) sm_update_rows<T, 64, 3, 4>(n, row, rdet, sPsi, sInv, Ainv);
+  else sm_update_rows<T, 64, 4, 4>(n, row, rdet, sPsi, sInv, Ainv);
+  return true;
+}
+
 // ---- FP64 re-evaluation of a near-tie Metropolis decision (FP32 form, K > 1).
 // The determinant ratio of the move, psiV64 . x with A64 x = e_row (A64: the FP64 Slater rows
 // at the current positions, the chunk's accepted rows taken from their proposals' FP64 values),
@@ -1102,31 +1209,21 @@ __device__ __forceinline__ void moves_body(const SysP<T>& S, const BatchP<T>& B,
       }
       ++ca;
       if (!KD) {
-        // Fahy/Sherman-Morrison (DelayedUpdate.h:166-173):
-        // Ainv[m] -= ((Ainv[m].psiV - [m == row]) / ratio) * Ainv_old[row]
-        double* tm = sTm;
-        for (int m0 = wid * 4; m0 < n; m0 += nw * 4) {
-          double sm[4] = {0, 0, 0, 0};
-          const T* am = Ainv + (size_t)m0 * n;
-          const int nr = min(4, n - m0);
-          for (int j = lane; j < n; j += 64) {
-            const double pv = (double)sPsi[j];
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (r < nr) sm[r] += (double)am[(size_t)r * n + j] * pv;
+        if (!sm_update<T>(n, row, rdet, sPsi, sInv, Ainv)) {
+          // rows that are not whole 16-byte vectors: the dot products first, then the update
+          double* tm = sTm;
+          for (int m = wid; m < n; m += nw) {
+            double sm = 0;
+            for (int j = lane; j < n; j += 64) sm += (double)Ainv[(size_t)m * n + j] * (double)sPsi[j];
+            sm = wave_sum(sm);
+            if (lane == 0) tm[m] = (sm - (m == row ? 1.0 : 0.0)) / rdet;
           }
-          wave_sums_rows<4>(sm);
-          // row r of the wave holds the sum of row m0 + r
-          if ((lane & 15) == 0 && (lane >> 4) < nr) {
-            const int m = m0 + (lane >> 4);
-            tm[m] = (sm[0] - (m == row ? 1.0 : 0.0)) / rdet;
+          lds_sync();
+          for (int m = wid; m < n; m += nw) {
+            const T t = (T)tm[m];
+            T* am = Ainv + (size_t)m * n;
+            for (int j = lane; j < n; j += 64) am[j] -= t * sInv[j];
           }
-        }
-        lds_sync();
-        for (int m = wid; m < n; m += nw) {
-          const T t = (T)tm[m];
-          T* am = Ainv + (size_t)m * n;
-          for (int j = lane; j < n; j += 64) am[j] -= t * sInv[j];
         }
       } else {
         // acceptRow (DelayedUpdate.h:124-153): p_d = -V_d . psiV (d <= c) and, for the
