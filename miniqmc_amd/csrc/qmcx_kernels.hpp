@@ -13,6 +13,8 @@
 //   rows    int    [W][K]          delayed rows;  ndelay int [W]
 //   logdet, phase double [W][2]; jlog double [W][3] (J1, J2, J3)
 #pragma once
+#include <limits.h>
+
 #include "qmcx_device.hpp"
 #include "qmcx_j3.hpp"
 
@@ -645,367 +647,333 @@ __global__ __launch_bounds__(64 * kFlushWaves) void k_flush_mfma(SysP<float> S, 
 // ------------------------------------------------------------------ FP64 inverse (recompute)
 // psiM = (A^T)^-1 = transpose of A^-1 with log|det A| and its phase, the work of
 // DiracMatrix::invert_transpose (DiracMatrix.h:93-121: transpose, getrf, log det
-// from the pivots, getri).  Here: X = A^T in FP64, then an in-place blocked
-// Gauss-Jordan inversion with partial (row) pivoting.  Its pivots are the U
-// diagonal of LU with partial pivoting, so log|det| and the sign come out the
-// same way.  One workgroup per matrix; the panel of b columns (all n rows)
-// lives in LDS; the other columns get the panel's rank-b update
-//   X[i, c] <- (i in pivot rows ? 0 : Xsw[i, c]) + sum_t P[i, t] Xsw[k0 + t, c]
-// in column chunks streamed through HBM (Xsw = rows after the panel's swaps).
-// The column swaps that undo the pivoting are applied on the way out.
-constexpr int kGJChunk = 64;
-// Tiles per wave in a column chunk's update: three 16-row tiles by one 16-column tile (the waves
-// split into four column groups).  With 512 threads the kernel then needs about 150 registers, so
-// its CU keeps room for the proposals kernel's waves beside it.
-template <int NT>
-constexpr int gj_row_tiles() { return 3; }
-template <int NT>
-constexpr int gj_col_tiles() { return 1; }
-
+// from the pivots, getri).  Here: an in-place blocked Gauss-Jordan inversion of X = A^T in
+// FP64 with partial pivoting on X's rows.  Its pivots are the U diagonal of LU with partial
+// pivoting, so log|det| and the sign come out the same way.  One workgroup per matrix.
+//
+// X is kept transposed, Y[c][i] = X[i][c], so the first pass reads A as it is (and converts it)
+// and a panel of X's columns is a set of Y's rows.  No rows are exchanged: row i of X that was the
+// pivot of step k stays in place (kof[i] = k, piv[k] = i), and the permutations are applied as
+// psiM is written:  psiM[k][j] = Y[kof[j]][piv[k]].
+//
+// A panel is B columns of X in LDS (P[c][i]), factored in sub-panels of 16 columns: thread i
+// holds row i's 16 entries in registers for the 16 elimination steps; the panel's other sub-panel
+// then gets their rank-16 update, and the other columns of X the panel's rank-B update
+//   Y[c][i] <- (i a pivot row of the panel ? 0 : Y[c][i]) + sum_t Y[c][p_t] P[t][i]
+// on the FP64 matrix cores (v_mfma_f64_16x16x4f64).  A wave owns a 16-column tile of X from its
+// pivot-row entries to its last row, so the update needs no barriers, and it loads row tiles ahead
+// of the one it multiplies.
+//
+// Bound: latency of the pivot steps (0.75 us each: two barriers, the pivot search, one division)
+// and of a wave's tile; with as many matrices as CUs at n = 384 the passes over X, whose working
+// set (302 MB) exceeds the last-level cache.  n = 384: one matrix 1.10 ms, 128 at once 1.31, 256 at
+// once 1.95 (the form that exchanged rows, held 32-column panel rows in registers and streamed X in
+// 64-column chunks through LDS: 2.45, 2.49 and 2.92); n = 192: 0.29 (0.62) ms.
+constexpr int kGJSub = 16;     // columns of a sub-panel
+constexpr int kGJAhead = 4;    // row tiles in flight per wave (even)
+// LDS row stride of the panel (doubles): an odd multiple of 16, so that the four 16-lane groups of
+// a matrix operand read different banks
+__host__ __device__ inline int gj_stride(int n) { return 16 * (((n + 15) / 16) | 1); }
 struct GJLds {
-  size_t oP, oXR, oXA, oF, oPr, oRed, oRi, oPiv, oSrc, oSlot, oDl, total;
+  size_t oP, oPr, oDv, oRed, oRi, oPiv, oKof, total;
 };
 __host__ __device__ inline GJLds gj_lds_b(int n, int b) {
   GJLds L;
   size_t o = 0;
   auto take = [&](size_t bytes) { const size_t at = o; o += (bytes + 15) & ~(size_t)15; return at; };
-  L.oP = take(sizeof(double) * (size_t)n * (b + 1));      // panel, row stride b+1
-  L.oXR = take(sizeof(double) * (size_t)b * kGJChunk);   // pivot rows of a column chunk
-  L.oXA = take(sizeof(double) * (size_t)b * kGJChunk);   // rows displaced by the swaps
-  L.oF = take(sizeof(double) * (size_t)(n > b ? n : b)); // the pivot position's old row (b entries)
-  L.oPr = take(sizeof(double) * (size_t)b);              // scaled pivot row of a step
-  L.oRed = take(sizeof(double) * 16);
-  L.oRi = take(sizeof(int) * 16);
-  L.oPiv = take(sizeof(int) * (size_t)n);
-  L.oSrc = take(sizeof(int) * (size_t)n);                // row source of the panel's swaps / column source at the end
-  L.oSlot = take(sizeof(int) * (size_t)n);
-  L.oDl = take(sizeof(int) * (size_t)b);
+  L.oP = take(sizeof(double) * (size_t)b * (gj_stride(n) + 1));   // the panel; on the way out rows of stride + 1
+  L.oPr = take(sizeof(double) * 2 * kGJSub);                     // pivot row of a step (two in turn)
+  L.oDv = take(sizeof(double) * (size_t)n);                      // the pivots
+  L.oRed = take(sizeof(double) * 2 * 16);                        // per wave: best pivot candidate (two in turn)
+  L.oRi = take(sizeof(int) * 2 * 16);                            // and its row
+  L.oPiv = take(sizeof(int) * (size_t)gj_stride(n));             // row of each step's pivot
+  L.oKof = take(sizeof(int) * (size_t)gj_stride(n));             // step in which each row was the pivot
   L.total = o;
   return L;
 }
-// panel width: a thread per row (512 threads for b = 32, 1024 below), the panel within the LDS
-__host__ __device__ inline int gj_panel(int n) {
-  if (n <= 512 && gj_lds_b(n, 32).total <= 160 * 1024) return 32;
-  if (n <= 1024 && gj_lds_b(n, 16).total <= 160 * 1024) return 16;
-  return 8;
-}
+// panel width: a thread per row (512 threads for 32 columns, 1024 for 16), the panel within the LDS
+__host__ __device__ inline int gj_panel(int n) { return n <= 512 ? 32 : 16; }
 __host__ __device__ inline GJLds gj_lds(int n) { return gj_lds_b(n, gj_panel(n)); }
+
+// the rank-B update of the columns outside the panel [k0, k0 + bb); TS: TI for the first panel
+// (src = the input matrix), double after
+template <typename TS, int B>
+__device__ __forceinline__ void gj_update(int n, int ns, int k0, int bb, const TS* src, double* Y, const double* P,
+                                          const int* piv, const int* kof) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int lj = lane & 15, lg = lane >> 4;
+  const int nt = (n + 15) >> 4, ptile = k0 >> 4, np = (bb + 15) >> 4;   // tiles; the panel's tiles
+  const bool whole = (n & 15) == 0;
+  for (int idx = wid; idx < nt - np; idx += nw) {
+    const int ct = idx < ptile ? idx : idx + np;
+    // A operand, lane (j, g): column 16 ct + j of pivot row p_t, t = 4 s + g
+    double a[B / 4];
+    const TS* ac = src + (size_t)min(16 * ct + lj, n - 1) * n;
+#pragma unroll
+    for (int s = 0; s < B / 4; ++s) {
+      const int t = 4 * s + lg;
+      const double v = (double)ac[piv[k0 + min(t, bb - 1)]];
+      a[s] = t < bb ? v : 0.0;
+    }
+    // C/D register r of lane (j, g): column 16 ct + g + 4 r, row 16 it + j
+    const int c0 = 16 * ct + lg;
+    const TS* xr[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) xr[r] = src + (size_t)min(c0 + 4 * r, n - 1) * n;
+    // X entries of the next kGJAhead row tiles and the B operand (and pivot steps) of the next one
+    // are on their way while a tile is multiplied
+    TS x[kGJAhead][4];
+    double b[2][B / 4];
+    int kk[2];
+    auto load = [&](int it, TS (&v)[4]) {
+      const int i = min(16 * it + lj, n - 1);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = xr[r][i];
+    };
+    auto operand = [&](int it, double (&v)[B / 4], int& k) {
+      const int i = min(16 * it + lj, ns - 1);
+#pragma unroll
+      for (int s = 0; s < B / 4; ++s) v[s] = P[(size_t)(4 * s + lg) * ns + i];
+      k = kof[i];
+    };
+#pragma unroll
+    for (int q = 0; q < kGJAhead; ++q) load(q, x[q]);
+    operand(0, b[0], kk[0]);
+    for (int it0 = 0; it0 < nt; it0 += kGJAhead) {
+#pragma unroll
+      for (int q = 0; q < kGJAhead; ++q) {
+        const int it = it0 + q;
+        if (it < nt) {
+          f64x4 acc;
+          const bool pivot = (unsigned)(kk[q & 1] - k0) < (unsigned)bb;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[r] = pivot ? 0.0 : (double)x[q][r];
+          load(it + kGJAhead, x[q]);
+          operand(it + 1, b[(q + 1) & 1], kk[(q + 1) & 1]);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int s = 0; s < B / 4; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[q & 1][s], acc, 0, 0, 0);
+          const int i = 16 * it + lj;
+          double* yr = Y + (size_t)c0 * n + i;
+          if (whole) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) yr[(size_t)(4 * r) * n] = acc[r];
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (i < n && c0 + 4 * r < n) yr[(size_t)(4 * r) * n] = acc[r];
+          }
+        }
+      }
+    }
+  }
+}
 
 template <typename TI, typename TO, int B, int NT>
 __global__ __launch_bounds__(NT) void k_gj_invert(int n, const TI* A, TO* psiM, double* ws, double* logdet,
                                                           double* phase, int ld_stride, int mat_stride, const int* only) {
-  const int mat = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
+  const int mat = blockIdx.x, tid = threadIdx.x;
   if (only != nullptr && only[mat] == 0) return;   // only the matrices whose flag is set
-  const int lane = tid & 63, wid = tid >> 6, nw = nt >> 6;
-  const int b = B, ps = b + 1;
-  const GJLds L = gj_lds(n);
+  constexpr int nw = NT / 64, NS = B / kGJSub;
+  const int lane = tid & 63, wid = tid >> 6, lj = lane & 15, lg = lane >> 4;
+  const int ns = gj_stride(n), nt = (n + 15) >> 4;
+  const GJLds L = gj_lds_b(n, B);
   extern __shared__ __align__(16) unsigned char smem[];
   double* P = (double*)(smem + L.oP);
-  double* XR = (double*)(smem + L.oXR);
-  double* XA = (double*)(smem + L.oXA);
-  double* fcol = (double*)(smem + L.oF);
   double* prow = (double*)(smem + L.oPr);
+  double* dv = (double*)(smem + L.oDv);
   double* rv = (double*)(smem + L.oRed);
   int* ri = (int*)(smem + L.oRi);
   int* piv = (int*)(smem + L.oPiv);
-  int* src = (int*)(smem + L.oSrc);
-  int* slot = (int*)(smem + L.oSlot);
-  int* dl = (int*)(smem + L.oDl);
+  int* kof = (int*)(smem + L.oKof);
   const size_t mo = (size_t)mat * mat_stride;   // matrix slot (every mat_stride-th matrix)
-  double* X = ws + mo * 2 * n * n;
+  double* Y = ws + mo * 2 * n * n;
   const TI* a = A + mo * n * n;
+  const bool own = tid < n;
+  bool used = false;   // this thread's row has been a pivot
+  unsigned par = 0;    // parity of the wave's unused rows below each pivot (the permutation's inversions)
+  for (int i = tid; i < ns; i += NT) {
+    piv[i] = min(i, n - 1);
+    kof[i] = INT_MAX;
+  }
+  __syncthreads();
 
-  // X = A^T, b rows of A at a time through LDS (the panel buffer is free yet;
-  // b (n + 1) <= n (b + 1) doubles)
-  for (int s0 = 0; s0 < n; s0 += b) {
-    const int sb = min(b, n - s0);
-    double* T = P;   // [sb][n + 1]
-    // eight loads in flight per thread before their LDS stores
-    for (int e0 = tid; e0 < sb * n; e0 += nt * 8) {
-      double v[8];
+  for (int k0 = 0; k0 < n; k0 += B) {
+    const int bb = min(B, n - k0);
+    // ---- the panel's columns into LDS (zeros past bb)
+    {
+      double v[B];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int e = e0 + u * nt;
-        const int ec = e < sb * n ? e : 0;   // clamped: the loads stay unconditional
-        v[u] = (double)a[(size_t)(s0 + ec / n) * n + ec % n];
+      for (int c = 0; c < B; ++c) {
+        const size_t at = (size_t)(k0 + min(c, bb - 1)) * n + (own ? tid : 0);
+        v[c] = k0 == 0 ? (double)a[at] : Y[at];
       }
+      if (own)
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int e = e0 + u * nt;
-        if (e < sb * n) T[(e / n) * (n + 1) + e % n] = v[u];
+        for (int c = 0; c < B; ++c) P[(size_t)c * ns + tid] = c < bb ? v[c] : 0.0;
+    }
+#pragma unroll 1
+    for (int sp = 0; sp < NS; ++sp) {
+      const int ks = k0 + kGJSub * sp, bs = min(kGJSub, n - ks);   // the sub-panel's first step and its steps
+      if (bs <= 0) break;
+      double* Ps = P + (size_t)kGJSub * sp * ns;
+      double pr[kGJSub];
+#pragma unroll
+      for (int c = 0; c < kGJSub; ++c) pr[c] = Ps[(size_t)c * ns + (own ? tid : 0)];
+#pragma unroll
+      for (int j = 0; j < kGJSub; ++j) {
+        if (j < bs) {
+          const int k = ks + j;
+          double* pw = prow + kGJSub * (j & 1);
+          double* rw = rv + 16 * (j & 1);
+          int* iw = ri + 16 * (j & 1);
+          const double prj = pr[j];
+          // pivot: the largest |P[j][i]| of the rows not used yet, the lowest of them: the wave's
+          // largest magnitude and its first lane, then the waves' candidates side by side in the
+          // lanes of every wave.  Candidates and pivot rows alternate between two slots, so a step
+          // needs no barrier between its reads and the next step's writes
+          const double av = (own && !used) ? fabs(prj) : -1.0;
+          const double best = wave_max(av);
+          const unsigned long long hit = __ballot(av == best);
+          if (lane == 0) {
+            rw[wid] = best;
+            iw[wid] = min(wid * 64 + max(__ffsll((long long)hit) - 1, 0), n - 1);
+          }
+          lds_sync();
+          const double cv = rw[lane & (nw - 1)];
+          const int cr = iw[lane & (nw - 1)];
+          double cb = cv;
+          cb = dpp_max<0xB1, 0xf>(cb);
+          cb = dpp_max<0x4E, 0xf>(cb);
+          cb = dpp_max<0x141, 0xf>(cb);   // of eight lanes
+          if constexpr (nw > 8) cb = dpp_max<0x140, 0xf>(cb);
+          const int qb = max(__ffsll((long long)__ballot(cv == cb)) - 1, 0);   // 0 if a NaN hid the maximum
+          const int p = __builtin_amdgcn_readlane(cr, qb);                     // in [0, n)
+          const bool isp = tid == p;
+          par ^= (unsigned)__popcll(__ballot(own && !used && tid < p)) & 1u;
+          if (isp) {
+#pragma unroll
+            for (int c = 0; c < kGJSub; ++c) {
+              pw[c] = pr[c];
+              pr[c] = 0.0;
+            }
+            dv[k] = prj;
+            piv[k] = p;
+            kof[p] = k;
+            used = true;
+          }
+          const double rinv = 1.0 / cb;   // 1 / |pivot|, while the pivot row is on its way
+          lds_sync();
+          // the pivot row becomes prow / d (its entry in the pivot column 1 / d), every other row
+          // loses its multiple of it (its entry there -f / d)
+          const double dinv = pw[j] < 0.0 ? -rinv : rinv;
+          const double f = isp ? -dinv : prj * dinv;
+#pragma unroll
+          for (int c = 0; c < kGJSub; ++c)
+            if (c != j) pr[c] -= f * pw[c];
+          pr[j] = -f;
+        }
+      }
+      if (own)
+#pragma unroll
+        for (int c = 0; c < kGJSub; ++c) Ps[(size_t)c * ns + tid] = pr[c];
+      __syncthreads();
+      if (NS > 1 && bb > kGJSub) {
+        // ---- the panel's other sub-panel: P[c][i] <- (i a pivot row ? 0 : P[c][i]) + sum_t P[c][p_t] Ps[t][i]
+        double* Po = P + (size_t)kGJSub * (1 - sp) * ns;
+        double a4[kGJSub / 4];
+#pragma unroll
+        for (int s = 0; s < kGJSub / 4; ++s) {
+          const int t = 4 * s + lg;
+          const double v = Po[(size_t)lj * ns + piv[ks + min(t, bs - 1)]];
+          a4[s] = t < bs ? v : 0.0;
+        }
+        __syncthreads();
+        for (int it = wid; it < nt; it += nw) {
+          const int i = 16 * it + lj;
+          const unsigned kk = (unsigned)(kof[i] - ks);
+          f64x4 acc;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const double x = Po[(size_t)(lg + 4 * r) * ns + i];
+            acc[r] = kk < (unsigned)bs ? 0.0 : x;
+          }
+#pragma unroll
+          for (int s = 0; s < kGJSub / 4; ++s)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a4[s], Ps[(size_t)(4 * s + lg) * ns + i], acc, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) Po[(size_t)(lg + 4 * r) * ns + i] = acc[r];
+        }
+        __syncthreads();
       }
     }
-    __syncthreads();
-    for (int e = tid; e < sb * n; e += nt) {
-      const int c = e / sb, r = e % sb;   // X[c][s0 + r] = A[s0 + r][c]
-      X[(size_t)c * n + s0 + r] = T[r * (n + 1) + c];
-    }
+    // ---- the other columns, then the panel itself, back to Y
+    if (k0 == 0)
+      gj_update<TI, B>(n, ns, k0, bb, a, Y, P, piv, kof);
+    else
+      gj_update<double, B>(n, ns, k0, bb, Y, Y, P, piv, kof);
+    if (own)
+      for (int c = 0; c < bb; ++c) Y[(size_t)(k0 + c) * n + tid] = P[(size_t)c * ns + tid];
     __syncthreads();
   }
 
-  // product of the pivots' magnitudes as mantissa and binary exponent (one log at the end)
-  double pmant = 1.0;
-  int pexp = 0;
-  int sign = 1;
-  for (int k0 = 0; k0 < n; k0 += b) {
-    const int bb = min(b, n - k0);
-    // ---- panel: columns [k0, k0 + bb); thread i holds row i in registers
-    const bool own = tid < n;
-    double pr[B];
-#pragma unroll
-    for (int c = 0; c < B; ++c) pr[c] = X[(size_t)(own ? tid : 0) * n + k0 + (c < bb ? c : 0)];
-#pragma unroll
-    for (int c = 0; c < B; ++c) pr[c] = (own && c < bb) ? pr[c] : 0.0;
-    double* swp = fcol;   // old pivot-position row, for the thread that takes it
-    // Steps go in groups of four: within a group step u works on pr[u] (a register fixed at
-    // compile time), and after the group each thread's panel entries rotate four places left (all
-    // threads alike, the pivot-row copies included), so no register is picked by a runtime index
-    // and B places of rotation bring them back.
-#pragma unroll 1
-    for (int j0 = 0; j0 < bb; j0 += 4) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int j = j0 + u;
-        if (j < bb) {
-          const int k = k0 + j;
-          const double prj = pr[u];
-          // pivot: first row of largest |P[i][j]|, i >= k (idamax semantics): the wave's largest
-          // magnitude, then its first lane (rows ascend with the lanes)
-          const double av = (own && tid >= k) ? fabs(prj) : -1.0;
-          const double best = wave_max(av);
-          const unsigned long long hit = __ballot(av == best);
-          const int bi = best >= 0.0 ? wid * 64 + (__ffsll((long long)hit) - 1) : k;
-          if (lane == 0) { rv[wid] = best; ri[wid] = bi; }
-          __syncthreads();
-          // the waves' candidates side by side in the lanes of every wave: the largest
-          // magnitude, ties to the first wave (its rows are the lowest)
-          const double cv = lane < nw ? rv[lane] : -2.0;
-          const int cr = lane < nw ? ri[lane] : 0;
-          const double cbest = wave_max(cv);
-          const int qb = max(__ffsll((long long)__ballot(cv == cbest)) - 1, 0);   // 0 if a NaN hid the maximum
-          const int p = __builtin_amdgcn_readlane(cr, qb);   // in [k, n)
-          if (tid == p)
-#pragma unroll
-            for (int c = 0; c < B; ++c) prow[c] = pr[c];
-          if (tid == k && p != k)
-#pragma unroll
-            for (int c = 0; c < B; ++c) swp[c] = pr[c];
-          __syncthreads();
-          const double d = prow[u];
-          const double dinv = 1.0 / d;
-          if (tid == 0) {
-            piv[k] = p;
-            if (p != k) sign = -sign;
-            if (d < 0) sign = -sign;
-            int e;
-            pmant = frexp(pmant * fabs(d), &e);
-            pexp += e;
-          }
-          if (own) {
-            if (tid == k) {
-#pragma unroll
-              for (int c = 0; c < B; ++c) pr[c] = c == u ? dinv : prow[c] * dinv;
-            } else {
-              double f = prj;
-              if (tid == p) {
-#pragma unroll
-                for (int c = 0; c < B; ++c) pr[c] = swp[c];
-                f = swp[u];
-              }
-#pragma unroll
-              for (int c = 0; c < B; ++c) pr[c] = c == u ? -f * dinv : pr[c] - f * (prow[c] * dinv);
-            }
-          }
-        }
-      }
-      double r4[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) r4[c] = pr[c];
-#pragma unroll
-      for (int c = 0; c + 4 < B; ++c) pr[c] = pr[c + 4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) pr[B - 4 + c] = r4[c];
+  // ---- log|det| and phase: the product of the pivots as mantissa and binary exponent, the parity
+  // of the row permutation and of the negative pivots
+  {
+    double m = 1.0;
+    int ex = 0;
+    unsigned neg = lane == 0 ? par : 0u;
+    for (int k = tid; k < n; k += NT) {
+      int e;
+      const double d = dv[k];
+      m = frexp(m * fabs(d), &e);
+      ex += e;
+      neg ^= d < 0.0 ? 1u : 0u;
     }
-    // a short last panel: rotate the remaining B - 4 ceil(bb / 4) places
-    for (int j = (bb + 3) / 4 * 4; j < B; j += 4) {
-      double r4[4];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) r4[c] = pr[c];
-#pragma unroll
-      for (int c = 0; c + 4 < B; ++c) pr[c] = pr[c + 4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) pr[B - 4 + c] = r4[c];
+    for (int q = 1; q < 64; q <<= 1) {
+      int e;
+      m = frexp(m * __shfl_xor(m, q), &e);
+      ex += __shfl_xor(ex, q) + e;
+      neg ^= __shfl_xor((int)neg, q);
     }
-    if (own)
-#pragma unroll
-      for (int c = 0; c < B; ++c)
-        if (c < bb) P[tid * ps + c] = pr[c];
-    __syncthreads();
-    // ---- panel back to X; row sources of the panel's swaps; rows the swaps displaced
-    for (int e = tid; e < n * bb; e += nt) {
-      const int i = e / bb, j = e % bb;
-      X[(size_t)i * n + k0 + j] = P[i * ps + j];
-    }
-    for (int i = tid; i < n; i += nt) {
-      src[i] = i;
-      slot[i] = -1;
+    if (lane == 0) {
+      rv[wid] = m;
+      ri[wid] = ex;
+      ri[16 + wid] = (int)neg;
     }
     __syncthreads();
     if (tid == 0) {
-      for (int k = k0; k < k0 + bb; ++k) {
-        const int t = src[k];
-        src[k] = src[piv[k]];
-        src[piv[k]] = t;
+      for (int q = 1; q < nw; ++q) {
+        int e;
+        m = frexp(m * rv[q], &e);
+        ex += ri[q] + e;
+        neg ^= (unsigned)ri[16 + q];
       }
-      int nd = 0;
-      for (int k = k0; k < k0 + bb; ++k) {
-        const int p = piv[k];
-        if (p >= k0 + bb && src[p] != p && slot[p] < 0) {
-          slot[p] = nd;
-          dl[nd++] = p;
-        }
-      }
-      rv[0] = (double)nd;
-    }
-    __syncthreads();
-    const int nd = (int)rv[0];
-    // ---- rank-bb update of the other columns, kGJChunk at a time, on the FP64 matrix cores
-    // (v_mfma_f64_16x16x4f64).  A wave takes kGJRowTiles 16-row tiles (rows 16 rt .., rt =
-    // base + wr + q nrg) across kGJColTiles of the chunk's four 16-column tiles.  Operand layouts, lane
-    // (j, g) = lane j + 16 g: A (16 x 4) = P[16 rt + j][t0 + g], B (4 x 16) = XR[t0 + g][16 ct + j],
-    // C/D register r = row 16 rt + g + 4 r, column 16 ct + j (rows interleave over the lane
-    // groups, unlike the FP32 16x16x4 layout).  The wave's X values of a chunk
-    // are loaded before the chunk's pivot and displaced rows are staged, so both rounds of loads
-    // are in flight together.
-    constexpr int kGJRowTiles = gj_row_tiles<NT>(), kGJColTiles = gj_col_tiles<NT>();
-    const int nrt = (n + 15) >> 4;
-    const int lj = lane & 15, lg = lane >> 4;
-    constexpr int nrg = NT / 64 / (4 / kGJColTiles);          // waves per column group
-    const int wr = wid % nrg, ct0 = (wid / nrg) * kGJColTiles;   // row slot, first column tile
-    for (int c0 = 0; c0 < n; c0 += kGJChunk) {
-      const int cw = min(kGJChunk, n - c0);
-      if (c0 >= k0 && c0 + cw <= k0 + bb) continue;   // the chunk is the panel
-      f64x4 acc[kGJRowTiles][kGJColTiles];
-      auto load_group = [&](int base) {
-#pragma unroll
-        for (int q = 0; q < kGJRowTiles; ++q)
-#pragma unroll
-          for (int ct = 0; ct < kGJColTiles; ++ct)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int i = 16 * (base + wr + q * nrg) + lg + 4 * r, cc = 16 * (ct0 + ct) + lj;
-              const bool in = i < n && cc < cw;
-              acc[q][ct][r] = X[in ? (size_t)i * n + c0 + cc : 0];   // unconditional load, selected below
-            }
-      };
-      load_group(0);
-      for (int e0 = tid; e0 < (bb + nd) * cw; e0 += nt * 8) {
-        double v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int e = e0 + u * nt;
-          const int t = e / cw, col = c0 + e % cw;
-          const bool ok = e < (bb + nd) * cw;
-          const int srow = ok ? src[t < bb ? k0 + t : dl[t - bb]] : 0;
-          v[u] = X[(size_t)srow * n + (ok ? col : 0)];   // unconditional; panel columns never read back
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int e = e0 + u * nt;
-          const int t = e / cw, c = e % cw;
-          if (e < (bb + nd) * cw) {
-            if (t < bb) XR[t * kGJChunk + c] = v[u];
-            else XA[(t - bb) * kGJChunk + c] = v[u];
-          }
-        }
-      }
-      __syncthreads();
-      for (int base = 0; base < nrt; base += kGJRowTiles * nrg) {
-        if (base > 0) load_group(base);
-        // the base of each row: 0 for the pivot rows, the displaced row's old entries for rows a
-        // swap moved, else the row itself
-#pragma unroll
-        for (int q = 0; q < kGJRowTiles; ++q)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int i = 16 * (base + wr + q * nrg) + lg + 4 * r;
-            const int sl = i < n ? slot[i] : -1;
-            const bool prow_i = i >= k0 && i < k0 + bb;
-#pragma unroll
-            for (int ct = 0; ct < kGJColTiles; ++ct) {
-              const int cc = 16 * (ct0 + ct) + lj;
-              double x = acc[q][ct][r];
-              if (sl >= 0) x = XA[sl * kGJChunk + (cc < cw ? cc : 0)];
-              acc[q][ct][r] = prow_i ? 0.0 : x;
-            }
-          }
-        for (int t0 = 0; t0 < bb; t0 += 4) {
-          const int t = t0 + lg;
-          double av[kGJRowTiles], bv[kGJColTiles];
-#pragma unroll
-          for (int q = 0; q < kGJRowTiles; ++q) {
-            const int i = 16 * (base + wr + q * nrg) + lj;
-            av[q] = (i < n && t < bb) ? P[i * ps + t] : 0.0;
-          }
-#pragma unroll
-          for (int ct = 0; ct < kGJColTiles; ++ct) {
-            const int cc = 16 * (ct0 + ct) + lj;
-            bv[ct] = (t < bb && cc < cw) ? XR[t * kGJChunk + cc] : 0.0;
-          }
-#pragma unroll
-          for (int q = 0; q < kGJRowTiles; ++q)
-#pragma unroll
-            for (int ct = 0; ct < kGJColTiles; ++ct)
-              acc[q][ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[q], bv[ct], acc[q][ct], 0, 0, 0);
-        }
-#pragma unroll
-        for (int q = 0; q < kGJRowTiles; ++q)
-#pragma unroll
-          for (int ct = 0; ct < kGJColTiles; ++ct)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int i = 16 * (base + wr + q * nrg) + lg + 4 * r, cc = 16 * (ct0 + ct) + lj, col = c0 + cc;
-              if (i < n && cc < cw && !(col >= k0 && col < k0 + bb)) X[(size_t)i * n + col] = acc[q][ct][r];
-            }
-      }
-      __syncthreads();
+      logdet[(size_t)mat * ld_stride] = log(m) + (double)ex * 0.69314718055994530942;
+      phase[(size_t)mat * ld_stride] = neg ? M_PI : 0.0;
     }
   }
-  // ---- undo the pivoting: columns swapped back in reverse order, then out in TO
-  if (tid == 0) {
-    for (int c = 0; c < n; ++c) src[c] = c;
-    for (int k = n - 1; k >= 0; --k) {
-      const int t = src[k];
-      src[k] = src[piv[k]];
-      src[piv[k]] = t;
-    }
-    logdet[(size_t)mat * ld_stride] = log(pmant) + (double)pexp * 0.69314718055994530942;
-    phase[(size_t)mat * ld_stride] = sign > 0 ? 0.0 : M_PI;
-  }
-  __syncthreads();
-  // psiM[i][j] = X[i][src[j]], b rows at a time through LDS
+  // ---- psiM[k][j] = Y[kof[j]][piv[k]], B columns j at a time through LDS (row stride ns + 1, so
+  // the lanes' rows fall in different banks)
   TO* out = psiM + mo * n * n;
-  for (int s0 = 0; s0 < n; s0 += b) {
-    const int sb = min(b, n - s0);
-    double* T = P;   // [sb][n + 1]
-    for (int e0 = tid; e0 < sb * n; e0 += nt * 8) {
-      double v[8];
+  for (int j0 = 0; j0 < n; j0 += B) {
+    const int jb = min(B, n - j0);
+    {
+      double v[B];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int e = e0 + u * nt;
-        const int ec = e < sb * n ? e : 0;
-        v[u] = X[(size_t)(s0 + ec / n) * n + ec % n];
+      for (int c = 0; c < B; ++c) {
+        const int l = min((unsigned)kof[j0 + min(c, jb - 1)], (unsigned)(n - 1));
+        v[c] = Y[(size_t)l * n + (own ? tid : 0)];
       }
+      if (own)
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int e = e0 + u * nt;
-        if (e < sb * n) T[(e / n) * (n + 1) + e % n] = v[u];
-      }
+        for (int c = 0; c < B; ++c) P[(size_t)c * (ns + 1) + tid] = v[c];
     }
     __syncthreads();
-    for (int e = tid; e < sb * n; e += nt) {
-      const int r = e / n, j = e % n;
-      out[(size_t)(s0 + r) * n + j] = (TO)T[r * (n + 1) + src[j]];
+    for (int e = tid; e < n * B; e += NT) {
+      const int k = e / B, c = e % B;
+      if (c < jb) out[(size_t)k * n + j0 + c] = (TO)P[(size_t)c * (ns + 1) + piv[k]];
     }
     __syncthreads();
   }
@@ -1017,19 +985,14 @@ template <typename TI, typename TO>
 inline hipError_t launch_gj_invert(int n, int nmat, hipStream_t st, const TI* A, TO* psiM, double* ws,
                                    double* logdet, double* phase, int ld_stride, int mat_stride = 1,
                                    const int* only = nullptr) {
-  // one thread per row of the panel: 512 threads up to n = 448 (32 registers pairs of panel row),
-  // 1024 threads beyond
+  // a thread per row: 512 threads with panels of 32 columns, 1024 with 16 past n = 512
   const size_t lds = gj_lds(n).total;
-  const int b = gj_panel(n);
-  if (b == 32)
+  if (gj_panel(n) == 32)
     hipLaunchKernelGGL((k_gj_invert<TI, TO, 32, 512>), dim3(nmat), dim3(512), lds, st, n, A, psiM, ws, logdet, phase,
                        ld_stride, mat_stride, only);
-  else if (b == 16)
+  else
     hipLaunchKernelGGL((k_gj_invert<TI, TO, 16, 1024>), dim3(nmat), dim3(1024), lds, st, n, A, psiM, ws, logdet,
                        phase, ld_stride, mat_stride, only);
-  else
-    hipLaunchKernelGGL((k_gj_invert<TI, TO, 8, 1024>), dim3(nmat), dim3(1024), lds, st, n, A, psiM, ws, logdet, phase,
-                       ld_stride, mat_stride, only);
   return hipGetLastError();
 }
 
