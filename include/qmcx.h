@@ -202,8 +202,8 @@ int qmcx_flex_evaluate_ratios(qmcx_batch_t b, int iel, int nvp, const double* vp
  * 1 <= max_pairs <= 64; QMCX_ERR_ARG when an electron has more than max_pairs ions inside rmax. */
 int qmcx_nlpp_evaluate(qmcx_batch_t b, double rmax, const double* spheres, int max_pairs, double* ratios,
                        int* npairs);
-/* Tuning knob of qmcx_nlpp_evaluate: knots of one electron-ion pair per work unit (1, 2, 4 or 6; 0 = chosen by
- * orbital count and precision).  QMCX_ERR_ARG at evaluation when the unit's value rows do not fit a workgroup. */
+/* Tuning knob of qmcx_nlpp_evaluate: runs of knots a wave takes from the ordered knot list at a time (1, 2, 4 or 6;
+ * 0 = 1).  QMCX_ERR_ARG at evaluation when that many value rows do not fit a workgroup of 768 lanes. */
 int qmcx_batch_set_nlpp_unit(qmcx_batch_t b, int knots_per_unit);
 
 /* Per-move record of the most recent sweep, [nw][N][9]:

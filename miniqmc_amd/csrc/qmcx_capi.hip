@@ -315,10 +315,11 @@ struct qmcx_batch_s {
   double* nl_out = nullptr;       // [W][N][nl_cap][12] NonLocalPP ratios
   int* nl_cnt = nullptr;          // [W][N] electron-ion pairs inside rmax
   double* nl_near = nullptr;      // [W][N][nl_cap][4] listed pairs: distance, displacement
+  double* nl_jexp = nullptr;      // [W][N][nl_cap][12] Jastrow exponents of their knots
   int* nl_items = nullptr;        // [W*N*nl_cap] work list of listed pairs, then its length
   int nl_cap = 0;
   double* nl_sph = nullptr;       // [W][12][3] each walker's rotated quadrature knots
-  int nl_unit = 0;                // knots per NonLocalPP work unit (0: by size and precision)
+  int nl_unit = 0;                // runs of knots a wave of the ratio kernel takes at a time (0: one)
   hipStream_t stream = nullptr;
   // FP64 recompute stream: a determinant's refresh runs there, on the CUs the move
   // kernel leaves idle, while the other determinant's electrons move
@@ -531,8 +532,9 @@ constexpr int kPropWorkgroups = 1024;
 constexpr int kMaxVirtualPoints = 1 << 16;
 // electron-ion pairs per electron held by qmcx_nlpp_evaluate
 constexpr int kMaxNlppPairs = 64;
-// workgroups of the NonLocalPP ratio launch (they walk the pair list)
-constexpr int kNlppWorkgroups = 8192;
+// workgroups of the NonLocalPP ratio launch (they walk the ordered knots), a multiple of the XCDs
+constexpr int kNlppWorkgroups = 2048;
+constexpr int kNlppThreads = 768;
 
 template <typename T>
 int launch_proposals(qmcx_batch_t b, hipStream_t st, int det, int e0, int ne, uint64_t seed, double tau,
@@ -1171,74 +1173,79 @@ static int launch_virtual_ratios(qmcx_batch_t b, int iel, int nvp) {
   return 0;
 }
 
-template <typename T, int P, int PER>
-static int launch_nlpp_p(qmcx_batch_t b, double rmax, int maxp) {
+// blocks of the NonLocalPP knot order: 4 grid cells per axis, more while the blocks outnumber kNlppKeys
+constexpr int kNlppKeys = 32768;
+static NlppBlocks nlpp_blocks(const qmcx_system_s* s) {
+  NlppBlocks nb;
+  for (nb.shift = 2;; ++nb.shift) {
+    for (int d = 0; d < 3; ++d) nb.nb[d] = (s->ng[d] + (1 << nb.shift) - 1) >> nb.shift;
+    if ((long long)nb.nb[0] * nb.nb[1] * nb.nb[2] <= kNlppKeys) return nb;
+  }
+}
+
+// LK lanes per knot with Q 16-byte orbital groups each; take: runs of 64 / LK knots a wave takes at a time
+template <typename T, int LK, int Q>
+static int launch_nlpp_ratios(qmcx_batch_t b, int maxp, int take, const int* units, const int* cnt) {
   const qmcx_system_s* s = b->sys;
-  const int WN = b->W * s->N;
-  // nl_items: work list [WN*maxp], its length, per-key counts and cursors [M*kNlppRadialBins each],
-  // pair keys [WN*maxp]
-  const int nkeys = s->nions * kNlppRadialBins;
-  int* count = b->nl_items + (size_t)WN * maxp;
-  int* icnt = count + 1;
-  int* icur = icnt + nkeys;
-  int* pkey = icur + nkeys;
-  hipLaunchKernelGGL(k_zero_ints, dim3(4), dim3(256), 0, b->stream, icnt, nkeys);
-  hipLaunchKernelGGL(k_nlpp_pairs<T>, dim3((WN + 255) / 256), dim3(256), 0, b->stream, s->params<T>(), b->params<T>(),
-                     rmax, maxp, b->nl_near, pkey, b->nl_cnt, icnt);
-  hipLaunchKernelGGL(k_nlpp_offsets, dim3(1), dim3(256), 0, b->stream, icnt, icur, nkeys, count);
-  hipLaunchKernelGGL(k_nlpp_scatter, dim3((WN + 255) / 256), dim3(256), 0, b->stream, WN, maxp, b->nl_cnt, pkey, icur,
-                     b->nl_items);
-  constexpr int SL = 16 / PER;
-  const int nq = s->npad / (16 / (int)sizeof(T));
-  const int nt = std::max(64, (P * SL * nq + 63) / 64 * 64);
-  const size_t lds = sizeof(T) * (size_t)P * SL * s->npad + sizeof(double) * 3 * P * 16;
-  // workgroups walk the work list (P knots of a pair per unit); its length is only known on the device
-  const int grid = (std::max(1, std::min(WN * maxp * (kNlppKnots / P), kNlppWorkgroups)) + 7) / 8 * 8;
-  if (b->j3)
-    hipLaunchKernelGGL((k_nlpp_ratios<T, P, PER, true>), dim3(grid), dim3(nt), lds, b->stream, s->params<T>(),
-                       b->params<T>(), b->nl_sph, maxp, b->nl_near, b->nl_items, count, b->nl_out);
-  else
-    hipLaunchKernelGGL((k_nlpp_ratios<T, P, PER, false>), dim3(grid), dim3(nt), lds, b->stream, s->params<T>(),
-                       b->params<T>(), b->nl_sph, maxp, b->nl_near, b->nl_items, count, b->nl_out);
+  const int grid = kNlppWorkgroups;   // they walk the ordered knots; their number is only known on the device
+  hipLaunchKernelGGL((k_nlpp_ratios<T, LK, Q>), dim3(grid), dim3(256), 0, b->stream, s->params<T>(), b->params<T>(),
+                     b->nl_sph, maxp, b->nl_near, b->nl_items, units, cnt, b->nl_jexp, take, b->nl_out);
   HIPCHK(hipGetLastError());
   return 0;
 }
 
-// Work-unit shape: P knots of a pair per unit, PER of the 16 stencil columns per lane.  With the
-// shared sphere of an earlier form, NiO-64 (384 orbitals, 128 walkers, 33k electron-ion pairs) ran
-// fastest in FP32 at one knot per unit with two stencil slices, and in FP64 with the most knots
-// whose value rows fit (four).  `unit` (qmcx_batch_set_nlpp_unit) forces P.
 template <typename T>
 static int launch_nlpp(qmcx_batch_t b, double rmax, int maxp) {
-  const int nq = b->sys->npad / (16 / (int)sizeof(T));
+  const qmcx_system_s* s = b->sys;
+  const int nq = s->npad / (16 / (int)sizeof(T));
+  // `unit` (qmcx_batch_set_nlpp_unit) is limited to the value rows of a workgroup of kNlppThreads lanes
   const int unit = b->nl_unit;
-  auto fits = [&](int p, int per) { return p * (16 / per) * nq <= kNlppThreads; };
-  if (unit == 0) {
-    if (sizeof(T) == 4 && fits(1, 8)) return launch_nlpp_p<T, 1, 8>(b, rmax, maxp);
-    if (fits(6, 16)) return launch_nlpp_p<T, 6, 16>(b, rmax, maxp);
-    if (fits(4, 16)) return launch_nlpp_p<T, 4, 16>(b, rmax, maxp);
-    if (fits(2, 16)) return launch_nlpp_p<T, 2, 16>(b, rmax, maxp);
-    if (fits(1, 16)) return launch_nlpp_p<T, 1, 16>(b, rmax, maxp);
-    return fail(QMCX_ERR_ARG, "spline row does not fit a workgroup");
-  }
-  switch (unit) {
-    case 1:
-      if (fits(1, 8)) return launch_nlpp_p<T, 1, 8>(b, rmax, maxp);
-      if (fits(1, 16)) return launch_nlpp_p<T, 1, 16>(b, rmax, maxp);
-      break;
-    case 2:
-      if (fits(2, 16)) return launch_nlpp_p<T, 2, 16>(b, rmax, maxp);
-      break;
-    case 4:
-      if (fits(4, 16)) return launch_nlpp_p<T, 4, 16>(b, rmax, maxp);
-      break;
-    case 6:
-      if (fits(6, 16)) return launch_nlpp_p<T, 6, 16>(b, rmax, maxp);
-      break;
-    default:
-      break;
-  }
-  return fail(QMCX_ERR_ARG, "NonLocalPP work unit of " + std::to_string(unit) + " knots does not fit a workgroup");
+  if ((unit > 0 ? unit : 1) * nq > kNlppThreads)
+    return fail(QMCX_ERR_ARG, unit > 0 ? "NonLocalPP work unit of " + std::to_string(unit) + " knots does not fit a workgroup"
+                                       : "spline row does not fit a workgroup");
+  const int WN = b->W * s->N;
+  // nl_items: pair list [WN*maxp], its length, per-key counts and cursors, the knots' keys and the
+  // ordered knots [WN*maxp*12 each]
+  const NlppBlocks nb = nlpp_blocks(s);
+  const int nkeys = nb.keys();
+  const size_t cap = (size_t)WN * maxp;
+  int* cnt = b->nl_items + cap;
+  int* kcnt = cnt + 1;
+  int* kcur = kcnt + nkeys;
+  int* ukey = kcur + nkeys;
+  int* units = ukey + cap * kNlppKnots;
+  const SysP<T> S = s->params<T>();
+  const BatchP<T> B = b->params<T>();
+  hipLaunchKernelGGL(k_zero_ints, dim3(16), dim3(256), 0, b->stream, cnt, 1 + nkeys);
+  hipLaunchKernelGGL(k_nlpp_pairs<T>, dim3((WN + 255) / 256), dim3(256), 0, b->stream, S, B, rmax, maxp, b->nl_near,
+                     b->nl_items, b->nl_cnt, cnt);
+  // about eight workgroups per CU over the walkers, a wave for at least four electrons
+  const int parts = std::max(1, std::min((s->N + 15) / 16, 2048 / b->W));
+  const size_t jlds = nlpp_jastrow_lds<T>(s->N, s->nions);
+  if (b->j3)
+    hipLaunchKernelGGL((k_nlpp_jastrow<T, true>), dim3(parts, b->W), dim3(256), jlds, b->stream, S, B, b->nl_sph, maxp,
+                       b->nl_near, b->nl_cnt, b->nl_jexp);
+  else
+    hipLaunchKernelGGL((k_nlpp_jastrow<T, false>), dim3(parts, b->W), dim3(256), jlds, b->stream, S, B, b->nl_sph, maxp,
+                       b->nl_near, b->nl_cnt, b->nl_jexp);
+  const int kgrid = (int)std::min<size_t>((cap * kNlppKnots + 255) / 256, 1024);
+  hipLaunchKernelGGL(k_nlpp_keys<T>, dim3(kgrid), dim3(256), 0, b->stream, S, B, b->nl_sph, maxp, b->nl_near,
+                     b->nl_items, cnt, nb, ukey, kcnt);
+  hipLaunchKernelGGL(k_nlpp_offsets, dim3(1), dim3(1024), 0, b->stream, kcnt, kcur, nkeys);
+  hipLaunchKernelGGL(k_nlpp_scatter, dim3(kgrid), dim3(256), 0, b->stream, cnt, ukey, kcur, units);
+  HIPCHK(hipGetLastError());
+  // the fewest lanes per knot that hold its orbitals in at most three groups each (four past 192
+  // groups): a wave then works on several knots of a small system, and no lane idles at NiO-64
+  const int take = unit > 0 ? unit : 1;
+  if (nq <= 16) return launch_nlpp_ratios<T, 16, 1>(b, maxp, take, units, cnt);
+  if (nq <= 32) return launch_nlpp_ratios<T, 16, 2>(b, maxp, take, units, cnt);
+  if (nq <= 64) return launch_nlpp_ratios<T, 32, 2>(b, maxp, take, units, cnt);
+  if (nq <= 96) return launch_nlpp_ratios<T, 32, 3>(b, maxp, take, units, cnt);
+  if (nq <= 128) return launch_nlpp_ratios<T, 64, 2>(b, maxp, take, units, cnt);
+  if (nq <= 192) return launch_nlpp_ratios<T, 64, 3>(b, maxp, take, units, cnt);
+  if (nq <= 256) return launch_nlpp_ratios<T, 64, 4>(b, maxp, take, units, cnt);
+  if (nq <= 512) return launch_nlpp_ratios<T, 64, 8>(b, maxp, take, units, cnt);
+  return launch_nlpp_ratios<T, 64, 12>(b, maxp, take, units, cnt);
 }
 
 extern "C" {
@@ -1720,6 +1727,7 @@ int qmcx_batch_destroy(qmcx_batch_t b) {
   if (b->nl_out) hipFree(b->nl_out);
   if (b->nl_cnt) hipFree(b->nl_cnt);
   if (b->nl_near) hipFree(b->nl_near);
+  if (b->nl_jexp) hipFree(b->nl_jexp);
   if (b->nl_items) hipFree(b->nl_items);
   if (b->nl_sph) hipFree(b->nl_sph);
   // the streams are the device's shared ones and stay
@@ -2145,14 +2153,16 @@ int qmcx_nlpp_evaluate(qmcx_batch_t b, double rmax, const double* spheres, int m
     b->nl_cnt = nullptr;
     b->nl_cap = 0;
     if (b->nl_near) hipFree(b->nl_near);
+    if (b->nl_jexp) hipFree(b->nl_jexp);
     if (b->nl_items) hipFree(b->nl_items);
-    b->nl_near = nullptr;
+    b->nl_near = b->nl_jexp = nullptr;
     b->nl_items = nullptr;
     HIPCHK(hipMalloc(&b->nl_out, sizeof(double) * WN * max_pairs * kNlppKnots));
     HIPCHK(hipMalloc(&b->nl_cnt, sizeof(int) * WN));
     HIPCHK(hipMalloc(&b->nl_near, sizeof(double) * 4 * WN * max_pairs));
+    HIPCHK(hipMalloc(&b->nl_jexp, sizeof(double) * WN * max_pairs * kNlppKnots));
     HIPCHK(hipMalloc(&b->nl_items,
-                     sizeof(int) * (2 * WN * max_pairs + 1 + 2 * (size_t)b->sys->nions * kNlppRadialBins)));
+                     sizeof(int) * (WN * max_pairs * (1 + 2 * kNlppKnots) + 1 + 2 * (size_t)kNlppKeys)));
     b->nl_cap = max_pairs;
   }
   if (!b->nl_sph) HIPCHK(hipMalloc(&b->nl_sph, sizeof(double) * 3 * kNlppKnots * (size_t)b->W));
@@ -2160,12 +2170,23 @@ int qmcx_nlpp_evaluate(qmcx_batch_t b, double rmax, const double* spheres, int m
                         b->stream));
   const int rc = b->prec == QMCX_FP32 ? launch_nlpp<float>(b, rmax, max_pairs) : launch_nlpp<double>(b, rmax, max_pairs);
   if (rc) return rc;
-  std::vector<int> cnt(WN);
+  std::vector<int> cnt(WN), items;
+  std::vector<double> rat;
+  int listed = 0;
   HIPCHK(hipMemcpyAsync(cnt.data(), b->nl_cnt, sizeof(int) * WN, hipMemcpyDeviceToHost, b->stream));
-  if (ratios)
-    HIPCHK(hipMemcpyAsync(ratios, b->nl_out, sizeof(double) * WN * max_pairs * kNlppKnots, hipMemcpyDeviceToHost,
-                          b->stream));
+  HIPCHK(hipMemcpyAsync(&listed, b->nl_items + WN * max_pairs, sizeof(int), hipMemcpyDeviceToHost, b->stream));
   HIPCHK(hipStreamSynchronize(b->stream));
+  if (ratios && listed > 0) {
+    // the listed pairs' ratios to their places; the other slots stay as they were
+    items.resize(listed);
+    rat.resize((size_t)listed * kNlppKnots);
+    HIPCHK(hipMemcpyAsync(items.data(), b->nl_items, sizeof(int) * listed, hipMemcpyDeviceToHost, b->stream));
+    HIPCHK(hipMemcpyAsync(rat.data(), b->nl_out, sizeof(double) * rat.size(), hipMemcpyDeviceToHost, b->stream));
+    HIPCHK(hipStreamSynchronize(b->stream));
+    for (int i = 0; i < listed; ++i)
+      std::memcpy(ratios + (size_t)items[i] * kNlppKnots, rat.data() + (size_t)i * kNlppKnots,
+                  sizeof(double) * kNlppKnots);
+  }
   if (npairs) std::copy(cnt.begin(), cnt.end(), npairs);
   for (size_t i = 0; i < WN; ++i)
     if (cnt[i] > max_pairs) return fail(QMCX_ERR_ARG, "more ions within rmax of an electron than max_pairs");

@@ -357,6 +357,19 @@ __device__ inline T min_image_ortho(const Cell<T>& C, T d0, T d1, T d2, T flip, 
     return sqrt(x * x + y * y + z * z);
 }
 
+// The distance of min_image_ortho with a correctly rounded square root (for sums of values alone).
+template <typename T>
+__device__ inline T image_distance_ortho(const Cell<T>& C, T d0, T d1, T d2) {
+  const T f0 = d0 * C.g[0] + d1 * C.g[3] + d2 * C.g[6];
+  const T f1 = d0 * C.g[1] + d1 * C.g[4] + d2 * C.g[7];
+  const T f2 = d0 * C.g[2] + d1 * C.g[5] + d2 * C.g[8];
+  const T s0 = rint(f0), s1 = rint(f1), s2 = rint(f2);   // whole cells to the nearest image
+  const T x = d0 - (s0 * C.rb[0] + s1 * C.rb[3] + s2 * C.rb[6]);
+  const T y = d1 - (s0 * C.rb[1] + s1 * C.rb[4] + s2 * C.rb[7]);
+  const T z = d2 - (s0 * C.rb[2] + s1 * C.rb[5] + s2 * C.rb[8]);
+  return sqrt(x * x + y * y + z * z);
+}
+
 // ------------------------------------------------------------------ spline location
 // toUnit_floor with the SPO lattice, then the grid cell and fraction per axis
 // (CrystalLattice.h:185-196, MultiBsplineEvalHelper.hpp:43-64); kept in FP64.

@@ -1306,21 +1306,21 @@ __global__ __launch_bounds__(1024) void k_virtual_ratios(SysP<T> S, BatchP<T> B,
 }
 
 // NonLocalPP::evaluate (NonLocalPP.hpp:115-140) for every electron of every walker.
-// k_nlpp_pairs: one lane per (walker, electron) lists the ions within rmax in ion order
-// (minimum image, ion - electron as the BA table's displacement) into
-// near[(w*N + e)*maxp + p][4] = dist, displacement and pkey[...] = ion * kNlppRadialBins + the
-// distance's bin in [0, rmax), counts them in npairs[w][e] (the full count, also beyond maxp) and
-// per key in icnt[key].  k_nlpp_offsets and k_nlpp_scatter order the listed pairs by key into the
-// work list items[] (count[0] entries).  k_nlpp_ratios walks knot-major over that list, each
-// XCD over a contiguous run of ion keys.  Every walker has its own randomly rotated knots
-// (spheres[w][12][3], one rotation per walker and evaluation as the reference's per-mover
-// NonLocalPP::randomize, NonLocalPP.hpp:100-113, miniqmc.cpp:470); knot k of a pair sits at
-// dist * spheres[w][k] + displ + r_e (NonLocalPP.hpp:133); ratios[w][e][maxp][kNlppKnots].
+// k_nlpp_pairs: one lane per (walker, electron) finds the ions within rmax in ion order (minimum
+// image, ion - electron as the BA table's displacement), counts them in npairs[w][e] (the full
+// count, also beyond maxp) and lists the first maxp: near[item][4] = distance, displacement of item =
+// (w*N + e)*maxp + p, items[pos] = item in the order of arrival, cnt[0] = listed pairs.  Knot k of a
+// pair sits at dist * spheres[w][k] + displ + r_e (NonLocalPP.hpp:133; every walker has its own
+// randomly rotated knots, one rotation per walker and evaluation as the reference's per-mover
+// NonLocalPP::randomize, NonLocalPP.hpp:100-113, miniqmc.cpp:470).
+// k_nlpp_jastrow: the Jastrow exponents of the listed pairs' knots, jexp[item][12], walker by walker
+// (its positions and the functors in LDS, a wave per pair, lanes over the electrons).
+// k_nlpp_keys, k_nlpp_offsets and k_nlpp_scatter order all the knots (unit = pos * 12 + knot) by the
+// block of spline grid cells they fall in, and k_nlpp_ratios walks that order, each XCD over a
+// contiguous eighth of it: knots whose stencils overlap run at the same time on CUs that share an
+// L2, so the orbital table is read from HBM about once instead of once per knot.  ratios[pos][12] =
+// (value row . inverse row) exp(jexp).
 constexpr int kNlppKnots = 12;
-constexpr int kNlppRadialBins = 16;
-struct NlppKnots {
-  double p[kNlppKnots][3];
-};
 
 __global__ void k_zero_ints(int* p, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
@@ -1328,9 +1328,10 @@ __global__ void k_zero_ints(int* p, int n) {
 
 template <typename T>
 __global__ __launch_bounds__(256) void k_nlpp_pairs(SysP<T> S, BatchP<T> B, double rmax, int maxp, double* near,
-                                                    int* pkey, int* npairs, int* icnt) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x, N = S.N, M = S.M;
-  if (idx >= B.W * N) return;
+                                                    int* items, int* npairs, int* cnt) {
+  const int at = blockIdx.x * blockDim.x + threadIdx.x, N = S.N;
+  const bool live = at < B.W * N;
+  const int idx = live ? at : 0, M = live ? S.M : 0;
   const int w = idx / N, e = idx - w * N;
   const Cell<T> C = *S.cell;
   const double* R = B.R + (size_t)w * 3 * N;
@@ -1347,152 +1348,284 @@ __global__ __launch_bounds__(256) void k_nlpp_pairs(SysP<T> S, BatchP<T> B, doub
         q[1] = (double)dx;
         q[2] = (double)dy;
         q[3] = (double)dz;
-        const int bin = (int)((double)r / rmax * kNlppRadialBins);
-        const int key = ci * kNlppRadialBins + (bin < kNlppRadialBins - 1 ? bin : kNlppRadialBins - 1);
-        pkey[(size_t)idx * maxp + c] = key;
-        atomicAdd(icnt + key, 1);
       }
       ++c;
     }
   }
-  npairs[idx] = c;
+  if (live) npairs[idx] = c;
+  // the workgroup's pairs take one run of the list
+  const int m = live ? min(c, maxp) : 0, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  int inc = m;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int t = __shfl_up(inc, d);
+    if (lane >= d) inc += t;
+  }
+  __shared__ int tot[4], base;
+  if (lane == 63) tot[wid] = inc;
+  __syncthreads();
+  if (threadIdx.x == 0) base = atomicAdd(cnt, tot[0] + tot[1] + tot[2] + tot[3]);
+  __syncthreads();
+  int pos = base + inc - m;
+  for (int q = 0; q < wid; ++q) pos += tot[q];
+  for (int p = 0; p < m; ++p) items[pos + p] = idx * maxp + p;
 }
 
-// exclusive prefix of the per-key counts into the per-key cursors; count[0] = listed pairs.
-// One workgroup of 256 lanes: each lane sums a contiguous run of keys, lane 0 scans the 256 run
-// sums in LDS, and each lane writes its run's cursors.
-__global__ __launch_bounds__(256) void k_nlpp_offsets(const int* icnt, int* icur, int nkeys, int* count) {
-  __shared__ int run[256];
-  const int t = threadIdx.x, per = (nkeys + 255) / 256, a = t * per;
-  const int b = a + per < nkeys ? a + per : nkeys;
+// Blocks of 2^shift grid cells per axis, nb blocks per axis: the key of a knot is its block's index
+struct NlppBlocks {
+  int shift, nb[3];
+  __host__ __device__ int keys() const { return nb[0] * nb[1] * nb[2]; }
+};
+// the point of unit u (pair u / 12, knot u % 12); w, e: the pair's walker and electron
+template <typename T>
+__device__ inline void nlpp_point(const SysP<T>& S, const BatchP<T>& B, const double* spheres, int maxp,
+                                  const double* near, const int* items, int u, int& w, int& e, double p[3]) {
+  const int pos = u / kNlppKnots, k = u - pos * kNlppKnots, N = S.N;
+  const int item = items[pos], idx = item / maxp;
+  w = idx / N;
+  e = idx - w * N;
+  const double* R = B.R + (size_t)w * 3 * N;
+  const double* sp = spheres + ((size_t)w * kNlppKnots + k) * 3;
+  const double* q = near + (size_t)item * 4;
+  const double d = q[0];
+  const double ox = R[e] + q[1], oy = R[N + e] + q[2], oz = R[2 * N + e] + q[3];
+  p[0] = d * sp[0] + ox;
+  p[1] = d * sp[1] + oy;
+  p[2] = d * sp[2] + oz;
+}
+template <typename T>
+__global__ __launch_bounds__(256) void k_nlpp_keys(SysP<T> S, BatchP<T> B, const double* spheres, int maxp,
+                                                   const double* near, const int* items, const int* cnt,
+                                                   NlppBlocks nb, int* ukey, int* kcnt) {
+  const int nu = cnt[0] * kNlppKnots;
+  for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nu; u += gridDim.x * blockDim.x) {
+    int w, e, ix[3];
+    double p[3], t[3];
+    nlpp_point(S, B, spheres, maxp, near, items, u, w, e, p);
+    spline_locate(S.spoG, S.ng, p[0], p[1], p[2], ix, t);
+    const int key = ((ix[0] >> nb.shift) * nb.nb[1] + (ix[1] >> nb.shift)) * nb.nb[2] + (ix[2] >> nb.shift);
+    ukey[u] = key;
+    atomicAdd(kcnt + key, 1);
+  }
+}
+
+// Exclusive prefix of the per-key counts into the per-key cursors.  One workgroup of 1024 lanes:
+// each lane sums a contiguous run of keys, the run sums are scanned, each lane writes its cursors.
+__global__ __launch_bounds__(1024) void k_nlpp_offsets(const int* kcnt, int* kcur, int nkeys) {
+  __shared__ int run[16];
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6, per = (nkeys + 1023) / 1024, a = min(t * per, nkeys);
+  const int b = min(a + per, nkeys);
   int s = 0;
-  for (int c = a; c < b; ++c) s += icnt[c];
-  run[t] = s;
-  __syncthreads();
-  if (t == 0) {
-    int acc = 0;
-    for (int i = 0; i < 256; ++i) {
-      const int v = run[i];
-      run[i] = acc;
-      acc += v;
-    }
-    count[0] = acc;
+  for (int c = a; c < b; ++c) s += kcnt[c];
+  int x = s;   // inclusive scan of the wave's run sums
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(x, d);
+    if (lane >= d) x += y;
   }
+  if (lane == 63) run[wid] = x;
   __syncthreads();
-  int o = run[t];
+  int o = x - s;
+  for (int q = 0; q < wid; ++q) o += run[q];
   for (int c = a; c < b; ++c) {
-    icur[c] = o;
-    o += icnt[c];
+    kcur[c] = o;
+    o += kcnt[c];
   }
 }
 
-__global__ __launch_bounds__(256) void k_nlpp_scatter(int WN, int maxp, const int* npairs, const int* pkey, int* icur,
-                                                      int* items) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= WN) return;
-  const int c = npairs[idx] < maxp ? npairs[idx] : maxp;
-  for (int p = 0; p < c; ++p) items[atomicAdd(icur + pkey[(size_t)idx * maxp + p], 1)] = idx * maxp + p;
+__global__ __launch_bounds__(256) void k_nlpp_scatter(const int* cnt, const int* ukey, int* kcur, int* units) {
+  const int nu = cnt[0] * kNlppKnots;
+  for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nu; u += gridDim.x * blockDim.x)
+    units[atomicAdd(kcur + ukey[u], 1)] = u;
 }
 
-// A work unit is P of a pair's twelve knots.  Lanes [g*L, (g+1)*L), L = (16/PER)*nq, gather
-// knot g's value row (a lane: one 16-byte orbital group, PER of the 16 stencil columns), then
-// every lane takes a share of the P dot products and of the P Jastrow sums, reading each
-// electron's position once for all P knots.  J3: the system has a three-body Jastrow (its sums
-// at the knots join the J2 sums, as both enter the exponent alike).
-constexpr int kNlppThreads = 768;
-template <typename T, int P, int PER, bool J3>
-__global__ __launch_bounds__(kNlppThreads) void k_nlpp_ratios(SysP<T> S, BatchP<T> B, const double* spheres, int maxp,
-                                                              const double* near, const int* items, const int* count,
-                                                              double* ratios) {
-  constexpr int SL = 16 / PER, KG = kNlppKnots / P;
+// J1, J2 (and J3) exponents of every listed pair's knots: sums at the electron's position (kept by the
+// moves) less those at the knot (OneBodyJastrow.h:136-140, TwoBodyJastrow.h:103-107,
+// ThreeBodyJastrow.h:262-273).  grid (parts, W): a workgroup stages its walker's positions, the ions,
+// functors and cell in LDS; its waves take electrons part * 4 + wave, + 4 parts, ...; a wave takes
+// four of a pair's knots at a time, so a position is read once for the four.
+// Bound: vector arithmetic, (N + M) image distances per knot.  NiO-64, 128 walkers, 396k knots: 0.92 ms
+// in FP32 (it was part of the ratio kernel, where it waited for global loads of positions and
+// functors).
+constexpr int kNlppTake = 4;
+template <typename T>
+__host__ __device__ inline size_t nlpp_jastrow_lds(int N, int M) {
+  return sizeof(double) * 3 * (size_t)(N + M) + sizeof(Functor<T>) * (kMaxSpecies + 2) + sizeof(Cell<T>) + 64;
+}
+template <typename T, bool J3>
+__global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, const double* spheres, int maxp,
+                                                      const double* near, const int* npairs, double* jexp) {
   extern __shared__ __align__(16) unsigned char smem[];
-  T* part = (T*)smem;                                        // [P][SL][npad]
-  double* red = (double*)(part + (size_t)P * SL * S.npad);   // [3P][16]
-  const int N = S.N, n = S.n, M = S.M;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const Cell<T> C = *S.cell;
-  const int L = SL * (S.npad / V16<T>::n);
-  const int g = tid / L;
-  // XCD-aware walk: workgroup b runs on XCD b % 8, and XCD x takes the x-th eighth of the
-  // knot-major units, so each XCD's L2 sees a contiguous run of keys (gridDim.x % 8 == 0)
-  const int nitems = count[0];
-  const int nunits = nitems * KG;
-  const int xcd = blockIdx.x & 7, per = gridDim.x >> 3;
-  const int lo = (int)((long long)nunits * xcd / 8), hi = (int)((long long)nunits * (xcd + 1) / 8);
-  for (int un = lo + (int)(blockIdx.x >> 3); un < hi; un += per) {
-    const int kg = un / nitems;
-    const int item = items[un - kg * nitems];
-    const int k0 = kg * P;
-    const int idx = item / maxp;
-    const int w = idx / N, e = idx - w * N;
-    const double* R = B.R + (size_t)w * 3 * N;
-    const double* sp = spheres + (size_t)w * 3 * kNlppKnots;   // this walker's knots
-    const double* q = near + (size_t)item * 4;
-    const double d = q[0];
-    const double ox = R[e] + q[1], oy = R[N + e] + q[2], oz = R[2 * N + e] + q[3];
-    const int det = e < n ? 0 : 1, row = e - det * n;
-    const T* arow = B.Ainv + ((size_t)w * 2 + det) * n * n + (size_t)row * n;
+  const int w = blockIdx.y, N = S.N, n = S.n, M = S.M, tid = threadIdx.x, nt = blockDim.x;
+  const int lane = tid & 63, wid = tid >> 6, nw = nt >> 6;
+  double* sR = (double*)smem;
+  double* sI = sR + 3 * N;
+  Functor<T>* sFn = (Functor<T>*)(smem + ((sizeof(double) * 3 * (size_t)(N + M) + 15) & ~(size_t)15));
+  Cell<T>* sCell = (Cell<T>*)(sFn + kMaxSpecies + 2);
+  for (int i = tid; i < 3 * N; i += nt) sR[i] = B.R[(size_t)w * 3 * N + i];
+  for (int i = tid; i < 3 * M; i += nt) sI[i] = S.ions[i];
+  for (int i = tid; i < (int)(sizeof(Functor<T>) * (kMaxSpecies + 2) / 4); i += nt) ((int*)sFn)[i] = ((const int*)S.fn)[i];
+  for (int i = tid; i < (int)(sizeof(Cell<T>) / 4); i += nt) ((int*)sCell)[i] = ((const int*)S.cell)[i];
+  __syncthreads();
+  const Cell<T>& C = *sCell;
+  const bool ortho = C.ortho != T(0);
+  auto value = [&](const Functor<T>& f, T dx, T dy, T dz) -> double {
+    T ox, oy, oz;
+    const T r = ortho ? image_distance_ortho(C, -dx, -dy, -dz) : min_image(C, dx, dy, dz, T(-1), ox, oy, oz);
+    const bool in = r < f.rcut;   // an interior radius keeps the lookup in range
+    const T u = functor_v(f, in ? r : f.rcut * T(0.5));
+    return in ? (double)u : 0.0;
+  };
+  for (int e = blockIdx.x * nw + wid; e < N; e += gridDim.x * nw) {
+    const size_t idx = (size_t)w * N + e;
+    const int np = min(npairs[idx], maxp);
+    if (np == 0) continue;
     const size_t o = (size_t)w * 5 * N + e;
     const double j1o = (double)B.J1[o], j2o = (double)B.J2[o] + (J3 ? (double)B.J3[o] : 0.0);
     const bool up = e < n;
-    double* out = ratios + (size_t)item * kNlppKnots;
-    {
-      if (g < P) {
-        const int k = k0 + g;
-        spline_gather<T, 1, PER>(S, S.spoG, d * sp[3 * k] + ox, d * sp[3 * k + 1] + oy, d * sp[3 * k + 2] + oz,
-                                 part + (size_t)g * SL * S.npad, tid - g * L);
-      }
-      double v[3 * P];   // det ratios, J1 sums, J2 (+ J3) sums of the P knots
+    for (int p = 0; p < np; ++p) {
+      const size_t item = idx * maxp + p;
+      const double* q = near + item * 4;
+      const double d = q[0], ox = sR[e] + q[1], oy = sR[N + e] + q[2], oz = sR[2 * N + e] + q[3];
+      for (int k0 = 0; k0 < kNlppKnots; k0 += kNlppTake) {
+        const double* sp = spheres + ((size_t)w * kNlppKnots + k0) * 3;
+        double px[kNlppTake], py[kNlppTake], pz[kNlppTake], v[2 * kNlppTake];
 #pragma unroll
-      for (int i = 0; i < 3 * P; ++i) v[i] = 0.0;
-      T dx, dy, dz;   // the values only: each knot needs u, not its derivatives
-      for (int ci = tid; ci < M; ci += nt) {
-        const Functor<T>& f = S.fn[S.species[ci]];
-        if (f.ncoef == 0) continue;
-        const double ix = S.ions[ci], iy = S.ions[M + ci], iz = S.ions[2 * M + ci];
-#pragma unroll
-        for (int gg = 0; gg < P; ++gg) {
-          const double px = d * sp[3 * (k0 + gg)] + ox, py = d * sp[3 * (k0 + gg) + 1] + oy, pz = d * sp[3 * (k0 + gg) + 2] + oz;
-          const T r = min_image(C, (T)(ix - px), (T)(iy - py), (T)(iz - pz), T(-1), dx, dy, dz);
-          if (r < f.rcut) v[P + gg] += (double)functor_v(f, r);
+        for (int k = 0; k < kNlppTake; ++k) {
+          px[k] = d * sp[3 * k] + ox;
+          py[k] = d * sp[3 * k + 1] + oy;
+          pz[k] = d * sp[3 * k + 2] + oz;
+          v[k] = v[kNlppTake + k] = 0.0;
         }
-      }
-      for (int j = tid; j < N; j += nt) {
-        if (j == e) continue;
-        const Functor<T>& f = S.fn[kMaxSpecies + (((j < n) == up) ? 0 : 1)];
-        const double rx = R[j], ry = R[N + j], rz = R[2 * N + j];
+        for (int ci = lane; ci < M; ci += 64) {
+          const Functor<T>& f = sFn[S.species[ci]];
+          if (f.ncoef == 0) continue;
+          const double x = sI[ci], y = sI[M + ci], z = sI[2 * M + ci];
 #pragma unroll
-        for (int gg = 0; gg < P; ++gg) {
-          const double px = d * sp[3 * (k0 + gg)] + ox, py = d * sp[3 * (k0 + gg) + 1] + oy, pz = d * sp[3 * (k0 + gg) + 2] + oz;
-          const T r = min_image(C, (T)(rx - px), (T)(ry - py), (T)(rz - pz), T(-1), dx, dy, dz);
-          if (r < f.rcut) v[2 * P + gg] += (double)functor_v(f, r);
+          for (int k = 0; k < kNlppTake; ++k) v[k] += value(f, (T)(x - px[k]), (T)(y - py[k]), (T)(z - pz[k]));
         }
-      }
-      if constexpr (J3)
+        for (int j = lane; j < N; j += 64) {
+          const Functor<T>& f = sFn[kMaxSpecies + (((j < n) == up) ? 0 : 1)];
+          const double x = sR[j], y = sR[N + j], z = sR[2 * N + j];
+          const bool self = j == e;
 #pragma unroll
-        for (int gg = 0; gg < P; ++gg) {
-          const double px = d * sp[3 * (k0 + gg)] + ox, py = d * sp[3 * (k0 + gg) + 1] + oy, pz = d * sp[3 * (k0 + gg) + 2] + oz;
-          v[2 * P + gg] += j3_value_partial<T>(S, B, C, w, e, px, py, pz, tid, nt);
+          for (int k = 0; k < kNlppTake; ++k) {
+            const double u = value(f, (T)(x - px[k]), (T)(y - py[k]), (T)(z - pz[k]));
+            v[kNlppTake + k] += self ? 0.0 : u;
+          }
         }
-      __syncthreads();   // the P value rows are in LDS
-      for (int ii = tid; ii < P * n; ii += nt) {
-        const int gi = ii / n, j = ii - gi * n;
-        T sv = 0;
+        if constexpr (J3)
 #pragma unroll
-        for (int sl = 0; sl < SL; ++sl) sv += part[((size_t)gi * SL + sl) * S.npad + j];
-        const double t = (double)sv * (double)arow[j];
-#pragma unroll
-        for (int gg = 0; gg < P; ++gg)
-          if (gg == gi) v[gg] += t;
-      }
-      block_sum<double, 3 * P>(v, red);   // ends with a barrier: part and red are free again
-      if (tid < P) {
-#pragma unroll
-        for (int gg = 0; gg < P; ++gg)
-          if (gg == tid) out[k0 + gg] = v[gg] * exp((j1o - v[P + gg]) + (j2o - v[2 * P + gg]));
+          for (int k = 0; k < kNlppTake; ++k)
+            v[kNlppTake + k] += j3_value_partial<T>(S, B, C, w, e, px[k], py[k], pz[k], lane, 64);
+        wave_sums_rows<2 * kNlppTake>(v);
+        // row r (lanes 16r ..) holds sums 2r and 2r + 1: the J1 sums of knots k in rows 0 and 1, the J2
+        // sums in rows 2 and 3; lanes 0 and 16 take their knots' J2 sums from lanes 32 and 48
+        const double b0 = __shfl(v[0], (lane & 31) + 32), b1 = __shfl(v[1], (lane & 31) + 32);
+        if ((lane & 15) == 0 && lane < 32) {
+          double* out = jexp + item * kNlppKnots + k0 + (lane >> 4) * 2;
+          out[0] = (j1o - v[0]) + (j2o - b0);
+          out[1] = (j1o - v[1]) + (j2o - b1);
+        }
       }
     }
   }
+}
+
+// Determinant part and the ratios, in the order of the knot list: LK lanes of a wave take a knot and
+// hold all of its 64 stencil points' sums for Q 16-byte orbital groups each (no LDS, no barriers).
+// A wave takes `take` runs of 64 / LK consecutive knots at a time.  The stencil rows come from L2 and
+// the CU's cache (cached loads: neighbouring knots want them).
+// Bound: L2 and L1 bandwidth of the stencils, 64 rows per knot.  NiO-64, 128 walkers, 396k knots:
+// 1.64 ms in FP32 (28 TB/s of stencil bytes); the whole evaluation's kernels 2.7 ms against 7.4 for a
+// workgroup per knot in the order of ions, whose stencils came from HBM (38 GB at 5.2 TB/s).
+template <typename T, int LK, int Q>
+__global__ __launch_bounds__(256) void k_nlpp_ratios(SysP<T> S, BatchP<T> B, const double* spheres, int maxp,
+                                                     const double* near, const int* items, const int* units,
+                                                     const int* cnt, const double* jexp, int take, double* ratios) {
+  using VT = typename V16<T>::type;
+  constexpr int VW = V16<T>::n, KW = 64 / LK;
+  const int N = S.N, n = S.n, nq = S.npad / VW;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int lk = lane & (LK - 1), slot = lane / LK;
+  // workgroup b runs on XCD b % 8, and XCD x takes the x-th eighth of the list (gridDim.x % 8 == 0)
+  const int nu = cnt[0] * kNlppKnots, run = KW * take, nruns = (nu + run - 1) / run;
+  const int xcd = blockIdx.x & 7, per = (gridDim.x >> 3) * nw;
+  const int lo = (int)((long long)nruns * xcd / 8), hi = (int)((long long)nruns * (xcd + 1) / 8);
+  for (int rn = lo + (int)(blockIdx.x >> 3) * nw + wid; rn < hi; rn += per)
+    for (int t = 0; t < take; ++t) {
+      const int at = rn * run + t * KW + slot;
+      const int u = units[min(at, nu - 1)];   // past the end: the last knot again, not stored
+      int w, e;
+      double pt[3];
+      nlpp_point(S, B, spheres, maxp, near, items, u, w, e, pt);
+      const int det = e < n ? 0 : 1, row = e - det * n;
+      const T* arow = B.Ainv + ((size_t)w * 2 + det) * n * n + (size_t)row * n;
+      VT av[Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int o = (lk + LK * q) * VW;
+        if (n % VW == 0)
+          av[q] = *reinterpret_cast<const VT*>(arow + (o < n ? o : 0));
+        else
+#pragma unroll
+          for (int v = 0; v < VW; ++v) av[q][v] = arow[o + v < n ? o + v : 0];
+#pragma unroll
+        for (int v = 0; v < VW; ++v) av[q][v] = o + v < n ? av[q][v] : T(0);
+      }
+      int ix[3];
+      double tt[3];
+      spline_locate(S.spoG, S.ng, pt[0], pt[1], pt[2], ix, tt);
+      const T* base = S.coefs + (size_t)ix[0] * S.xs + (size_t)ix[1] * S.ys + (size_t)ix[2] * S.zs;
+      int off[Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) off[q] = min(lk + LK * q, nq - 1) * VW;
+      T a[4], b[4], c[4], d1[4], d2[4];
+      bspline_weights<T>((T)tt[0], a, d1, d2);
+      bspline_weights<T>((T)tt[1], b, d1, d2);
+      bspline_weights<T>((T)tt[2], c, d1, d2);
+      T acc[Q][VW];
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int v = 0; v < VW; ++v) acc[q][v] = T(0);
+#pragma unroll
+      for (int p = 0; p < 16; ++p) {
+        const T* col = base + (size_t)(p >> 2) * S.xs + (size_t)(p & 3) * S.ys;
+        VT x[Q][4];
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) x[q][k] = *reinterpret_cast<const VT*>(col + (size_t)k * S.zs + off[q]);
+        const T wxy = a[p >> 2] * b[p & 3];
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+#pragma unroll
+          for (int v = 0; v < VW; ++v)
+            acc[q][v] += wxy * (c[0] * x[q][0][v] + c[1] * x[q][1][v] + c[2] * x[q][2][v] + c[3] * x[q][3][v]);
+      }
+      double s = 0.0;
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int v = 0; v < VW; ++v) s += (double)acc[q][v] * (double)av[q][v];
+      s = dpp_add<0xB1, 0xf>(s);   // the lane's row of 16
+      s = dpp_add<0x4E, 0xf>(s);
+      s = dpp_add<0x141, 0xf>(s);
+      s = dpp_add<0x140, 0xf>(s);
+      if constexpr (LK >= 32) {
+        double x = s, y = s;
+        swap_rows(x, y);
+        s = x + y;
+      }
+      if constexpr (LK == 64) {
+        double x = s, y = s;
+        swap_halves(x, y);
+        s = x + y;
+      }
+      if (lk == 0 && at < nu)
+        ratios[u] = s * exp(jexp[(size_t)items[u / kNlppKnots] * kNlppKnots + u % kNlppKnots]);
+    }
 }
 
 // stand-alone distance rows: lane per (source, target)

@@ -372,7 +372,7 @@ class WalkerBatch:
         return out
 
     def set_nlpp_unit(self, knots_per_unit):
-        """Knots per NonLocalPP work unit (1, 2, 4, 6; 0 = automatic)."""
+        """Runs of knots a wave of the NonLocalPP ratio kernel takes at a time (1, 2, 4, 6; 0 = automatic)."""
         _check(load().qmcx_batch_set_nlpp_unit(self.h, knots_per_unit))
 
     def nlpp_evaluate(self, rmax, spheres, max_pairs=4, copy_out=True, ratios=True):
