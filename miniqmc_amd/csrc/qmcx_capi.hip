@@ -287,6 +287,7 @@ struct GraphKey {
 struct qmcx_batch_s {
   qmcx_system_s* sys = nullptr;
   int W = 0, K = 1, prec = QMCX_FP64, walker0 = 0, slices = 0, nt = 0;
+  int cus = 256;   // compute units of the device
   int nch = 1;   // delayed-update state slots per walker and determinant: one per chunk
   int flush_kind = 0;   // 0: matrix cores when possible, 1: vector FMA, 2: matrix cores, U rows from HBM
   // streamed form of the delayed updates (stale rows and capacitance inverse in HBM, a flush launch
@@ -526,6 +527,25 @@ int launch_moves(qmcx_batch_t b, int nt, size_t lds, const MoveArgs& a, bool st)
   return (b->sys->N <= nt) ? launch_moves_jpt<T, 1, false>(b, nt, lds, a) : launch_moves_jpt<T, 2, false>(b, nt, lds, a);
 }
 
+// Side-stream holds (microseconds) after the event that releases the side work together with a
+// move launch: the FP64 refresh, and the proposals of each determinant (the second's are released
+// before evaluateGL, so they wait longer).  A hold lets the move workgroups, which need a CU each,
+// be placed first.
+//   * None when the move, refresh and proposals workgroups together are no more than the CUs: no
+//     move workgroup can then be kept out.  One walker of the cubic cell (n = 48) waited out the
+//     second determinant's 500 us in every sweep, whose two move launches take 340 us.
+//   * Else up to a share of the move launch, which lasts about 9 us per electron: 0.3 n and 1.3 n us
+//     (at n = 384 the constants 100 and 500 us, which measured best there; 37 walkers at n = 96
+//     lost 60 us per sweep to the full 500).
+constexpr int kHoldRefreshUs = 30, kHoldProp0Us = 100, kHoldProp1Us = 500;
+struct Holds {
+  int refresh, prop[2];
+};
+Holds side_holds(int W, int n, int prop_workgroups, int cus) {
+  if (2 * (long long)W + prop_workgroups <= cus) return Holds{0, {0, 0}};
+  return Holds{kHoldRefreshUs, {std::min(kHoldProp0Us, (3 * n + 9) / 10), std::min(kHoldProp1Us, (13 * n + 9) / 10)}};
+}
+
 // SPO rows at the proposals of electrons det*n + [e0, e0 + ne) of every walker
 constexpr int kPropWorkgroups = 1024;
 // virtual positions per walker in one qmcx_flex_evaluate_ratios call (grid x dimension)
@@ -535,6 +555,12 @@ constexpr int kMaxNlppPairs = 64;
 // workgroups of the NonLocalPP ratio launch (they walk the ordered knots), a multiple of the XCDs
 constexpr int kNlppWorkgroups = 2048;
 constexpr int kNlppThreads = 768;
+
+// proposals workgroups per walker for ne electrons
+int prop_grid(int W, int ne) { return std::max(1, std::min(ne, kPropWorkgroups / W)); }
+Holds batch_holds(const qmcx_batch_t b) {
+  return side_holds(b->W, b->sys->n, b->W * prop_grid(b->W, b->sys->n), b->cus);
+}
 
 template <typename T>
 int launch_proposals(qmcx_batch_t b, hipStream_t st, int det, int e0, int ne, uint64_t seed, double tau,
@@ -554,7 +580,7 @@ int launch_proposals(qmcx_batch_t b, hipStream_t st, int det, int e0, int ne, ui
                             sizeof(double) * (size_t)slices * s->npad);
   // about 1024 workgroups (four per CU), each looping over its electrons: the gather's burst of
   // HBM traffic stays below what slows the latency-bound move kernel beside it
-  const int gx = std::max(1, std::min(ne, kPropWorkgroups / b->W));
+  const int gx = prop_grid(b->W, ne);
   auto kern = [&](auto kslc, auto kv64) {
     hipLaunchKernelGGL((k_spo_proposals<T, decltype(kslc)::value, decltype(kv64)::value>), dim3(gx, b->W), dim3(nt),
                        lds, st, s->params<T>(), b->params<T>(), det, e0, ne, seed, b->sweep, std::sqrt(tau),
@@ -822,18 +848,6 @@ int refresh_det(qmcx_batch_t b, int det, bool into_fresh) {
   return 0;
 }
 
-// Side-stream holds (microseconds) after the event that releases the side work together with a
-// move launch: the FP64 refresh, and the proposals of each determinant (the second's are released
-// before evaluateGL, so they wait longer).
-#ifndef QMCX_HOLD_REFRESH_US
-#define QMCX_HOLD_REFRESH_US 30
-#endif
-#ifndef QMCX_HOLD_PROP0_US
-#define QMCX_HOLD_PROP0_US 100
-#endif
-#ifndef QMCX_HOLD_PROP1_US
-#define QMCX_HOLD_PROP1_US 500
-#endif
 int hold_stream(hipStream_t st, int us) {
   if (us <= 0) return 0;
   hipLaunchKernelGGL(k_hold, dim3(1), dim3(64), 0, st, (unsigned long long)us * 100ull);
@@ -848,7 +862,7 @@ int hold_stream(hipStream_t st, int us) {
 template <typename T>
 int issue_proposals(qmcx_batch_t b, int det, hipEvent_t after, uint64_t seed, double tau, bool hold = false) {
   if (after) HIPCHK(hipStreamWaitEvent(b->pre, after, 0));
-  if (hold && hold_stream(b->pre, det == 0 ? QMCX_HOLD_PROP0_US : QMCX_HOLD_PROP1_US)) return QMCX_ERR_HIP;
+  if (hold && hold_stream(b->pre, batch_holds(b).prop[det])) return QMCX_ERR_HIP;
   if (b->prof_record(4, b->pre)) return QMCX_ERR_HIP;
   if (int rc = launch_proposals<T>(b, b->pre, det, 0, b->sys->n, seed, tau, nullptr)) return rc;
   if (b->prof_close(b->pre)) return QMCX_ERR_HIP;
@@ -878,7 +892,7 @@ int sweep_impl(qmcx_batch_t b, uint64_t seed, double tau, int mode, bool recompu
     if (int rc = issue_proposals<T>(b, 0, b->ev_done[0], seed, tau, true)) return rc;
   if (recompute) {
     HIPCHK(hipStreamWaitEvent(b->aux, b->ev_done[0], 0));
-    if (hold_stream(b->aux, QMCX_HOLD_REFRESH_US)) return QMCX_ERR_HIP;
+    if (hold_stream(b->aux, batch_holds(b).refresh)) return QMCX_ERR_HIP;
     if (int rc = refresh_det<T>(b, 0, false)) return rc;
     HIPCHK(hipEventRecord(b->ev_fresh[0], b->aux));
   }
@@ -898,7 +912,7 @@ int sweep_impl(qmcx_batch_t b, uint64_t seed, double tau, int mode, bool recompu
   if (recompute) {
     HIPCHK(hipEventRecord(b->ev_gl, b->stream));
     HIPCHK(hipStreamWaitEvent(b->aux, b->ev_gl, 0));
-    if (hold_stream(b->aux, QMCX_HOLD_REFRESH_US)) return QMCX_ERR_HIP;
+    if (hold_stream(b->aux, batch_holds(b).refresh)) return QMCX_ERR_HIP;
     if (int rc = refresh_det<T>(b, 1, true)) return rc;
     hipLaunchKernelGGL(k_refresh_det, dim3((b->W + 63) / 64), dim3(64), 0, b->aux, b->W, 1, b->ld_fresh, b->ph_fresh,
                        b->logdet, b->phase, b->logv, b->hist, b->hist_cap, b->sweep);
@@ -1040,10 +1054,17 @@ int group_moves(qmcx_group_s* g, int det, int mode, bool flush) {
   return 0;
 }
 
+// the group's holds: its largest system sets the length of a move launch
+Holds group_holds(const qmcx_group_s* g) {
+  int n = 1;
+  for (qmcx_batch_t b : g->b) n = std::max(n, b->sys->n);
+  return side_holds(g->Wtot, n, g->pgx * g->Wtot, g->b[0]->cus);
+}
+
 // the proposals of determinant det of every batch, on the proposals stream after `after`
 int group_proposals(qmcx_group_s* g, int det, hipEvent_t after, uint64_t seed, double tau, bool hold) {
   if (after) HIPCHK(hipStreamWaitEvent(g->pre, after, 0));
-  if (hold && hold_stream(g->pre, det == 0 ? QMCX_HOLD_PROP0_US : QMCX_HOLD_PROP1_US)) return QMCX_ERR_HIP;
+  if (hold && hold_stream(g->pre, group_holds(g).prop[det])) return QMCX_ERR_HIP;
   PropGroup<float> P;
   std::memset(&P, 0, sizeof(P));
   P.ng = (int)g->b.size();
@@ -1085,7 +1106,7 @@ int group_sweep(qmcx_group_s* g, uint64_t seed, double tau, int mode, bool recom
     if (int rc = group_proposals(g, 0, g->ev_done[0], seed, tau, true)) return rc;
   if (recompute) {
     HIPCHK(hipStreamWaitEvent(g->aux, g->ev_done[0], 0));
-    if (hold_stream(g->aux, QMCX_HOLD_REFRESH_US)) return QMCX_ERR_HIP;
+    if (hold_stream(g->aux, group_holds(g).refresh)) return QMCX_ERR_HIP;
     for (qmcx_batch_t b : g->b)
       if (int rc = refresh_det<float>(b, 0, false)) return rc;
     HIPCHK(hipEventRecord(g->ev_fresh[0], g->aux));
@@ -1105,7 +1126,7 @@ int group_sweep(qmcx_group_s* g, uint64_t seed, double tau, int mode, bool recom
   if (recompute) {
     HIPCHK(hipEventRecord(g->ev_gl, g->stream));
     HIPCHK(hipStreamWaitEvent(g->aux, g->ev_gl, 0));
-    if (hold_stream(g->aux, QMCX_HOLD_REFRESH_US)) return QMCX_ERR_HIP;
+    if (hold_stream(g->aux, group_holds(g).refresh)) return QMCX_ERR_HIP;
     for (qmcx_batch_t b : g->b) {
       if (int rc = refresh_det<float>(b, 1, true)) return rc;
       hipLaunchKernelGGL(k_refresh_det, dim3((b->W + 63) / 64), dim3(64), 0, g->aux, b->W, 1, b->ld_fresh, b->ph_fresh,
@@ -1599,6 +1620,10 @@ int qmcx_batch_create(qmcx_batch_t* out, qmcx_system_t s, int nwalkers, int dela
   b->K = delay_rank;
   b->nch = delay_rank > 1 ? (s->n + delay_rank - 1) / delay_rank : 1;
   b->prec = precision;
+  {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->dev) == hipSuccess && cus > 0) b->cus = cus;
+  }
   const size_t es = precision == QMCX_FP32 ? 4 : 8;
   const size_t W = nwalkers, n = s->n, N = s->N, K = delay_rank;
   // LDS check for the move kernel
