@@ -10,6 +10,7 @@
 #include <limits>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/qmcx.h"
@@ -42,6 +43,62 @@ struct DevBuf {
     if (p) (void)hipFree(p);
   }
   hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes > 0 ? bytes : 1); }
+  template <typename P>
+  P* as() const { return (P*)p; }
+};
+
+// Pinned host memory given back by destroyed batches, up to kPinnedPool bytes, for later ones: a pinned
+// allocation takes longer than the small calls it serves.
+constexpr size_t kPinnedPool = size_t(32) << 20;
+struct PinnedPool {
+  std::mutex mu;
+  std::vector<std::pair<size_t, void*>> free;   // bytes, block
+  size_t bytes = 0;
+  void* take(size_t want, size_t* cap) {   // the smallest block that holds `want`, or null
+    std::lock_guard<std::mutex> lock(mu);
+    int best = -1;
+    for (int i = 0; i < (int)free.size(); ++i)
+      if (free[i].first >= want && (best < 0 || free[i].first < free[best].first)) best = i;
+    if (best < 0) return nullptr;
+    void* p = free[best].second;
+    *cap = free[best].first;
+    bytes -= *cap;
+    free.erase(free.begin() + best);
+    return p;
+  }
+  bool give(void* p, size_t cap) {
+    std::lock_guard<std::mutex> lock(mu);
+    if (bytes + cap > kPinnedPool) return false;
+    free.emplace_back(cap, p);
+    bytes += cap;
+    return true;
+  }
+};
+PinnedPool& pinned_pool() {
+  static PinnedPool* pool = new PinnedPool;   // outlives every batch, whatever the order of destruction
+  return *pool;
+}
+
+// Pinned host buffer of a batch, grown to what a call needs and kept: copies to and from it need no
+// staging by the runtime, and kernels read and write small ones in place.
+struct PinnedBuf {
+  void* p = nullptr;
+  size_t cap = 0;
+  void release() {
+    if (p && !pinned_pool().give(p, cap)) (void)hipHostFree(p);
+    p = nullptr;
+    cap = 0;
+  }
+  int need(size_t bytes) {
+    if (bytes <= cap) return 0;
+    release();
+    p = pinned_pool().take(bytes, &cap);
+    if (p) return 0;
+    HIPCHK(hipHostMalloc(&p, bytes, hipHostMallocPortable));
+    cap = bytes;
+    return 0;
+  }
+  ~PinnedBuf() { release(); }
   template <typename P>
   P* as() const { return (P*)p; }
 };
@@ -307,9 +364,23 @@ struct qmcx_batch_s {
   double band = 0.0;
   bool rows64 = false, rows64_stale = false;
   bool fp64_rows = false;   // FP64 Slater rows asked for on their own (rows64 also follows the band)
-  double* flex_displ = nullptr;   // [W][3] proposals of the pending flex move
-  int* flex_decide = nullptr;     // [W]
+  // flex calls: the kernels read the displacements [W][3] and decisions [W] from pinned host memory
+  // and write the move's records [W][9] there; flex_none: device zeros (reject every move)
+  PinnedBuf flex_io;
+  int* flex_none = nullptr;
   int flex_iel = -1;
+  bool flex_rows = false;         // spo and prop hold electron flex_iel's proposal
+  std::vector<int> flex_cnt[2];   // pending delayed rows of each walker and determinant (state slot 0)
+  bool flex_live[2] = {false, false};   // slot 0 of the determinant holds the flex moves' rows
+  double* flex_displ() const { return flex_io.as<double>(); }
+  double* flex_record() const { return flex_displ() + 3 * (size_t)W; }
+  int* flex_decide() const { return (int*)(flex_record() + 9 * (size_t)W); }
+  void flex_clear() {   // no pending delayed rows
+    flex_pending = flex_live[0] = flex_live[1] = false;
+    for (auto& c : flex_cnt) c.assign(W, 0);
+  }
+  PinnedBuf vr_io;                // virtual positions [np][3] and ratios [np] of a small call
+  PinnedBuf nl_io;                // NonLocalPP counts, pair list and ratios on their way to the caller
   double* vr_pos = nullptr;       // [W][vr_cap][3] virtual positions of qmcx_flex_evaluate_ratios
   double* vr_out = nullptr;       // [W][vr_cap] their ratios
   int vr_cap = 0;
@@ -364,6 +435,7 @@ struct qmcx_batch_s {
     if (gexec) hipGraphExecDestroy(gexec);
     gexec = nullptr;
     ++epoch;
+    flex_rows = false;   // a setting may change what the proposals write
   }
   int* flags = nullptr;   // [1] kernel error bits
   double* A64 = nullptr;   // FP32 form: [W][2][n][n] FP64 Slater rows (the FP64 refresh inverts these)
@@ -548,6 +620,8 @@ Holds side_holds(int W, int n, int prop_workgroups, int cus) {
 
 // SPO rows at the proposals of electrons det*n + [e0, e0 + ne) of every walker
 constexpr int kPropWorkgroups = 1024;
+// points of a qmcx_flex_evaluate_ratios call up to which the kernel works on pinned host memory in place
+constexpr size_t kVirtualInPlace = 2048;
 // virtual positions per walker in one qmcx_flex_evaluate_ratios call (grid x dimension)
 constexpr int kMaxVirtualPoints = 1 << 16;
 // electron-ion pairs per electron held by qmcx_nlpp_evaluate
@@ -795,23 +869,36 @@ int moves_det(qmcx_batch_t b, int det, int mode, bool flush) {
   return 0;
 }
 
-// The delayed rows flex_* moves left pending (state slot 0 of each determinant) reach the inverse
+// The delayed rows flex_* moves left pending (state slot 0 of a determinant) reach the inverse
 // (DiracDeterminant::completeUpdates, DiracDeterminant.cpp:294-321), or, with thr > 1, only those of
-// the walkers whose pending rows reached thr; the applied slots are emptied.
+// the walkers whose pending rows reached thr; the applied slots are emptied.  The host counts the
+// rows too (the decisions are the caller's), so launches with nothing to apply are left out.
 template <typename T>
-int flush_pending_t(qmcx_batch_t b, int thr) {
-  for (int det = 0; det < 2; ++det) {
-    if (int rc = launch_flush<T>(b, b->stream, det, 0, 1, thr)) return rc;
-    hipLaunchKernelGGL(k_reset_delay<T>, dim3((b->W + 255) / 256), dim3(256), 0, b->stream, b->params<T>(), det, thr);
-    HIPCHK(hipGetLastError());
-  }
+int flush_slot(qmcx_batch_t b, int det, int thr) {
+  if (int rc = launch_flush<T>(b, b->stream, det, 0, 1, thr)) return rc;
+  hipLaunchKernelGGL(k_reset_delay<T>, dim3((b->W + 255) / 256), dim3(256), 0, b->stream, b->params<T>(), det, thr);
+  HIPCHK(hipGetLastError());
   return 0;
 }
-int flush_pending(qmcx_batch_t b, int thr = 1) {
+int flush_pending(qmcx_batch_t b) {
   if (!b->flex_pending) return 0;
-  const int rc = b->prec == QMCX_FP32 ? flush_pending_t<float>(b, thr) : flush_pending_t<double>(b, thr);
+  for (int det = 0; det < 2; ++det) {
+    const auto& c = b->flex_cnt[det];
+    if (std::all_of(c.begin(), c.end(), [](int x) { return x == 0; })) continue;
+    const int rc = b->prec == QMCX_FP32 ? flush_slot<float>(b, det, 1) : flush_slot<double>(b, det, 1);
+    if (rc) return rc;
+  }
+  b->flex_clear();
+  return 0;
+}
+// the rows of determinant det's walkers that reached the delay rank (DelayedUpdate.h:151-152)
+int flush_full(qmcx_batch_t b, int det) {
+  auto& c = b->flex_cnt[det];
+  if (std::none_of(c.begin(), c.end(), [&](int x) { return x >= b->K; })) return 0;
+  const int rc = b->prec == QMCX_FP32 ? flush_slot<float>(b, det, b->K) : flush_slot<double>(b, det, b->K);
   if (rc) return rc;
-  if (thr <= 1) b->flex_pending = false;
+  for (int& x : c)
+    if (x >= b->K) x = 0;
   return 0;
 }
 
@@ -1181,7 +1268,7 @@ static int check_flags(qmcx_batch_t b) {
 }
 
 template <typename T>
-static int launch_virtual_ratios(qmcx_batch_t b, int iel, int nvp) {
+static int launch_virtual_ratios(qmcx_batch_t b, int iel, int nvp, const double* pos, double* out) {
   const qmcx_system_s* s = b->sys;
   const int nq = s->npad / (16 / (int)sizeof(T));
   const int slices = proposal_slices<T>(s, b->slices);
@@ -1189,7 +1276,7 @@ static int launch_virtual_ratios(qmcx_batch_t b, int iel, int nvp) {
   if (nt > 1024) return fail(QMCX_ERR_ARG, "spline row does not fit a workgroup");
   const size_t lds = sizeof(T) * (size_t)slices * s->npad + sizeof(double) * 16 * 3;
   hipLaunchKernelGGL(k_virtual_ratios<T>, dim3(nvp, b->W), dim3(nt), lds, b->stream, s->params<T>(), b->params<T>(),
-                     iel, nvp, b->vr_pos, b->vr_out, slices);
+                     iel, nvp, pos, out, slices);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -1618,6 +1705,7 @@ int qmcx_batch_create(qmcx_batch_t* out, qmcx_system_t s, int nwalkers, int dela
   b->sys = s;
   b->W = nwalkers;
   b->K = delay_rank;
+  b->flex_clear();
   b->nch = delay_rank > 1 ? (s->n + delay_rank - 1) / delay_rank : 1;
   b->prec = precision;
   {
@@ -1743,8 +1831,7 @@ int qmcx_batch_destroy(qmcx_batch_t b) {
   for (void* p : b->allocs) hipFree(p);
   if (b->trace) hipFree(b->trace);
   if (b->hist) hipFree(b->hist);
-  if (b->flex_displ) hipFree(b->flex_displ);
-  if (b->flex_decide) hipFree(b->flex_decide);
+  if (b->flex_none) hipFree(b->flex_none);
   if (b->cad) hipFree(b->cad);
   if (b->cad_flag) hipFree(b->cad_flag);
   if (b->vr_pos) hipFree(b->vr_pos);
@@ -1779,7 +1866,8 @@ int qmcx_batch_set_positions(qmcx_batch_t b, const double* R) {
     for (int i = 0; i < N; ++i)
       for (int d = 0; d < 3; ++d) soa[((size_t)w * 3 + d) * N + i] = R[((size_t)w * N + i) * 3 + d];
   HIPCHK(hipMemcpy(b->R, soa.data(), sizeof(double) * soa.size(), hipMemcpyHostToDevice));
-  b->flex_pending = false;   // the state is rebuilt by the next evaluateLog; pending rows are void
+  b->flex_clear();   // the state is rebuilt by the next evaluateLog; pending rows are void
+  b->flex_rows = false;
   return 0;
 }
 
@@ -1855,7 +1943,7 @@ int qmcx_evaluate_log(qmcx_batch_t b, double* log_out) {
   if (int rc = b->sys->sync_functors()) return rc;
   int rc = b->prec == QMCX_FP32 ? evaluate_log_impl<float>(b) : evaluate_log_impl<double>(b);
   if (rc) return rc;
-  b->flex_pending = false;   // the inverse is rebuilt from scratch: pending delayed rows are void
+  b->flex_clear();   // the inverse is rebuilt from scratch: pending delayed rows are void
   if (b->cad) {
     hipLaunchKernelGGL(k_cadence_reset, dim3((b->W + 255) / 256), dim3(256), 0, b->stream, b->cad, b->W, -1);
     HIPCHK(hipGetLastError());
@@ -1902,12 +1990,9 @@ int qmcx_run_sweeps(qmcx_batch_t b, int nsweeps, uint64_t seed, double tau, int 
   }
   // this run's counters: evaluateGL writes its history from slot 0 (sweep[1] = the first sweep),
   // the first proposals belong to that sweep (sweep[2])
-  int cur[4];
-  HIPCHK(hipStreamSynchronize(b->stream));
-  HIPCHK(hipMemcpy(cur, b->sweep, sizeof(cur), hipMemcpyDeviceToHost));
-  cur[1] = cur[0];
-  cur[2] = cur[0];
-  HIPCHK(hipMemcpy(b->sweep, cur, sizeof(cur), hipMemcpyHostToDevice));
+  b->flex_rows = false;
+  hipLaunchKernelGGL(k_begin_run, dim3(1), dim3(64), 0, b->stream, b->sweep);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(b->ev0, b->stream));
   if (nsweeps > 0) {
     const GraphKey key{nsweeps, seed, tau, accept_mode, recompute_every};
@@ -2033,9 +2118,11 @@ static int flex_launch(qmcx_batch_t b, int iel, bool apply) {
   int rc = choose_shape(s, nt);
   if (rc) return rc;
   const int det = iel < s->n ? 0 : 1;
-  rc = f32 ? launch_proposals<float>(b, b->stream, det, iel - det * s->n, 1, 0, 1.0, b->flex_displ)
-           : launch_proposals<double>(b, b->stream, det, iel - det * s->n, 1, 0, 1.0, b->flex_displ);
-  if (rc) return rc;
+  if (!b->flex_rows) {
+    rc = f32 ? launch_proposals<float>(b, b->stream, det, iel - det * s->n, 1, 0, 1.0, b->flex_displ())
+             : launch_proposals<double>(b, b->stream, det, iel - det * s->n, 1, 0, 1.0, b->flex_displ());
+    if (rc) return rc;
+  }
   MoveArgs a;
   std::memset(&a, 0, sizeof(a));
   a.spo = b->spo;
@@ -2047,12 +2134,13 @@ static int flex_launch(qmcx_batch_t b, int iel, bool apply) {
   a.nchunks = 1;
   a.mode = QMCX_ACCEPT_METROPOLIS;
   a.slices = 0;
-  a.decide = b->flex_decide;
+  a.decide = apply ? b->flex_decide() : b->flex_none;
+  a.record = apply ? nullptr : b->flex_record();
   // delay rank > 1: the streamed form keeps each walker's accepted rows pending in state slot 0
   // of the determinant (DelayedUpdate::acceptRow, DelayedUpdate.h:124-153) until the walker's
   // count reaches the delay rank (flushed after the accept) or completeUpdates
   const bool st = b->K > 1;
-  a.resume = b->flex_pending ? 1 : 0;
+  a.resume = b->flex_live[det] ? 1 : 0;   // else the slot may hold a sweep's rows, long applied
   const bool trace_was = b->trace_on;
   b->trace_on = true;
   if (f32) {
@@ -2065,9 +2153,11 @@ static int flex_launch(qmcx_batch_t b, int iel, bool apply) {
   b->trace_on = trace_was;
   if (rc) return rc;
   if (st) {
-    b->flex_pending = true;
-    if (apply)
-      if (int rc2 = flush_pending(b, b->K)) return rc2;
+    b->flex_pending = b->flex_live[det] = true;
+    if (apply) {
+      for (int w = 0; w < b->W; ++w) b->flex_cnt[det][w] += b->flex_decide()[w] != 0 ? 1 : 0;
+      if (int rc2 = flush_full(b, det)) return rc2;
+    }
   }
   return 0;
 }
@@ -2076,28 +2166,26 @@ int qmcx_flex_ratio_grad(qmcx_batch_t b, int iel, const double* displ, double* r
                          double* grad_new) {
   if (!b || !displ || iel < 0 || iel >= b->sys->N) return fail(QMCX_ERR_ARG, "bad argument");
   if (int rc = check_j3(b)) return rc;
-  if (!b->flex_displ) {
-    HIPCHK(hipMalloc(&b->flex_displ, sizeof(double) * 3 * b->W));
-    HIPCHK(hipMalloc(&b->flex_decide, sizeof(int) * b->W));
+  const size_t W = b->W;
+  if (!b->flex_none) {
+    if (int rc = b->flex_io.need(sizeof(double) * 12 * W + sizeof(int) * W)) return rc;
+    HIPCHK(hipMalloc(&b->flex_none, sizeof(int) * W));
+    HIPCHK(hipMemset(b->flex_none, 0, sizeof(int) * W));
   }
-  if (!b->trace) HIPCHK(hipMalloc(&b->trace, sizeof(double) * 9 * (size_t)b->W * b->sys->N));
-  std::vector<int> none(b->W, 0);
-  HIPCHK(hipMemcpyAsync(b->flex_displ, displ, sizeof(double) * 3 * b->W, hipMemcpyHostToDevice, b->stream));
-  HIPCHK(hipMemcpyAsync(b->flex_decide, none.data(), sizeof(int) * b->W, hipMemcpyHostToDevice, b->stream));
+  if (!b->trace) HIPCHK(hipMalloc(&b->trace, sizeof(double) * 9 * W * b->sys->N));
+  std::memcpy(b->flex_displ(), displ, sizeof(double) * 3 * W);   // earlier flex launches have been waited for
+  b->flex_rows = false;
   if (int rc = flex_launch(b, iel, false)) return rc;
-  // the electron's [W] slice of the trace ([W][N][9]) in one strided copy
-  std::vector<double> rec(9 * (size_t)b->W);
-  HIPCHK(hipMemcpy2DAsync(rec.data(), sizeof(double) * 9, b->trace + (size_t)iel * 9, sizeof(double) * 9 * b->sys->N,
-                          sizeof(double) * 9, b->W, hipMemcpyDeviceToHost, b->stream));
   HIPCHK(hipStreamSynchronize(b->stream));
-  for (int w = 0; w < b->W; ++w) {
-    const double* q = rec.data() + 9 * (size_t)w;
+  for (size_t w = 0; w < W; ++w) {
+    const double* q = b->flex_record() + 9 * w;
     if (ratio) ratio[w] = q[0];
     for (int d = 0; d < 3; ++d) {
       if (grad_now) grad_now[3 * w + d] = q[3 + d];
       if (grad_new) grad_new[3 * w + d] = q[6 + d];
     }
   }
+  b->flex_rows = true;
   b->flex_iel = iel;
   return 0;
 }
@@ -2105,10 +2193,11 @@ int qmcx_flex_ratio_grad(qmcx_batch_t b, int iel, const double* displ, double* r
 int qmcx_flex_accept_restore(qmcx_batch_t b, int iel, const int* accepted) {
   if (!b || !accepted) return fail(QMCX_ERR_ARG, "null argument");
   if (iel != b->flex_iel) return fail(QMCX_ERR_STATE, "accept_restore must follow ratio_grad of the same electron");
-  HIPCHK(hipMemcpyAsync(b->flex_decide, accepted, sizeof(int) * b->W, hipMemcpyHostToDevice, b->stream));
+  std::memcpy(b->flex_decide(), accepted, sizeof(int) * b->W);
   if (int rc = flex_launch(b, iel, true)) return rc;
   HIPCHK(hipStreamSynchronize(b->stream));
   b->flex_iel = -1;
+  b->flex_rows = false;
   return 0;
 }
 
@@ -2134,6 +2223,22 @@ int qmcx_flex_evaluate_ratios(qmcx_batch_t b, int iel, int nvp, const double* vp
     return fail(QMCX_ERR_ARG, "bad argument");
   if (int rc = check_j3(b)) return rc;   // the kernel reads the batch's J3 state when the system has one
   if (int rc = flush_pending(b)) return rc;   // the ratios read the up-to-date inverse rows
+  const size_t np = (size_t)nvp * b->W;
+  auto launch = [&](const double* pos, double* out) {
+    return b->prec == QMCX_FP32 ? launch_virtual_ratios<float>(b, iel, nvp, pos, out)
+                                : launch_virtual_ratios<double>(b, iel, nvp, pos, out);
+  };
+  if (np <= kVirtualInPlace) {
+    // a small call: the kernel reads the points and writes the ratios in pinned host memory
+    if (int rc = b->vr_io.need(sizeof(double) * 4 * kVirtualInPlace)) return rc;
+    double* pos = b->vr_io.as<double>();
+    double* out = pos + 3 * kVirtualInPlace;
+    std::memcpy(pos, vpos, sizeof(double) * 3 * np);
+    if (int rc = launch(pos, out)) return rc;
+    HIPCHK(hipStreamSynchronize(b->stream));
+    std::memcpy(ratios, out, sizeof(double) * np);
+    return 0;
+  }
   if (nvp > b->vr_cap) {
     HIPCHK(hipStreamSynchronize(b->stream));
     if (b->vr_pos) hipFree(b->vr_pos);
@@ -2144,11 +2249,8 @@ int qmcx_flex_evaluate_ratios(qmcx_batch_t b, int iel, int nvp, const double* vp
     HIPCHK(hipMalloc(&b->vr_out, sizeof(double) * (size_t)nvp * b->W));
     b->vr_cap = nvp;
   }
-  const size_t np = (size_t)nvp * b->W;
   HIPCHK(hipMemcpyAsync(b->vr_pos, vpos, sizeof(double) * 3 * np, hipMemcpyHostToDevice, b->stream));
-  const int rc = b->prec == QMCX_FP32 ? launch_virtual_ratios<float>(b, iel, nvp)
-                                      : launch_virtual_ratios<double>(b, iel, nvp);
-  if (rc) return rc;
+  if (int rc = launch(b->vr_pos, b->vr_out)) return rc;
   HIPCHK(hipMemcpyAsync(ratios, b->vr_out, sizeof(double) * np, hipMemcpyDeviceToHost, b->stream));
   HIPCHK(hipStreamSynchronize(b->stream));
   return 0;
@@ -2195,26 +2297,28 @@ int qmcx_nlpp_evaluate(qmcx_batch_t b, double rmax, const double* spheres, int m
                         b->stream));
   const int rc = b->prec == QMCX_FP32 ? launch_nlpp<float>(b, rmax, max_pairs) : launch_nlpp<double>(b, rmax, max_pairs);
   if (rc) return rc;
-  std::vector<int> cnt(WN), items;
-  std::vector<double> rat;
-  int listed = 0;
-  HIPCHK(hipMemcpyAsync(cnt.data(), b->nl_cnt, sizeof(int) * WN, hipMemcpyDeviceToHost, b->stream));
-  HIPCHK(hipMemcpyAsync(&listed, b->nl_items + WN * max_pairs, sizeof(int), hipMemcpyDeviceToHost, b->stream));
+  // counts and the pair list's length, then (with ratios) the list and its ratios, through pinned memory
+  if (int rc2 = b->nl_io.need(sizeof(int) * (WN + 2))) return rc2;
+  int* cnt = b->nl_io.as<int>();
+  HIPCHK(hipMemcpyAsync(cnt, b->nl_cnt, sizeof(int) * WN, hipMemcpyDeviceToHost, b->stream));
+  HIPCHK(hipMemcpyAsync(cnt + WN, b->nl_items + WN * max_pairs, sizeof(int), hipMemcpyDeviceToHost, b->stream));
   HIPCHK(hipStreamSynchronize(b->stream));
+  const size_t listed = (size_t)cnt[WN];
+  if (npairs) std::copy(cnt, cnt + WN, npairs);
+  bool over = false;
+  for (size_t i = 0; i < WN; ++i) over = over || cnt[i] > max_pairs;
   if (ratios && listed > 0) {
     // the listed pairs' ratios to their places; the other slots stay as they were
-    items.resize(listed);
-    rat.resize((size_t)listed * kNlppKnots);
-    HIPCHK(hipMemcpyAsync(items.data(), b->nl_items, sizeof(int) * listed, hipMemcpyDeviceToHost, b->stream));
-    HIPCHK(hipMemcpyAsync(rat.data(), b->nl_out, sizeof(double) * rat.size(), hipMemcpyDeviceToHost, b->stream));
+    if (int rc2 = b->nl_io.need((sizeof(double) * kNlppKnots + sizeof(int)) * listed)) return rc2;
+    double* rat = b->nl_io.as<double>();
+    int* items = (int*)(rat + listed * kNlppKnots);
+    HIPCHK(hipMemcpyAsync(items, b->nl_items, sizeof(int) * listed, hipMemcpyDeviceToHost, b->stream));
+    HIPCHK(hipMemcpyAsync(rat, b->nl_out, sizeof(double) * listed * kNlppKnots, hipMemcpyDeviceToHost, b->stream));
     HIPCHK(hipStreamSynchronize(b->stream));
-    for (int i = 0; i < listed; ++i)
-      std::memcpy(ratios + (size_t)items[i] * kNlppKnots, rat.data() + (size_t)i * kNlppKnots,
-                  sizeof(double) * kNlppKnots);
+    for (size_t i = 0; i < listed; ++i)
+      std::memcpy(ratios + (size_t)items[i] * kNlppKnots, rat + i * kNlppKnots, sizeof(double) * kNlppKnots);
   }
-  if (npairs) std::copy(cnt.begin(), cnt.end(), npairs);
-  for (size_t i = 0; i < WN; ++i)
-    if (cnt[i] > max_pairs) return fail(QMCX_ERR_ARG, "more ions within rmax of an electron than max_pairs");
+  if (over) return fail(QMCX_ERR_ARG, "more ions within rmax of an electron than max_pairs");
   return 0;
 }
 
@@ -2586,11 +2690,9 @@ int qmcx_group_run_sweeps(qmcx_group_t g, int nsweeps, uint64_t seed, double tau
       b->drop_graph();
       g->drop_graph();   // the group's graph holds the old history buffer
     }
-    int cur[4];
-    HIPCHK(hipMemcpy(cur, b->sweep, sizeof(cur), hipMemcpyDeviceToHost));
-    cur[1] = cur[0];
-    cur[2] = cur[0];
-    HIPCHK(hipMemcpy(b->sweep, cur, sizeof(cur), hipMemcpyHostToDevice));
+    b->flex_rows = false;
+    hipLaunchKernelGGL(k_begin_run, dim3(1), dim3(64), 0, g->stream, b->sweep);
+    HIPCHK(hipGetLastError());
   }
   HIPCHK(hipEventRecord(g->ev0, g->stream));
   if (nsweeps > 0) {

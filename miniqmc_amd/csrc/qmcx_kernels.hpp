@@ -116,6 +116,7 @@ struct MoveArgs {
   int* cad;
   int* cad_flag;
   const int* decide;     // [W] caller accept decisions (flex_acceptrestoreMove) or null
+  double* record;        // [W][9] the move's trace record for the flex calls (host memory), or null
   // FP32 form, Metropolis: a move whose uniform u lies within band * ratio^2 of ratio^2 is
   // decided on its FP64 ratio (0: off)
   double band;
@@ -1883,6 +1884,11 @@ __global__ void k_hold(unsigned long long ticks) {
     const unsigned long long t0 = wall_clock64();
     while (wall_clock64() - t0 < ticks) __builtin_amdgcn_s_sleep(8);
   }
+}
+
+// a run begins: its history starts at slot 0 and its first proposals belong to the current sweep
+__global__ void k_begin_run(int* sweep) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) sweep[1] = sweep[2] = sweep[0];
 }
 
 __global__ void k_count(int* counter) {

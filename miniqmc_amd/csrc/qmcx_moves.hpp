@@ -1173,7 +1173,7 @@ __device__ __forceinline__ void moves_body(const SysP<T>& S, const BatchP<T>& B,
       }
     }
     if (B.trace != nullptr && tid == 0) {
-      double* t = B.trace + ((size_t)w * N + iel) * 9;
+      double t[9];
       t[0] = ratio;
       t[1] = rdet;
       t[2] = accept ? 1.0 : 0.0;
@@ -1183,6 +1183,12 @@ __device__ __forceinline__ void moves_body(const SysP<T>& S, const BatchP<T>& B,
       t[6] = red[4] / rdet + pr[kPropJ1 + 2] + red[8] + cur3[1];
       t[7] = red[5] / rdet + pr[kPropJ1 + 3] + red[9] + cur3[2];
       t[8] = red[6] / rdet + pr[kPropJ1 + 4] + red[10] + cur3[3];
+      double* out = B.trace + ((size_t)w * N + iel) * 9;
+#pragma unroll
+      for (int q = 0; q < 9; ++q) out[q] = t[q];
+      if (a.record != nullptr)
+#pragma unroll
+        for (int q = 0; q < 9; ++q) a.record[(size_t)w * 9 + q] = t[q];
     }
     if (accept) {
       if (tid == 0) {
