@@ -657,20 +657,22 @@ __global__ __launch_bounds__(64 * kFlushWaves) void k_flush_mfma(SysP<float> S, 
 // pivot of step k stays in place (kof[i] = k, piv[k] = i), and the permutations are applied as
 // psiM is written:  psiM[k][j] = Y[kof[j]][piv[k]].
 //
-// A panel is B columns of X in LDS (P[c][i]), factored in sub-panels of 16 columns: thread i
-// holds row i's 16 entries in registers for the 16 elimination steps; the panel's other sub-panel
-// then gets their rank-16 update, and the other columns of X the panel's rank-B update
+// A panel is B columns of X: thread i holds row i's B entries in registers for the panel's
+// elimination steps.  The other columns of X then get the panel's rank-B update, P[c][i] the
+// finished panel in LDS,
 //   Y[c][i] <- (i a pivot row of the panel ? 0 : Y[c][i]) + sum_t Y[c][p_t] P[t][i]
 // on the FP64 matrix cores (v_mfma_f64_16x16x4f64).  A wave owns a 16-column tile of X from its
 // pivot-row entries to its last row, so the update needs no barriers, and it loads row tiles ahead
 // of the one it multiplies.
 //
-// Bound: latency of the pivot steps (0.75 us each: two barriers, the pivot search, one division)
+// Bound: latency of the pivot steps (about 1 us each: two barriers, the pivot search, one division)
 // and of a wave's tile; with as many matrices as CUs at n = 384 the passes over X, whose working
-// set (302 MB) exceeds the last-level cache.  n = 384: one matrix 1.10 ms, 128 at once 1.31, 256 at
-// once 1.95 (the form that exchanged rows, held 32-column panel rows in registers and streamed X in
-// 64-column chunks through LDS: 2.45, 2.49 and 2.92); n = 192: 0.29 (0.62) ms.
-constexpr int kGJSub = 16;     // columns of a sub-panel
+// set (302 MB) exceeds the last-level cache.  n = 384: one matrix 1.17 ms, 128 at once 1.39, 256 at
+// once 2.1 (the form that exchanged rows and streamed X in 64-column chunks through LDS between
+// barriers: 2.32, 2.51 and 2.97); n = 192, 256 at once: 0.41 (0.66) ms.  Sub-panels of 16 columns
+// with a rank-16 update between them take 1.10, 1.30 and 2.0 ms but round differently: an element of
+// the FP32 inverse may then differ by one ulp, which a chain of FP32 moves without a refresh amplifies
+// to 1e-3 in an ill-conditioned walker.
 constexpr int kGJAhead = 4;    // row tiles in flight per wave (even)
 // LDS row stride of the panel (doubles): an odd multiple of 16, so that the four 16-lane groups of
 // a matrix operand read different banks
@@ -683,7 +685,7 @@ __host__ __device__ inline GJLds gj_lds_b(int n, int b) {
   size_t o = 0;
   auto take = [&](size_t bytes) { const size_t at = o; o += (bytes + 15) & ~(size_t)15; return at; };
   L.oP = take(sizeof(double) * (size_t)b * (gj_stride(n) + 1));   // the panel; on the way out rows of stride + 1
-  L.oPr = take(sizeof(double) * 2 * kGJSub);                     // pivot row of a step (two in turn)
+  L.oPr = take(sizeof(double) * 2 * (size_t)(b + 2));            // scaled pivot row of a step and 1 / pivot (two in turn)
   L.oDv = take(sizeof(double) * (size_t)n);                      // the pivots
   L.oRed = take(sizeof(double) * 2 * 16);                        // per wave: best pivot candidate (two in turn)
   L.oRi = take(sizeof(int) * 2 * 16);                            // and its row
@@ -775,9 +777,9 @@ __global__ __launch_bounds__(NT) void k_gj_invert(int n, const TI* A, TO* psiM, 
                                                           double* phase, int ld_stride, int mat_stride, const int* only) {
   const int mat = blockIdx.x, tid = threadIdx.x;
   if (only != nullptr && only[mat] == 0) return;   // only the matrices whose flag is set
-  constexpr int nw = NT / 64, NS = B / kGJSub;
-  const int lane = tid & 63, wid = tid >> 6, lj = lane & 15, lg = lane >> 4;
-  const int ns = gj_stride(n), nt = (n + 15) >> 4;
+  constexpr int nw = NT / 64;
+  const int lane = tid & 63, wid = tid >> 6;
+  const int ns = gj_stride(n);
   const GJLds L = gj_lds_b(n, B);
   extern __shared__ __align__(16) unsigned char smem[];
   double* P = (double*)(smem + L.oP);
@@ -801,113 +803,75 @@ __global__ __launch_bounds__(NT) void k_gj_invert(int n, const TI* A, TO* psiM, 
 
   for (int k0 = 0; k0 < n; k0 += B) {
     const int bb = min(B, n - k0);
-    // ---- the panel's columns into LDS (zeros past bb)
-    {
-      double v[B];
+    // ---- the panel's columns (zeros past bb) and its elimination steps
+    double pr[B];
 #pragma unroll
-      for (int c = 0; c < B; ++c) {
-        const size_t at = (size_t)(k0 + min(c, bb - 1)) * n + (own ? tid : 0);
-        v[c] = k0 == 0 ? (double)a[at] : Y[at];
-      }
-      if (own)
-#pragma unroll
-        for (int c = 0; c < B; ++c) P[(size_t)c * ns + tid] = c < bb ? v[c] : 0.0;
+    for (int c = 0; c < B; ++c) {
+      const size_t at = (size_t)(k0 + min(c, bb - 1)) * n + (own ? tid : 0);
+      pr[c] = k0 == 0 ? (double)a[at] : Y[at];
     }
-#pragma unroll 1
-    for (int sp = 0; sp < NS; ++sp) {
-      const int ks = k0 + kGJSub * sp, bs = min(kGJSub, n - ks);   // the sub-panel's first step and its steps
-      if (bs <= 0) break;
-      double* Ps = P + (size_t)kGJSub * sp * ns;
-      double pr[kGJSub];
 #pragma unroll
-      for (int c = 0; c < kGJSub; ++c) pr[c] = Ps[(size_t)c * ns + (own ? tid : 0)];
+    for (int c = 0; c < B; ++c) pr[c] = (own && c < bb) ? pr[c] : 0.0;
 #pragma unroll
-      for (int j = 0; j < kGJSub; ++j) {
-        if (j < bs) {
-          const int k = ks + j;
-          double* pw = prow + kGJSub * (j & 1);
-          double* rw = rv + 16 * (j & 1);
-          int* iw = ri + 16 * (j & 1);
-          const double prj = pr[j];
-          // pivot: the largest |P[j][i]| of the rows not used yet, the lowest of them: the wave's
-          // largest magnitude and its first lane, then the waves' candidates side by side in the
-          // lanes of every wave.  Candidates and pivot rows alternate between two slots, so a step
-          // needs no barrier between its reads and the next step's writes
-          const double av = (own && !used) ? fabs(prj) : -1.0;
-          const double best = wave_max(av);
-          const unsigned long long hit = __ballot(av == best);
-          if (lane == 0) {
-            rw[wid] = best;
-            iw[wid] = min(wid * 64 + max(__ffsll((long long)hit) - 1, 0), n - 1);
-          }
-          lds_sync();
-          const double cv = rw[lane & (nw - 1)];
-          const int cr = iw[lane & (nw - 1)];
-          double cb = cv;
-          cb = dpp_max<0xB1, 0xf>(cb);
-          cb = dpp_max<0x4E, 0xf>(cb);
-          cb = dpp_max<0x141, 0xf>(cb);   // of eight lanes
-          if constexpr (nw > 8) cb = dpp_max<0x140, 0xf>(cb);
-          const int qb = max(__ffsll((long long)__ballot(cv == cb)) - 1, 0);   // 0 if a NaN hid the maximum
-          const int p = __builtin_amdgcn_readlane(cr, qb);                     // in [0, n)
-          const bool isp = tid == p;
-          par ^= (unsigned)__popcll(__ballot(own && !used && tid < p)) & 1u;
-          if (isp) {
-#pragma unroll
-            for (int c = 0; c < kGJSub; ++c) {
-              pw[c] = pr[c];
-              pr[c] = 0.0;
-            }
-            dv[k] = prj;
-            piv[k] = p;
-            kof[p] = k;
-            used = true;
-          }
-          const double rinv = 1.0 / cb;   // 1 / |pivot|, while the pivot row is on its way
-          lds_sync();
-          // the pivot row becomes prow / d (its entry in the pivot column 1 / d), every other row
-          // loses its multiple of it (its entry there -f / d)
-          const double dinv = pw[j] < 0.0 ? -rinv : rinv;
-          const double f = isp ? -dinv : prj * dinv;
-#pragma unroll
-          for (int c = 0; c < kGJSub; ++c)
-            if (c != j) pr[c] -= f * pw[c];
-          pr[j] = -f;
+    for (int j = 0; j < B; ++j) {
+      if (j < bb) {
+        const int k = k0 + j;
+        double* pw = prow + (B + 2) * (j & 1);
+        double* rw = rv + 16 * (j & 1);
+        int* iw = ri + 16 * (j & 1);
+        const double prj = pr[j];
+        // pivot: the largest |P[j][i]| of the rows not used yet, the lowest of them: the wave's
+        // largest magnitude and its first lane, then the waves' candidates side by side in the
+        // lanes of every wave.  Candidates and pivot rows alternate between two slots, so a step
+        // needs no barrier between its reads and the next step's writes
+        const double av = (own && !used) ? fabs(prj) : -1.0;
+        const double best = wave_max(av);
+        const unsigned long long hit = __ballot(av == best);
+        if (lane == 0) {
+          rw[wid] = best;
+          iw[wid] = min(wid * 64 + max(__ffsll((long long)hit) - 1, 0), n - 1);
         }
-      }
-      if (own)
+        lds_sync();
+        const double cv = rw[lane & (nw - 1)];
+        const int cr = iw[lane & (nw - 1)];
+        double cb = cv;
+        cb = dpp_max<0xB1, 0xf>(cb);
+        cb = dpp_max<0x4E, 0xf>(cb);
+        cb = dpp_max<0x141, 0xf>(cb);   // of eight lanes
+        if constexpr (nw > 8) cb = dpp_max<0x140, 0xf>(cb);
+        const int qb = max(__ffsll((long long)__ballot(cv == cb)) - 1, 0);   // 0 if a NaN hid the maximum
+        const int p = __builtin_amdgcn_readlane(cr, qb);                     // in [0, n)
+        const bool isp = tid == p;
+        par ^= (unsigned)__popcll(__ballot(own && !used && tid < p)) & 1u;
+        const double rinv = 1.0 / cb;   // 1 / |pivot|
+        if (isp) {
+          // the scaled pivot row for the others; its own new entries are left to the update below
+          const double dinv = prj < 0.0 ? -rinv : rinv;
 #pragma unroll
-        for (int c = 0; c < kGJSub; ++c) Ps[(size_t)c * ns + tid] = pr[c];
-      __syncthreads();
-      if (NS > 1 && bb > kGJSub) {
-        // ---- the panel's other sub-panel: P[c][i] <- (i a pivot row ? 0 : P[c][i]) + sum_t P[c][p_t] Ps[t][i]
-        double* Po = P + (size_t)kGJSub * (1 - sp) * ns;
-        double a4[kGJSub / 4];
-#pragma unroll
-        for (int s = 0; s < kGJSub / 4; ++s) {
-          const int t = 4 * s + lg;
-          const double v = Po[(size_t)lj * ns + piv[ks + min(t, bs - 1)]];
-          a4[s] = t < bs ? v : 0.0;
-        }
-        __syncthreads();
-        for (int it = wid; it < nt; it += nw) {
-          const int i = 16 * it + lj;
-          const unsigned kk = (unsigned)(kof[i] - ks);
-          f64x4 acc;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const double x = Po[(size_t)(lg + 4 * r) * ns + i];
-            acc[r] = kk < (unsigned)bs ? 0.0 : x;
+          for (int c = 0; c < B; ++c) {
+            pw[c] = pr[c] * dinv;
+            pr[c] = 0.0;
           }
-#pragma unroll
-          for (int s = 0; s < kGJSub / 4; ++s)
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a4[s], Ps[(size_t)(4 * s + lg) * ns + i], acc, 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) Po[(size_t)(lg + 4 * r) * ns + i] = acc[r];
+          pw[B] = dinv;
+          dv[k] = prj;
+          piv[k] = p;
+          kof[p] = k;
+          used = true;
         }
-        __syncthreads();
+        lds_sync();
+        // the pivot row becomes the scaled row (its entry in the pivot column 1 / d), every other
+        // row loses its multiple of it (its entry there -f / d)
+        const double f = isp ? -1.0 : prj;
+#pragma unroll
+        for (int c = 0; c < B; ++c)
+          if (c != j) pr[c] -= f * pw[c];
+        pr[j] = -f * pw[B];
       }
     }
+    if (own)
+#pragma unroll
+      for (int c = 0; c < B; ++c) P[(size_t)c * ns + tid] = pr[c];
+    __syncthreads();
     // ---- the other columns, then the panel itself, back to Y
     if (k0 == 0)
       gj_update<TI, B>(n, ns, k0, bb, a, Y, P, piv, kof);
