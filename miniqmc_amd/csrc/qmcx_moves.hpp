@@ -193,9 +193,17 @@ __host__ __device__ inline bool flush_own_fits(int N, int n, int K, int E) {
   return L.total - L.oQ >= flush_own_lds(n, K);
 }
 
+// The flush is a function of its own (not inlined: its registers would push the move loop into
+// spills), so its pointers carry their address space: a generic pointer would turn every LDS read
+// into a flat load through the vector memory path.
+template <typename P>
+using Lds = __attribute__((address_space(3))) P;
+template <typename P>
+using Glb = __attribute__((address_space(1))) P;
+
 // T2 = -(T Binv) in FP64 for one wave's 16-row tile: T (16 x cp, row stride KC) read from sT,
 // T2 written over it once every lane has read its T row
-__device__ inline void flush_own_t2(int c, int cp, int KC, int KP, const double* sBinv, float* sT) {
+__device__ inline void flush_own_t2(int c, int cp, int KC, int KP, const Lds<double>* sBinv, Lds<float>* sT) {
   const int lane = threadIdx.x & 63;
   float t2v[8];
 #pragma unroll
@@ -226,7 +234,7 @@ __device__ inline void flush_own_t2(int c, int cp, int KC, int KP, const double*
 // j + 16 g supplies A = T[j][4s + g] and B = Binv[4s + g][16b + j]; its result register r is
 // T2[g + 4r][16b + j] (the FP64 16x16x4 layout).  Entries past c are zero (T's are stored as
 // zeros, Binv's are masked here).
-__device__ inline void flush_own_t2_mfma(int c, int cp, int KC, int KP, const double* sBinv, float* sT) {
+__device__ inline void flush_own_t2_mfma(int c, int cp, int KC, int KP, const Lds<double>* sBinv, Lds<float>* sT) {
   const int lane = threadIdx.x & 63, lj = lane & 15, lg = lane >> 4;
   f64x4 acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
   for (int s4 = 0; s4 < cp; s4 += 4) {
@@ -258,39 +266,60 @@ __device__ inline void flush_own_t2_mfma(int c, int cp, int KC, int KP, const do
 // stride n + 4), rows 16 .. c-1 from the slots of the chunk's rejected moves in sAc (sRej[d -
 // 16], row stride sa), both staged at the chunk's end; V rows are the chunk's stale inverse rows
 // (sAc rows sAl[d]), Binv in LDS (row stride KP).  c <= 16, or c <= 32 with K >= 32.
-__device__ __attribute__((noinline)) void flush_own_tile(int n, int K, int KP, int c, const int* sRows, const int* sAl,
-                                      const double* sBinv, const float* sAc, int sa, const float* sU,
-                                      const int* sRej, float* Ainv, float* scratch) {
+// NT: orbital tiles (of 16) held, at least n / 16; the ones past n are zeros, so the products need
+// no test per tile and the LDS operands of the next step are read while a step's matrix
+// instructions run.
+// Bound: LDS and matrix-core latency of one CU's eight waves.  With generic pointers (flat loads for
+// LDS) and a test and a wait per matrix instruction, a flush took 160k cycles at NiO-64 and 75k at
+// NiO-32; now three NiO-64 sweeps of 128 walkers take 23.0 ms against 25.8, three NiO-32 sweeps of 256
+// walkers 12.3 against 13.6, and a NiO-32 flush 40k cycles.
+template <int NT>
+__device__ __forceinline__ void flush_own_tile(int n, int K, int KP, int c, const Lds<int>* sRows, const Lds<int>* sAl,
+                                              const Lds<double>* sBinv, const Lds<float>* sAc, int sa,
+                                              const Lds<float>* sU, const Lds<int>* sRej, Glb<float>* Ainv,
+                                              Lds<float>* scratch) {
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nw = blockDim.x >> 6;
   const int li = lane & 15, g = lane >> 4;
   const int KC = (K + 15) & ~15, c4 = (c + 3) & ~3, cp = (c + 15) & ~15, nct = n >> 4, us = n + 4;
-  float* sT = scratch + (size_t)wid * 16 * KC;
+  constexpr int G = 3, G2 = NT % 6 == 0 ? 6 : 3;   // orbital tiles per step of the first and second product
+  Lds<float>* sT = scratch + (size_t)wid * 16 * KC;
   for (int tile = wid; tile < nct; tile += nw) {
     const int r0 = tile * 16;
-    float* ar = Ainv + (size_t)(r0 + li) * n + 4 * g;
-    f32x4_t a[kFlushOwnTiles];
+    Glb<float>* ar = Ainv + (size_t)(r0 + li) * n + 4 * g;
+    f32x4_t a[NT];
 #pragma unroll
-    for (int q = 0; q < kFlushOwnTiles; ++q)
-      a[q] = *reinterpret_cast<const f32x4_t*>(ar + min(q, nct - 1) * 16);
+    for (int q = 0; q < NT; ++q) a[q] = *reinterpret_cast<const Glb<f32x4_t>*>(ar + min(q, nct - 1) * 16);
+#pragma unroll
+    for (int q = 0; q < NT; ++q)
+      if (q >= nct) a[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     // ---- GEMM 1: T^T = U rows^T over all orbitals, 16 delayed rows per pass, two accumulators
     for (int dt = 0; dt < cp; dt += 16) {
       const int d = dt + li;
       const bool din = d < c;   // U row d of the A operand is a delayed row
-      const float* ul = (dt == 0 ? sU + (size_t)(din ? li : 0) * us : sAc + (size_t)(din ? sRej[li] : 0) * sa) + 4 * g;
+      const Lds<float>* ul = (dt == 0 ? sU + (size_t)(din ? li : 0) * us : sAc + (size_t)(din ? sRej[li] : 0) * sa) + 4 * g;
       f32x4_t acc0 = f32x4_t{0.f, 0.f, 0.f, 0.f}, acc1 = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      f32x4_t u[2][G];
 #pragma unroll
-      for (int q = 0; q < kFlushOwnTiles; ++q) {
-        if (q < nct) {
-          f32x4_t uv = *reinterpret_cast<const f32x4_t*>(ul + q * 16);
-          uv = din ? uv : f32x4_t{0.f, 0.f, 0.f, 0.f};
-          f32x4_t& acc = (q & 1) ? acc1 : acc0;
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(uv[0], a[q][0], acc, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(uv[1], a[q][1], acc, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(uv[2], a[q][2], acc, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(uv[3], a[q][3], acc, 0, 0, 0);
+      for (int q = 0; q < G; ++q) u[0][q] = *reinterpret_cast<const Lds<f32x4_t>*>(ul + min(q, nct - 1) * 16);
+#pragma unroll
+      for (int g0 = 0; g0 < NT / G; ++g0) {
+        if (g0 + 1 < NT / G)
+#pragma unroll
+          for (int q = 0; q < G; ++q)
+            u[(g0 + 1) & 1][q] = *reinterpret_cast<const Lds<f32x4_t>*>(ul + min((g0 + 1) * G + q, nct - 1) * 16);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+          const f32x4_t uv = u[g0 & 1][q], av = a[g0 * G + q];
+          f32x4_t& acc = ((g0 * G + q) & 1) ? acc1 : acc0;
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(uv[0], av[0], acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(uv[1], av[1], acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(uv[2], av[2], acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(uv[3], av[3], acc, 0, 0, 0);
         }
       }
-      // lane (i, g) register r: T[i][dt + 4g + r], minus E (row r0+i is delayed row dd)
+      // lane (i, g) register r: T[i][dt + 4g + r], minus E (row r0+i is delayed row dd); entries past
+      // c (their U row stood in for none) are zeros
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int dd = dt + 4 * g + r;
@@ -301,21 +330,36 @@ __device__ __attribute__((noinline)) void flush_own_tile(int n, int K, int KP, i
     }
     wave_lds_fence();
     flush_own_t2_mfma(c, cp, KC, KP, sBinv, sT);
-    // ---- GEMM 2: rows^T += V^T T2^T, four delayed rows per step; V rows from LDS
-    for (int d0 = 0; d0 < c4; d0 += 4) {
-      const int dk = d0 + g;
-      const float bv = sT[li * KC + dk];
-      const float* vr = sAc + (size_t)sAl[dk < c ? dk : 0] * sa + li;
+    // ---- GEMM 2: rows^T += V^T T2^T, four delayed rows per step; V rows from LDS (T2 is zero past c)
+    auto vrow = [&](int d0) { return sAc + (size_t)sAl[d0 + g < c ? d0 + g : 0] * sa + li; };
+    const Lds<float>* vr = vrow(0);
+    float bv = sT[li * KC + g], v[2][G2];
 #pragma unroll
-      for (int q = 0; q < kFlushOwnTiles; ++q)
-        if (q < nct) {
-          const float v = dk < c ? vr[q * 16] : 0.f;
-          a[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, bv, a[q], 0, 0, 0);
-        }
+    for (int q = 0; q < G2; ++q) v[0][q] = vr[min(q, nct - 1) * 16];
+    for (int d0 = 0; d0 < c4; d0 += 4) {
+      const Lds<float>* vn = vrow(d0 + 4);
+      const float bn = sT[li * KC + min(d0 + 4 + g, cp - 1)];
+#pragma unroll
+      for (int g0 = 0; g0 < NT / G2; ++g0) {
+        // the next operands: this step's next tiles, or the next step's first ones
+        const bool more = g0 + 1 < NT / G2;
+#pragma unroll
+        for (int q = 0; q < G2; ++q)
+          v[(g0 + 1) & 1][q] = more ? vr[min((g0 + 1) * G2 + q, nct - 1) * 16] : vn[min(q, nct - 1) * 16];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < G2; ++q)
+          a[g0 * G2 + q] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[g0 & 1][q], bv, a[g0 * G2 + q], 0, 0, 0);
+      }
+      if constexpr ((NT / G2) % 2 == 1)
+#pragma unroll
+        for (int q = 0; q < G2; ++q) v[0][q] = v[1][q];
+      vr = vn;
+      bv = bn;
     }
 #pragma unroll
-    for (int q = 0; q < kFlushOwnTiles; ++q)
-      if (q < nct) *reinterpret_cast<f32x4_t*>(ar + q * 16) = a[q];
+    for (int q = 0; q < NT; ++q)
+      if (q < nct) *reinterpret_cast<Glb<f32x4_t>*>(ar + q * 16) = a[q];
     wave_lds_fence();   // the next tile's T overwrites this one's T2
   }
   __syncthreads();   // the next chunk reads these rows
@@ -326,31 +370,32 @@ __device__ __attribute__((noinline)) void flush_own_tile(int n, int K, int KP, i
 // updates each half and stores it.  U rows are the new Slater rows in HBM (written at the
 // chunk's end, six orbital tiles' loads in flight).
 constexpr int kFlushOwnHalf = kFlushOwnTiles / 2;
-__device__ __attribute__((noinline)) void flush_own(int n, int K, int KP, int c, const int* sRows, const int* sAl, const double* sBinv,
-                                 const float* sAc, int sa, const float* Amat, float* Ainv, float* scratch) {
+__device__ __forceinline__ void flush_own_hbm(int n, int K, int KP, int c, const Lds<int>* sRows, const Lds<int>* sAl,
+                                              const Lds<double>* sBinv, const Lds<float>* sAc, int sa,
+                                              const Glb<float>* Amat, Glb<float>* Ainv, Lds<float>* scratch) {
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nw = blockDim.x >> 6;
   const int li = lane & 15, g = lane >> 4;
   const int KC = (K + 15) & ~15, cp = (c + 15) & ~15, nct = n >> 4;
-  float* sT = scratch + (size_t)wid * 16 * KC;
+  Lds<float>* sT = scratch + (size_t)wid * 16 * KC;
   for (int tile = wid; tile < nct; tile += nw) {
     const int r0 = tile * 16;
-    const float* ar = Ainv + (size_t)(r0 + li) * n + 4 * g;
+    const Glb<float>* ar = Ainv + (size_t)(r0 + li) * n + 4 * g;
     // ---- GEMM 1: T^T = U rows^T per 16 delayed rows, the orbitals in two halves
     for (int dt = 0; dt < cp / 16; ++dt) {
       const int d = dt * 16 + li;
-      const float* ur = Amat + (size_t)sRows[d < c ? d : 0] * n + 4 * g;
+      const Glb<float>* ur = Amat + (size_t)sRows[d < c ? d : 0] * n + 4 * g;
       f32x4_t acc0 = f32x4_t{0.f, 0.f, 0.f, 0.f}, acc1 = f32x4_t{0.f, 0.f, 0.f, 0.f};
       for (int h0 = 0; h0 < nct; h0 += kFlushOwnHalf) {
         f32x4_t a[kFlushOwnHalf];
 #pragma unroll
         for (int q = 0; q < kFlushOwnHalf; ++q)
-          a[q] = *reinterpret_cast<const f32x4_t*>(ar + min(h0 + q, nct - 1) * 16);
+          a[q] = *reinterpret_cast<const Glb<f32x4_t>*>(ar + min(h0 + q, nct - 1) * 16);
 #pragma unroll
         for (int kb = 0; kb < kFlushOwnHalf; kb += 6) {
           f32x4_t u[6];
 #pragma unroll
           for (int q = 0; q < 6; ++q)
-            u[q] = *reinterpret_cast<const f32x4_t*>(ur + min(h0 + kb + q, nct - 1) * 16);
+            u[q] = *reinterpret_cast<const Glb<f32x4_t>*>(ur + min(h0 + kb + q, nct - 1) * 16);
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int q = 0; q < 6; ++q) {
@@ -380,24 +425,43 @@ __device__ __attribute__((noinline)) void flush_own(int n, int K, int KP, int c,
       f32x4_t a[kFlushOwnHalf];
 #pragma unroll
       for (int q = 0; q < kFlushOwnHalf; ++q)
-        a[q] = *reinterpret_cast<const f32x4_t*>(ar + min(h0 + q, nct - 1) * 16);
+        a[q] = *reinterpret_cast<const Glb<f32x4_t>*>(ar + min(h0 + q, nct - 1) * 16);
       for (int d0 = 0; d0 < cp; d0 += 4) {
         const int dk = d0 + g;
         const float bv = sT[li * KC + dk];
-        const float* vr = sAc + (size_t)sAl[dk < c ? dk : 0] * sa + li;
+        const Lds<float>* vr = sAc + (size_t)sAl[dk < c ? dk : 0] * sa + li;
 #pragma unroll
         for (int q = 0; q < kFlushOwnHalf; ++q) {
           const float v = dk < c ? vr[min(h0 + q, nct - 1) * 16] : 0.f;
           a[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, bv, a[q], 0, 0, 0);
         }
       }
-      float* aw = Ainv + (size_t)(r0 + li) * n + 4 * g;
+      Glb<float>* aw = Ainv + (size_t)(r0 + li) * n + 4 * g;
 #pragma unroll
       for (int q = 0; q < kFlushOwnHalf; ++q)
-        if (h0 + q < nct) *reinterpret_cast<f32x4_t*>(aw + (h0 + q) * 16) = a[q];
+        if (h0 + q < nct) *reinterpret_cast<Glb<f32x4_t>*>(aw + (h0 + q) * 16) = a[q];
     }
   }
   __syncthreads();   // the next chunk reads these rows
+}
+
+// The chunk's delayed updates to the walker's whole inverse, U rows from LDS (in_lds) or HBM; the
+// fewest orbital tiles that hold a row.
+__device__ __attribute__((noinline)) void flush_own(int n, int K, int KP, int c, bool in_lds, const Lds<int>* sRows,
+                                                    const Lds<int>* sAl, const Lds<double>* sBinv,
+                                                    const Lds<float>* sAc, int sa, const Lds<float>* sU,
+                                                    const Lds<int>* sRej, const Glb<float>* Amat, Glb<float>* Ainv,
+                                                    Lds<float>* scratch) {
+  n = __builtin_amdgcn_readfirstlane(n);   // the same on every lane: scalar branches and addresses
+  K = __builtin_amdgcn_readfirstlane(K);
+  KP = __builtin_amdgcn_readfirstlane(KP);
+  c = __builtin_amdgcn_readfirstlane(c);
+  sa = __builtin_amdgcn_readfirstlane(sa);
+  if (!__builtin_amdgcn_readfirstlane((int)in_lds))
+    flush_own_hbm(n, K, KP, c, sRows, sAl, sBinv, sAc, sa, Amat, Ainv, scratch);
+  else if (n <= 96) flush_own_tile<6>(n, K, KP, c, sRows, sAl, sBinv, sAc, sa, sU, sRej, Ainv, scratch);
+  else if (n <= 192) flush_own_tile<12>(n, K, KP, c, sRows, sAl, sBinv, sAc, sa, sU, sRej, Ainv, scratch);
+  else flush_own_tile<24>(n, K, KP, c, sRows, sAl, sBinv, sAc, sa, sU, sRej, Ainv, scratch);
 }
 
 // Sherman-Morrison update of a walker's inverse after an accepted move (DelayedUpdate.h:166-173),
@@ -1508,10 +1572,10 @@ __device__ __forceinline__ void moves_body(const SysP<T>& S, const BatchP<T>& B,
       const int* sRej = (const int*)(smem + L.oInv);
       float* scratch = sU + (size_t)kFlushOwnU * (n + 4);
       // the same test as the staging of the new Slater rows at the chunk's end
-      if (a.flush_u > 0 && (c <= kFlushOwnU || (K >= 32 && c <= 32 && 2 * c <= kFlushOwnU + E)))
-        flush_own_tile(n, K, KP, c, sRows, sAl, sBinv, (const float*)sAc, sa, sU, sRej, (float*)Ainv, scratch);
-      else
-        flush_own(n, K, KP, c, sRows, sAl, sBinv, (const float*)sAc, sa, (const float*)Amat, (float*)Ainv, scratch);
+      const bool in_lds = a.flush_u > 0 && (c <= kFlushOwnU || (K >= 32 && c <= 32 && 2 * c <= kFlushOwnU + E));
+      flush_own(n, K, KP, c, in_lds, (const Lds<int>*)sRows, (const Lds<int>*)sAl, (const Lds<double>*)sBinv,
+                (const Lds<float>*)sAc, sa, (const Lds<float>*)sU, (const Lds<int>*)sRej, (const Glb<float>*)Amat,
+                (Glb<float>*)Ainv, (Lds<float>*)scratch);
     }
   }
   cbn = cb + Eend;
