@@ -820,6 +820,48 @@ __device__ inline void j3_apply(T* sJ3, int N, const int* sk, const T* sv, int n
   }
 }
 
+// Copies `rows` rows of nv vectors, vector j of row r from src(r)[j] to store(r, j, value): a wave
+// takes R rows by 64 H vectors at a time with all those loads in flight.  Per chunk of 32 moves at
+// NiO-64 the accepted rows take 17k cycles and the stale inverse rows 11k (25k and 17k with the
+// elements dealt to threads one by one, which divides by the row length for each).
+template <typename VT, int R, int H, typename Src, typename Store>
+__device__ __forceinline__ void copy_rows(int rows, int nv, Src src, Store store) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  for (int r1 = wid * R; r1 < rows; r1 += nw * R) {
+    const VT* row[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) row[k] = src(min(r1 + k, rows - 1));
+    for (int j0 = 0; j0 < nv; j0 += 64 * H) {
+      VT v[R][H];
+#pragma unroll
+      for (int k = 0; k < R; ++k)
+#pragma unroll
+        for (int h = 0; h < H; ++h) v[k][h] = row[k][min(j0 + 64 * h + lane, nv - 1)];
+#pragma unroll
+      for (int k = 0; k < R; ++k)
+#pragma unroll
+        for (int h = 0; h < H; ++h)
+          if (r1 + k < rows && j0 + 64 * h + lane < nv) store(r1 + k, j0 + 64 * h + lane, v[k][h]);
+    }
+  }
+}
+
+// E rows of n elements from HBM (contiguous) to LDS rows of stride ls
+template <typename T>
+__device__ __forceinline__ void stage_rows(int n, int E, const T* src, T* dst, int ls) {
+  using VT = typename V16<T>::type;
+  constexpr int VW = V16<T>::n;
+  if (n % VW != 0)
+    copy_rows<T, 4, 2>(E, n, [&](int r) { return src + (size_t)r * n; },
+                       [&](int r, int j, T v) { dst[(size_t)r * ls + j] = v; });
+  else if (n / VW <= 64)
+    copy_rows<VT, 8, 1>(E, n / VW, [&](int r) { return reinterpret_cast<const VT*>(src + (size_t)r * n); },
+                        [&](int r, int j, VT v) { reinterpret_cast<VT*>(dst + (size_t)r * ls)[j] = v; });
+  else
+    copy_rows<VT, 4, 2>(E, n / VW, [&](int r) { return reinterpret_cast<const VT*>(src + (size_t)r * n); },
+                        [&](int r, int j, VT v) { reinterpret_cast<VT*>(dst + (size_t)r * ls)[j] = v; });
+}
+
 // KD: delayed updates (K > 1: inverse-row cache, Woodbury bordering) or Sherman-Morrison (K = 1).
 // ARB: the FP64 re-evaluation of near-tie Metropolis decisions is compiled in (FP32, K > 1); only
 // that instantiation carries its code, whose registers would otherwise spill in every move.
@@ -951,9 +993,9 @@ __device__ __forceinline__ void moves_body(const SysP<T>& S, const BatchP<T>& B,
   // round of loads)
   {
     const unsigned je = (unsigned)(sizeof(T) * E);
-    const LdsCopy cp[6] = {{sAc, Ainv + (size_t)r0 * n, KD && !ST ? (unsigned)(sizeof(T) * E * n) : 0u,
-                            (unsigned)(sizeof(T) * n), (unsigned)(sizeof(T) * sa)},
-                           {sProp, prop, (unsigned)(sizeof(double) * kProp * E)},
+    if (KD && !ST)
+      stage_rows<T>(n, E, (const T*)Ainv + (size_t)r0 * n, sAc, sa);
+    const LdsCopy cp[5] = {{sProp, prop, (unsigned)(sizeof(double) * kProp * E)},
                            {sJ1o, J1 + cb, je},
                            {sJ1o + E, J1 + N + cb, je},
                            {sJ1o + 2 * E, J1 + 2 * N + cb, je},
@@ -1492,7 +1534,6 @@ __device__ __forceinline__ void moves_body(const SysP<T>& S, const BatchP<T>& B,
     constexpr int VW = V16<T>::n;
     const bool vec = n % VW == 0 && S.npad % VW == 0;
     const int nv = vec ? n / VW : n;   // vectors (or scalars) per row
-    const int tot = ca * 5 * nv;
     // The new Slater rows also go to LDS for the kernel's own flush (FP32): rows 0-15 to sU,
     // rows 16 on (k >= 32, while they fit) to the chunk's rejected moves' slots of sAc, whose
     // stale rows the flush does not read; their list goes to sRej (sInv's LDS, free here).
@@ -1511,37 +1552,27 @@ __device__ __forceinline__ void moves_body(const SysP<T>& S, const BatchP<T>& B,
       }
       __syncthreads();
     }
-    for (int b0 = 0; b0 < tot; b0 += 8 * nt) {
-      VT v[8];
-      T sv[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int i = min(b0 + k * nt + tid, tot - 1);
-        const int d = i / (5 * nv), rem = i - d * 5 * nv, o = rem / nv, j = rem - o * nv;
-        const T* src = spo + (size_t)sAl[d] * 5 * S.npad + (size_t)o * S.npad;
-        if (vec) v[k] = ((const VT*)src)[j];
-        else sv[k] = src[j];
-      }
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int i = b0 + k * nt + tid;
-        if (i < tot) {
-          const int d = i / (5 * nv), rem = i - d * 5 * nv, o = rem / nv, j = rem - o * nv;
-          const int rw = r0 + sAl[d];
-          T* dst = o == 0 ? Amat + (size_t)rw * n
-                          : (o < 4 ? dpsiM + (size_t)rw * 3 * n + (size_t)(o - 1) * n : d2psiM + (size_t)rw * n);
-          if (vec) ((VT*)dst)[j] = v[k];
-          else dst[j] = sv[k];
-          if constexpr (sizeof(T) == 4) {
-            if (stage_u && o == 0) {
-              float* ur = d < kFlushOwnU ? sU + (size_t)d * (n + 4) : (float*)sAc + (size_t)sRej[d - kFlushOwnU] * sa;
-              if (vec) *reinterpret_cast<VT*>(ur + j * VW) = v[k];
-              else ur[j] = sv[k];
-            }
-          }
+    // row q of 5 ca: output q % 5 of accepted move q / 5
+    const int rows5 = ca * 5;
+    auto store = [&](int q, int j, auto val) {   // vector (or scalar) j of row q
+      const int d = q / 5, o = q - 5 * d, rw = r0 + sAl[d];
+      T* dst = o == 0 ? Amat + (size_t)rw * n
+                      : (o < 4 ? dpsiM + (size_t)rw * 3 * n + (size_t)(o - 1) * n : d2psiM + (size_t)rw * n);
+      reinterpret_cast<decltype(val)*>(dst)[j] = val;
+      if constexpr (sizeof(T) == 4)
+        if (stage_u && o == 0) {
+          float* ur = d < kFlushOwnU ? sU + (size_t)d * (n + 4) : (float*)sAc + (size_t)sRej[d - kFlushOwnU] * sa;
+          reinterpret_cast<decltype(val)*>(ur)[j] = val;
         }
-      }
-    }
+    };
+    auto row_of = [&](int q) {
+      const int d = q / 5, o = q - 5 * d;
+      return spo + (size_t)sAl[d] * 5 * S.npad + (size_t)o * S.npad;
+    };
+    auto src_vec = [&](int q) { return reinterpret_cast<const VT*>(row_of(q)); };
+    if (!vec) copy_rows<T, 4, 2>(rows5, n, row_of, store);
+    else if (nv <= 64) copy_rows<VT, 12, 1>(rows5, nv, src_vec, store);
+    else copy_rows<VT, 6, 2>(rows5, nv, src_vec, store);
   }
   // the FP32 form's FP64 Slater rows of the accepted moves, from their proposals' FP64 values
   if (B.A64 != nullptr) {
