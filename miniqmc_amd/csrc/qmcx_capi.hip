@@ -441,6 +441,7 @@ struct qmcx_batch_s {
   double* A64 = nullptr;   // FP32 form: [W][2][n][n] FP64 Slater rows (the FP64 refresh inverts these)
   double* spo64 = nullptr; // FP32 form: [W][2][n][npad] FP64 values at the sweep's proposals
   double* prop = nullptr; // [W][2][n][kProp] proposal records of the sweep
+  int* order = nullptr;   // evaluateLog: electrons ordered by place [W*N], their keys [W*N], key counts and cursors
   int* rows = nullptr;
   int* ndelay = nullptr;
   double* logdet = nullptr;
@@ -686,6 +687,21 @@ int spline_slices_for(const qmcx_system_s* s, int nt) {
   return S;
 }
 
+// blocks of points ordered by place: 4 grid cells per axis, more while the blocks outnumber kBlockKeys
+constexpr int kBlockKeys = 32768;
+GridBlocks grid_blocks(const qmcx_system_s* s) {
+  GridBlocks nb;
+  for (nb.shift = 2;; ++nb.shift) {
+    for (int d = 0; d < 3; ++d) nb.nb[d] = (s->ng[d] + (1 << nb.shift) - 1) >> nb.shift;
+    if ((long long)nb.nb[0] * nb.nb[1] * nb.nb[2] <= kBlockKeys) return nb;
+  }
+}
+
+// evaluateLog's electrons are ordered by place when there are this many (the four ordering launches take
+// about 30 us, as long as the rows of a few thousand electrons), and their stencils cover the grid
+// this many times over (else there is little to share)
+constexpr long long kOrderPoints = 8192, kOrderReuse = 4;
+
 template <typename T>
 int launch_spo_rows(qmcx_batch_t b) {
   const qmcx_system_s* s = b->sys;
@@ -695,8 +711,41 @@ int launch_spo_rows(qmcx_batch_t b) {
   const int nt = std::max(64, (nq * slices + 63) / 64 * 64);
   size_t lds = sizeof(T) * ((size_t)slices * 5 * s->npad + 5 * (size_t)s->n);
   if (sizeof(T) == 4) lds = ((lds + 15) & ~(size_t)15) + sizeof(double) * (size_t)slices * s->npad;   // FP64 values
-  hipLaunchKernelGGL(k_spo_rows<T>, dim3(s->N, b->W), dim3(nt), lds, b->stream, s->params<T>(), b->params<T>(),
-                     slices);
+  const SysP<T> S = s->params<T>();
+  const BatchP<T> B = b->params<T>();
+  const long long np = (long long)s->N * b->W;
+  if (np > INT_MAX) return fail(QMCX_ERR_ARG, "walkers x electrons too large");
+  if (nq > kOrderedThreads || np < kOrderPoints || np * 64 < kOrderReuse * (long long)s->ng[0] * s->ng[1] * s->ng[2]) {
+    hipLaunchKernelGGL(k_spo_rows<T>, dim3(s->N, b->W), dim3(nt), lds, b->stream, S, B, slices);
+    HIPCHK(hipGetLastError());
+    return 0;
+  }
+  if (!b->order) {
+    HIPCHK(hipMalloc(&b->order, sizeof(int) * (2 * (size_t)np + 2 * (size_t)kBlockKeys)));
+    b->allocs.push_back(b->order);
+  }
+  int *key = b->order + np, *kcnt = key + np, *kcur = kcnt + kBlockKeys;
+  const GridBlocks nb = grid_blocks(s);
+  const int grid = (int)std::min<long long>((np + 255) / 256, 1024);
+  hipLaunchKernelGGL(k_zero_ints, dim3(16), dim3(256), 0, b->stream, kcnt, nb.keys());
+  hipLaunchKernelGGL(k_electron_keys<T>, dim3(grid), dim3(256), 0, b->stream, S, B, nb, key, kcnt);
+  hipLaunchKernelGGL(k_key_offsets, dim3(1), dim3(1024), 0, b->stream, kcnt, kcur, nb.keys());
+  hipLaunchKernelGGL(k_key_scatter, dim3(grid), dim3(256), 0, b->stream, nullptr, (int)np, key, kcur, b->order);
+  auto rows = [&](auto per) {
+    auto kern = [&](auto v64) {
+      hipLaunchKernelGGL((k_spo_rows_ordered<T, decltype(per)::value, decltype(v64)::value>),
+                         dim3((unsigned)((np + 7) / 8 * 8)), dim3((nq + 63) / 64 * 64), 0, b->stream, S, B, b->order);
+    };
+    if (B.A64 != nullptr) kern(std::true_type{});
+    else kern(std::false_type{});
+  };
+  switch (16 / slices) {
+    case 1: rows(std::integral_constant<int, 1>{}); break;
+    case 2: rows(std::integral_constant<int, 2>{}); break;
+    case 4: rows(std::integral_constant<int, 4>{}); break;
+    case 8: rows(std::integral_constant<int, 8>{}); break;
+    default: rows(std::integral_constant<int, 16>{}); break;
+  }
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -727,12 +776,20 @@ int launch_gl(qmcx_batch_t b, bool record) {
 template <typename T>
 int evaluate_log_impl(qmcx_batch_t b) {
   const qmcx_system_s* s = b->sys;
-  if (launch_spo_rows<T>(b)) return QMCX_ERR_HIP;
-  if (launch_lu_batch<T>(b)) return QMCX_ERR_HIP;
+  // the Jastrow sums need the positions only: they run on the recompute stream beside the SPO rows.
+  // Without a three-body Jastrow (whose sums read every electron's ion mask) a walker's electrons are
+  // split over workgroups of 128: at NiO-64 with 128 walkers 0.70 ms by a workgroup per walker
+  HIPCHK(hipEventRecord(b->ev_start, b->stream));
+  HIPCHK(hipStreamWaitEvent(b->aux, b->ev_start, 0));
   // positions, reduction scratch, functors, the minimum-image cell and the J3 ion masks
   const size_t lds = jastrow_init_lds<T>(s->N, s->has_j3 ? s->mw : 0);
-  hipLaunchKernelGGL(k_jastrow_init<T>, dim3(b->W), dim3(1024), lds, b->stream, s->params<T>(), b->params<T>());
+  const dim3 jgrid(b->W, b->j3 ? 1 : (s->N + 127) / 128), jblock(b->j3 ? 1024 : 128);
+  hipLaunchKernelGGL(k_jastrow_init<T>, jgrid, jblock, lds, b->aux, s->params<T>(), b->params<T>());
   HIPCHK(hipGetLastError());
+  HIPCHK(hipEventRecord(b->ev_gl, b->aux));
+  if (int rc = launch_spo_rows<T>(b)) return rc;
+  if (launch_lu_batch<T>(b)) return QMCX_ERR_HIP;
+  HIPCHK(hipStreamWaitEvent(b->stream, b->ev_gl, 0));
   HIPCHK(hipMemsetAsync(b->ndelay, 0, sizeof(int) * b->W * 2 * b->nch, b->stream));
   return launch_gl<T>(b, false);
 }
@@ -1281,16 +1338,6 @@ static int launch_virtual_ratios(qmcx_batch_t b, int iel, int nvp, const double*
   return 0;
 }
 
-// blocks of the NonLocalPP knot order: 4 grid cells per axis, more while the blocks outnumber kNlppKeys
-constexpr int kNlppKeys = 32768;
-static NlppBlocks nlpp_blocks(const qmcx_system_s* s) {
-  NlppBlocks nb;
-  for (nb.shift = 2;; ++nb.shift) {
-    for (int d = 0; d < 3; ++d) nb.nb[d] = (s->ng[d] + (1 << nb.shift) - 1) >> nb.shift;
-    if ((long long)nb.nb[0] * nb.nb[1] * nb.nb[2] <= kNlppKeys) return nb;
-  }
-}
-
 // LK lanes per knot with Q 16-byte orbital groups each; take: runs of 64 / LK knots a wave takes at a time
 template <typename T, int LK, int Q>
 static int launch_nlpp_ratios(qmcx_batch_t b, int maxp, int take, const int* units, const int* cnt) {
@@ -1314,7 +1361,7 @@ static int launch_nlpp(qmcx_batch_t b, double rmax, int maxp) {
   const int WN = b->W * s->N;
   // nl_items: pair list [WN*maxp], its length, per-key counts and cursors, the knots' keys and the
   // ordered knots [WN*maxp*12 each]
-  const NlppBlocks nb = nlpp_blocks(s);
+  const GridBlocks nb = grid_blocks(s);
   const int nkeys = nb.keys();
   const size_t cap = (size_t)WN * maxp;
   int* cnt = b->nl_items + cap;
@@ -1339,8 +1386,8 @@ static int launch_nlpp(qmcx_batch_t b, double rmax, int maxp) {
   const int kgrid = (int)std::min<size_t>((cap * kNlppKnots + 255) / 256, 1024);
   hipLaunchKernelGGL(k_nlpp_keys<T>, dim3(kgrid), dim3(256), 0, b->stream, S, B, b->nl_sph, maxp, b->nl_near,
                      b->nl_items, cnt, nb, ukey, kcnt);
-  hipLaunchKernelGGL(k_nlpp_offsets, dim3(1), dim3(1024), 0, b->stream, kcnt, kcur, nkeys);
-  hipLaunchKernelGGL(k_nlpp_scatter, dim3(kgrid), dim3(256), 0, b->stream, cnt, ukey, kcur, units);
+  hipLaunchKernelGGL(k_key_offsets, dim3(1), dim3(1024), 0, b->stream, kcnt, kcur, nkeys);
+  hipLaunchKernelGGL(k_key_scatter, dim3(kgrid), dim3(256), 0, b->stream, cnt, kNlppKnots, ukey, kcur, units);
   HIPCHK(hipGetLastError());
   // the fewest lanes per knot that hold its orbitals in at most three groups each (four past 192
   // groups): a wave then works on several knots of a small system, and no lane idles at NiO-64
@@ -2289,7 +2336,7 @@ int qmcx_nlpp_evaluate(qmcx_batch_t b, double rmax, const double* spheres, int m
     HIPCHK(hipMalloc(&b->nl_near, sizeof(double) * 4 * WN * max_pairs));
     HIPCHK(hipMalloc(&b->nl_jexp, sizeof(double) * WN * max_pairs * kNlppKnots));
     HIPCHK(hipMalloc(&b->nl_items,
-                     sizeof(int) * (WN * max_pairs * (1 + 2 * kNlppKnots) + 1 + 2 * (size_t)kNlppKeys)));
+                     sizeof(int) * (WN * max_pairs * (1 + 2 * kNlppKnots) + 1 + 2 * (size_t)kBlockKeys)));
     b->nl_cap = max_pairs;
   }
   if (!b->nl_sph) HIPCHK(hipMalloc(&b->nl_sph, sizeof(double) * 3 * kNlppKnots * (size_t)b->W));

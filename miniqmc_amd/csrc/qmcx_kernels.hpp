@@ -150,7 +150,9 @@ __device__ inline void knot_weight(int i, T t, T& w, T& dw, T& d2w) {
 // orbital q*VW + e, and with V64 the FP64 values acc64.  False for the lanes past the slices.
 // UNI (one slice only): the point is the same on every lane of the wave, so its grid cell moves
 // to scalar registers and every load takes a scalar address plus the lane's orbital offset.
-template <typename T, int NO, int PER, bool V64, bool UNI = false>
+// KEEP: cached loads (the points are ordered by place, so neighbours want the same coefficients);
+// else non-temporal ones.
+template <typename T, int NO, int PER, bool V64, bool UNI = false, bool KEEP = false>
 __device__ inline bool spline_gather_regs(const SysP<T>& S, const double* spoG, double x, double y, double z, int tid,
                                           T (&acc)[NO][V16<T>::n], double (&acc64)[V16<T>::n], int& q, int& s) {
   using VT = typename V16<T>::type;
@@ -198,8 +200,13 @@ __device__ inline bool spline_gather_regs(const SysP<T>& S, const double* spoG, 
     const int p = s * PER + g0 + pp;
     const T* src = base0 + (size_t)(p >> 2) * S.xs + (size_t)(p & 3) * S.ys;
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      v4[pp][k] = __builtin_nontemporal_load(reinterpret_cast<const VT*>(src + k * zs + lane_off));
+    for (int k = 0; k < 4; ++k) {
+      const VT* c4 = reinterpret_cast<const VT*>(src + k * zs + lane_off);
+      if constexpr (KEEP)
+        v4[pp][k] = *c4;
+      else
+        v4[pp][k] = __builtin_nontemporal_load(c4);
+    }
   }
 #pragma unroll
   for (int pp = 0; pp < G; ++pp) {
@@ -962,6 +969,31 @@ inline hipError_t launch_gj_invert(int n, int nmat, hipStream_t st, const TI* A,
 }
 
 // ------------------------------------------------------------------ SPO rows (evaluateLog)
+// Blocks of 2^shift grid cells per axis, nb blocks per axis: the key of a point is its block's index
+struct GridBlocks {
+  int shift, nb[3];
+  __host__ __device__ int keys() const { return nb[0] * nb[1] * nb[2]; }
+};
+template <typename T>
+__device__ inline int block_key(const SysP<T>& S, const GridBlocks& nb, double x, double y, double z) {
+  int ix[3];
+  double t[3];
+  spline_locate(S.spoG, S.ng, x, y, z, ix, t);
+  return ((ix[0] >> nb.shift) * nb.nb[1] + (ix[1] >> nb.shift)) * nb.nb[2] + (ix[2] >> nb.shift);
+}
+// keys of the electrons' positions (point w*N + e) and the per-key counts
+template <typename T>
+__global__ __launch_bounds__(256) void k_electron_keys(SysP<T> S, BatchP<T> B, GridBlocks nb, int* key, int* kcnt) {
+  const int N = S.N, np = B.W * N;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < np; i += gridDim.x * blockDim.x) {
+    const int w = i / N, e = i - w * N;
+    const double* R = B.R + (size_t)w * 3 * N;
+    const int k = block_key(S, nb, R[e], R[N + e], R[2 * N + e]);
+    key[i] = k;
+    atomicAdd(kcnt + k, 1);
+  }
+}
+
 // SPO at every electron of every walker -> A, dpsiM, d2psiM
 // (evaluate_notranspose, SPOSet.h:94; DiracDeterminant.cpp:264-280).
 template <typename T>
@@ -994,6 +1026,73 @@ __global__ __launch_bounds__(1024) void k_spo_rows(SysP<T> S, BatchP<T> B, int s
     dp[2 * n + j] = out[3 * n + j];
     d2[j] = out[4 * n + j];
   }
+}
+
+// The same for many electrons, which come ordered by the block of grid cells they are in, each XCD
+// (workgroup b runs on XCD b % 8) over a contiguous eighth of them, so that electrons whose
+// stencils overlap share an L2.  A workgroup takes an electron, a lane an orbital quad with all 64
+// stencil points, stored from registers; the sums go slice by slice (16 / PER slices of PER columns
+// each) in the order k_spo_rows adds them, so the rows are the same bit for bit.
+// Bound: L2 bandwidth of the stencils.  NiO-64 FP32, 98k electrons: 0.95 ms; unordered, from HBM with
+// eight slices reduced through LDS, 2.40 ms (4.0 TB/s); ordered in that form still 2.39.  The slice loop
+// is kept rolled: unrolled it spills and takes 2.0 ms.
+constexpr int kOrderedThreads = 256;
+template <typename T, int PER, bool V64>
+__global__ __launch_bounds__(kOrderedThreads) void k_spo_rows_ordered(SysP<T> S, BatchP<T> B, const int* order) {
+  using VT = typename V16<T>::type;
+  constexpr int VW = V16<T>::n, SL = 16 / PER;
+  const int N = S.N, n = S.n, nq = S.npad / VW;
+  const int np = B.W * N, x = blockIdx.x & 7, lo = (int)((long long)np * x / 8), hi = (int)((long long)np * (x + 1) / 8);
+  const int k = lo + (int)(blockIdx.x >> 3), qd = threadIdx.x;
+  if (k >= hi || qd >= nq) return;   // the grid is rounded up per XCD
+  const int at = order[k], w = at / N, e = at - w * N;
+  const double* R = B.R + (size_t)w * 3 * N;
+  const int det = e < n ? 0 : 1, row = e - det * n;
+  const size_t moff = ((size_t)w * 2 + det) * n * n;
+  const double px = R[e], py = R[N + e], pz = R[2 * N + e];
+  T sum[5][VW], acc[5][VW];
+  double sum64[VW], acc64[VW];
+#pragma unroll
+  for (int v = 0; v < VW; ++v) {
+    sum64[v] = 0.0;
+#pragma unroll
+    for (int o = 0; o < 5; ++o) sum[o][v] = T(0);
+  }
+#pragma unroll 1
+  for (int sl = 0; sl < SL; ++sl) {
+    int q, s;
+    spline_gather_regs<T, 5, PER, V64, false, true>(S, S.spoG, px, py, pz, qd + sl * nq, acc, acc64, q, s);
+#pragma unroll
+    for (int v = 0; v < VW; ++v) {
+      if constexpr (V64) sum64[v] += acc64[v];
+#pragma unroll
+      for (int o = 0; o < 5; ++o) sum[o][v] += acc[o][v];
+    }
+  }
+  const T gx = (T)S.ng[0], gy = (T)S.ng[1], gz = (T)S.ng[2];
+  T* Arow = B.A + moff + (size_t)row * n;
+  T* dp = B.dpsiM + ((size_t)w * 2 + det) * (size_t)n * 3 * n + (size_t)row * 3 * n;
+  T* d2 = B.d2psiM + moff + (size_t)row * n;
+  T* dst[5] = {Arow, dp, dp + n, dp + 2 * n, d2};
+  const int j = qd * VW;
+#pragma unroll
+  for (int o = 0; o < 5; ++o) {
+    const T f = vgh_scale<T>(o, gx, gy, gz);
+    if (n % VW == 0) {
+      VT v;
+#pragma unroll
+      for (int c = 0; c < VW; ++c) v[c] = sum[o][c] * f;
+      if (j < n) *reinterpret_cast<VT*>(dst[o] + j) = v;
+    } else {
+#pragma unroll
+      for (int c = 0; c < VW; ++c)
+        if (j + c < n) dst[o][j + c] = sum[o][c] * f;
+    }
+  }
+  if constexpr (V64)
+#pragma unroll
+    for (int c = 0; c < VW; ++c)
+      if (j + c < n) B.A64[moff + (size_t)row * n + j + c] = sum64[c];
 }
 
 // SPO values (v, d/dx, d/dy, d/dz, d2/dx2; einspline_spo.hpp:204-223) at the proposals of
@@ -1280,7 +1379,7 @@ __global__ __launch_bounds__(1024) void k_virtual_ratios(SysP<T> S, BatchP<T> B,
 // NonLocalPP::randomize, NonLocalPP.hpp:100-113, miniqmc.cpp:470).
 // k_nlpp_jastrow: the Jastrow exponents of the listed pairs' knots, jexp[item][12], walker by walker
 // (its positions and the functors in LDS, a wave per pair, lanes over the electrons).
-// k_nlpp_keys, k_nlpp_offsets and k_nlpp_scatter order all the knots (unit = pos * 12 + knot) by the
+// k_nlpp_keys, k_key_offsets and k_key_scatter order all the knots (unit = pos * 12 + knot) by the
 // block of spline grid cells they fall in, and k_nlpp_ratios walks that order, each XCD over a
 // contiguous eighth of it: knots whose stencils overlap run at the same time on CUs that share an
 // L2, so the orbital table is read from HBM about once instead of once per knot.  ratios[pos][12] =
@@ -1336,11 +1435,6 @@ __global__ __launch_bounds__(256) void k_nlpp_pairs(SysP<T> S, BatchP<T> B, doub
   for (int p = 0; p < m; ++p) items[pos + p] = idx * maxp + p;
 }
 
-// Blocks of 2^shift grid cells per axis, nb blocks per axis: the key of a knot is its block's index
-struct NlppBlocks {
-  int shift, nb[3];
-  __host__ __device__ int keys() const { return nb[0] * nb[1] * nb[2]; }
-};
 // the point of unit u (pair u / 12, knot u % 12); w, e: the pair's walker and electron
 template <typename T>
 __device__ inline void nlpp_point(const SysP<T>& S, const BatchP<T>& B, const double* spheres, int maxp,
@@ -1361,14 +1455,13 @@ __device__ inline void nlpp_point(const SysP<T>& S, const BatchP<T>& B, const do
 template <typename T>
 __global__ __launch_bounds__(256) void k_nlpp_keys(SysP<T> S, BatchP<T> B, const double* spheres, int maxp,
                                                    const double* near, const int* items, const int* cnt,
-                                                   NlppBlocks nb, int* ukey, int* kcnt) {
+                                                   GridBlocks nb, int* ukey, int* kcnt) {
   const int nu = cnt[0] * kNlppKnots;
   for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nu; u += gridDim.x * blockDim.x) {
-    int w, e, ix[3];
-    double p[3], t[3];
+    int w, e;
+    double p[3];
     nlpp_point(S, B, spheres, maxp, near, items, u, w, e, p);
-    spline_locate(S.spoG, S.ng, p[0], p[1], p[2], ix, t);
-    const int key = ((ix[0] >> nb.shift) * nb.nb[1] + (ix[1] >> nb.shift)) * nb.nb[2] + (ix[2] >> nb.shift);
+    const int key = block_key(S, nb, p[0], p[1], p[2]);
     ukey[u] = key;
     atomicAdd(kcnt + key, 1);
   }
@@ -1376,7 +1469,7 @@ __global__ __launch_bounds__(256) void k_nlpp_keys(SysP<T> S, BatchP<T> B, const
 
 // Exclusive prefix of the per-key counts into the per-key cursors.  One workgroup of 1024 lanes:
 // each lane sums a contiguous run of keys, the run sums are scanned, each lane writes its cursors.
-__global__ __launch_bounds__(1024) void k_nlpp_offsets(const int* kcnt, int* kcur, int nkeys) {
+__global__ __launch_bounds__(1024) void k_key_offsets(const int* kcnt, int* kcur, int nkeys) {
   __shared__ int run[16];
   const int t = threadIdx.x, lane = t & 63, wid = t >> 6, per = (nkeys + 1023) / 1024, a = min(t * per, nkeys);
   const int b = min(a + per, nkeys);
@@ -1398,8 +1491,9 @@ __global__ __launch_bounds__(1024) void k_nlpp_offsets(const int* kcnt, int* kcu
   }
 }
 
-__global__ __launch_bounds__(256) void k_nlpp_scatter(const int* cnt, const int* ukey, int* kcur, int* units) {
-  const int nu = cnt[0] * kNlppKnots;
+// points u (cnt[0] * per of them) to their places in the order of their keys
+__global__ __launch_bounds__(256) void k_key_scatter(const int* cnt, int per, const int* ukey, int* kcur, int* units) {
+  const int nu = (cnt != nullptr ? cnt[0] : 1) * per;
   for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nu; u += gridDim.x * blockDim.x)
     units[atomicAdd(kcur + ukey[u], 1)] = u;
 }
@@ -1626,6 +1720,7 @@ template <typename T>
 __global__ __launch_bounds__(1024) void k_jastrow_init(SysP<T> S, BatchP<T> B) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int w = blockIdx.x, tid = threadIdx.x, nt = blockDim.x, N = S.N, n = S.n, M = S.M;
+  const int i0 = blockIdx.y * nt;   // gridDim.y > 1 (no three-body Jastrow): nt electrons per workgroup
   double* sR = (double*)smem;
   double* sRed = sR + 3 * N;
   Functor<T>* sFn = (Functor<T>*)(sRed + 48);
@@ -1645,7 +1740,7 @@ __global__ __launch_bounds__(1024) void k_jastrow_init(SysP<T> S, BatchP<T> B) {
   T* J2 = B.J2 + (size_t)w * 5 * N;
   T* J1 = B.J1 + (size_t)w * 5 * N;
   double vsum = 0, usum = 0, tsum = 0;
-  for (int i = tid; i < N; i += nt) {
+  for (int i = i0 + tid; i < N; i += nt * gridDim.y) {
     const double x = sR[i], y = sR[N + i], z = sR[2 * N + i];
     T v = 0, gx = 0, gy = 0, gz = 0, lap = 0;
     T* rec = j3 ? B.j3near + ((size_t)w * N + i) * kJ3Rec : nullptr;
@@ -1753,6 +1848,7 @@ __global__ __launch_bounds__(1024) void k_jastrow_init(SysP<T> S, BatchP<T> B) {
       tsum += (double)acc[0];
     }
   }
+  if (gridDim.y > 1) return;   // the logs come with evaluateGL, which follows
   double red[3] = {vsum, usum, tsum};
   block_sum<double, 3>(red, sRed);
   if (tid == 0) {
