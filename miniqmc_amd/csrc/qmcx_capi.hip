@@ -699,7 +699,8 @@ GridBlocks grid_blocks(const qmcx_system_s* s) {
 
 // evaluateLog's electrons are ordered by place when there are this many (the four ordering launches take
 // about 30 us, as long as the rows of a few thousand electrons), and their stencils cover the grid
-// this many times over (else there is little to share)
+// this many times over (else there is little to share).  Batches that keep FP64 Slater rows are not: their
+// FP32 rows would round differently.
 constexpr long long kOrderPoints = 8192, kOrderReuse = 4;
 
 template <typename T>
@@ -715,7 +716,7 @@ int launch_spo_rows(qmcx_batch_t b) {
   const BatchP<T> B = b->params<T>();
   const long long np = (long long)s->N * b->W;
   if (np > INT_MAX) return fail(QMCX_ERR_ARG, "walkers x electrons too large");
-  if (nq > kOrderedThreads || np < kOrderPoints || np * 64 < kOrderReuse * (long long)s->ng[0] * s->ng[1] * s->ng[2]) {
+  if (B.A64 != nullptr || nq > kOrderedThreads || np < kOrderPoints || np * 64 < kOrderReuse * (long long)s->ng[0] * s->ng[1] * s->ng[2]) {
     hipLaunchKernelGGL(k_spo_rows<T>, dim3(s->N, b->W), dim3(nt), lds, b->stream, S, B, slices);
     HIPCHK(hipGetLastError());
     return 0;
@@ -732,12 +733,8 @@ int launch_spo_rows(qmcx_batch_t b) {
   hipLaunchKernelGGL(k_key_offsets, dim3(1), dim3(1024), 0, b->stream, kcnt, kcur, nb.keys());
   hipLaunchKernelGGL(k_key_scatter, dim3(grid), dim3(256), 0, b->stream, nullptr, (int)np, key, kcur, b->order);
   auto rows = [&](auto per) {
-    auto kern = [&](auto v64) {
-      hipLaunchKernelGGL((k_spo_rows_ordered<T, decltype(per)::value, decltype(v64)::value>),
-                         dim3((unsigned)((np + 7) / 8 * 8)), dim3((nq + 63) / 64 * 64), 0, b->stream, S, B, b->order);
-    };
-    if (B.A64 != nullptr) kern(std::true_type{});
-    else kern(std::false_type{});
+    hipLaunchKernelGGL((k_spo_rows_ordered<T, decltype(per)::value>), dim3((unsigned)((np + 7) / 8 * 8)),
+                       dim3((nq + 63) / 64 * 64), 0, b->stream, S, B, b->order);
   };
   switch (16 / slices) {
     case 1: rows(std::integral_constant<int, 1>{}); break;

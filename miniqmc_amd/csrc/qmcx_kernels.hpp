@@ -1037,7 +1037,7 @@ __global__ __launch_bounds__(1024) void k_spo_rows(SysP<T> S, BatchP<T> B, int s
 // eight slices reduced through LDS, 2.40 ms (4.0 TB/s); ordered in that form still 2.39.  The slice loop
 // is kept rolled: unrolled it spills and takes 2.0 ms.
 constexpr int kOrderedThreads = 256;
-template <typename T, int PER, bool V64>
+template <typename T, int PER>
 __global__ __launch_bounds__(kOrderedThreads) void k_spo_rows_ordered(SysP<T> S, BatchP<T> B, const int* order) {
   using VT = typename V16<T>::type;
   constexpr int VW = V16<T>::n, SL = 16 / PER;
@@ -1051,20 +1051,18 @@ __global__ __launch_bounds__(kOrderedThreads) void k_spo_rows_ordered(SysP<T> S,
   const size_t moff = ((size_t)w * 2 + det) * n * n;
   const double px = R[e], py = R[N + e], pz = R[2 * N + e];
   T sum[5][VW], acc[5][VW];
-  double sum64[VW], acc64[VW];
+  double acc64[VW];   // not used
 #pragma unroll
   for (int v = 0; v < VW; ++v) {
-    sum64[v] = 0.0;
 #pragma unroll
     for (int o = 0; o < 5; ++o) sum[o][v] = T(0);
   }
 #pragma unroll 1
   for (int sl = 0; sl < SL; ++sl) {
     int q, s;
-    spline_gather_regs<T, 5, PER, V64, false, true>(S, S.spoG, px, py, pz, qd + sl * nq, acc, acc64, q, s);
+    spline_gather_regs<T, 5, PER, false, false, true>(S, S.spoG, px, py, pz, qd + sl * nq, acc, acc64, q, s);
 #pragma unroll
     for (int v = 0; v < VW; ++v) {
-      if constexpr (V64) sum64[v] += acc64[v];
 #pragma unroll
       for (int o = 0; o < 5; ++o) sum[o][v] += acc[o][v];
     }
@@ -1089,10 +1087,6 @@ __global__ __launch_bounds__(kOrderedThreads) void k_spo_rows_ordered(SysP<T> S,
         if (j + c < n) dst[o][j + c] = sum[o][c] * f;
     }
   }
-  if constexpr (V64)
-#pragma unroll
-    for (int c = 0; c < VW; ++c)
-      if (j + c < n) B.A64[moff + (size_t)row * n + j + c] = sum64[c];
 }
 
 // SPO values (v, d/dx, d/dy, d/dz, d2/dx2; einspline_spo.hpp:204-223) at the proposals of
