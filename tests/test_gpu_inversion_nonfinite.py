@@ -1,0 +1,78 @@
+"""The FP64 inversion of matrices with NaN and infinite entries: where the results of the textbook
+elimination (partial pivoting with row exchanges, in numpy) are NaN or infinite, the kernel's are."""
+import numpy as np
+import pytest
+
+from miniqmc_amd import qmcx
+
+pytestmark = pytest.mark.gpu
+
+
+def gauss_jordan(a):
+    """(A^-1)^T and the pivots of X = A^T by blocked in-place elimination with row exchanges; a NaN is never
+    the largest candidate, and the row in the pivot's place is the pivot when all candidates are NaN."""
+    n = len(a)
+    width = 32 if n <= 512 else 16
+    x = a.T.copy()
+    cols, pivots = np.arange(n), []
+    for k0 in range(0, n, width):
+        b = min(width, n - k0)
+        panel, swaps = x[:, k0:k0 + b].copy(), []
+        for j in range(b):
+            k = k0 + j
+            cand = np.where(np.isnan(panel[k:, j]), -1.0, np.abs(panel[k:, j]))
+            p = k + int(np.argmax(cand)) if cand.max() >= 0 else k
+            panel[[k, p]] = panel[[p, k]]
+            swaps.append((k, p))
+            pivots.append(panel[k, j])
+            inv = 1.0 / panel[k, j]
+            row, f = panel[k] * inv, panel[:, j].copy()
+            panel -= np.outer(f, row)
+            panel[:, j] = -f * inv
+            panel[k] = row
+            panel[k, j] = inv
+        for k, p in swaps:
+            x[[k, p]] = x[[p, k]]
+        rows = x[k0:k0 + b].copy()
+        x[k0:k0 + b] = 0.0
+        for t in range(b):
+            x += np.outer(panel[:, t], rows[t])
+        x[:, k0:k0 + b] = panel
+        for k, p in swaps:
+            cols[[k, p]] = cols[[p, k]]
+    out = np.empty_like(x)
+    out[:, cols] = x
+    return out, np.array(pivots)
+
+
+def check(a):
+    with np.errstate(all="ignore"):
+        ref, pivots = gauss_jordan(a)
+        log = np.log(np.abs(pivots)).sum()
+    # the matrix between two ordinary ones, which it leaves alone
+    rng = np.random.default_rng(5)
+    other = rng.standard_normal(a.shape)
+    psiM, logdet, _ = qmcx.invert_transpose(np.stack([other, a, other]))
+    alone, la, _ = qmcx.invert_transpose(other[None])
+    for m in (0, 2):
+        np.testing.assert_array_equal(psiM[m], alone[0])
+        assert logdet[m] == la[0]
+    for test in (np.isnan, np.isinf):
+        np.testing.assert_array_equal(test(psiM[1]), test(ref))
+        assert test(logdet[1]) == test(log)
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("where", ["entry", "orbital", "electron"])
+@pytest.mark.parametrize("n", [1, 20, 33, 64, 130, 384, 513])
+def test_nan_and_inf(n, where, value):
+    """One entry, one column (an orbital) or one row (an electron) of the Slater matrix."""
+    a = np.random.default_rng(n).standard_normal((n, n))
+    i, j = n // 3, n // 2
+    if where == "entry":
+        a[i, j] = value
+    elif where == "orbital":
+        a[:, j] = value
+    else:
+        a[i] = value
+    check(a)
