@@ -802,7 +802,6 @@ __global__ __launch_bounds__(NT) void k_gj_invert(int n, const TI* A, TO* psiM, 
   const bool own = tid < n;
   bool used = false;   // this thread's row has been a pivot
   unsigned par = 0;    // parity of the wave's unused rows below each pivot (the permutation's inversions)
-  int knan = n;        // first step whose pivot is a NaN
   for (int i = tid; i < ns; i += NT) {
     piv[i] = min(i, n - 1);
     kof[i] = INT_MAX;
@@ -832,7 +831,8 @@ __global__ __launch_bounds__(NT) void k_gj_invert(int n, const TI* A, TO* psiM, 
         // largest magnitude and its first lane, then the waves' candidates side by side in the
         // lanes of every wave.  Candidates and pivot rows alternate between two slots, so a step
         // needs no barrier between its reads and the next step's writes
-        const double av = (own && !used) ? fabs(prj) : -1.0;
+        // (a NaN, which a maximum never takes, is the pivot once no other row is left)
+        const double av = (own && !used) ? fmax(fabs(prj), -0.5) : -1.0;
         const double best = wave_max(av);
         const unsigned long long hit = __ballot(av == best);
         if (lane == 0) {
@@ -848,16 +848,14 @@ __global__ __launch_bounds__(NT) void k_gj_invert(int n, const TI* A, TO* psiM, 
         cb = dpp_max<0x141, 0xf>(cb);   // of eight lanes
         if constexpr (nw > 8) cb = dpp_max<0x140, 0xf>(cb);
         const int qb = max(__ffsll((long long)__ballot(cv == cb)) - 1, 0);
-        // a maximum never takes a NaN: once every row left has a NaN candidate (its NaN is then the
-        // pivot, and the whole inverse NaN) no step takes a pivot any more
-        if (__ballot(cb >= 0.0) == 0) knan = min(knan, k);
-        const int p = knan > k ? __builtin_amdgcn_readlane(cr, qb) : -1;   // in [0, n), or none
+        const int p = __builtin_amdgcn_readlane(cr, qb);   // in [0, n)
         const bool isp = tid == p;
         par ^= (unsigned)__popcll(__ballot(own && !used && tid < p)) & 1u;
         const double rinv = 1.0 / cb;   // 1 / |pivot|
         if (isp) {
           // the scaled pivot row for the others; its own new entries are left to the update below
-          const double dinv = prj < 0.0 ? -rinv : rinv;
+          double dinv = prj < 0.0 ? -rinv : rinv;
+          if (prj != prj) dinv = prj;
 #pragma unroll
           for (int c = 0; c < B; ++c) {
             pw[c] = pr[c] * dinv;
@@ -879,28 +877,13 @@ __global__ __launch_bounds__(NT) void k_gj_invert(int n, const TI* A, TO* psiM, 
         pr[j] = -f * pw[B];
       }
     }
-    if (own)
+    if (own) {
 #pragma unroll
       for (int c = 0; c < B; ++c) P[(size_t)c * ns + tid] = pr[c];
-    __syncthreads();
-    if (knan < n) {
-      // the pivots that are left, for the permutation's sign: the row that row exchanges would have
-      // brought to place k.  Place k held row k first, and a step t that took the row of place k put that
-      // of its own place t there
-      for (int k = knan; k < n; ++k) {
-        int p = k;
-        for (int t = kof[p]; t < k; t = kof[p]) p = t;
-        par ^= (unsigned)__popcll(__ballot(own && !used && tid < p)) & 1u;
-        __syncthreads();
-        if (tid == p) {
-          dv[k] = __builtin_nan("");
-          kof[p] = k;
-          used = true;
-        }
-        __syncthreads();
-      }
-      break;
+      // zeros past bb (a zero pivot's scaled row is NaN there): the update multiplies all B columns
+      for (int c = bb; c < B; ++c) P[(size_t)c * ns + tid] = 0.0;
     }
+    __syncthreads();
     // ---- the other columns, then the panel itself, back to Y
     if (k0 == 0)
       gj_update<TI, B>(n, ns, k0, bb, a, Y, P, piv, kof);
@@ -911,6 +894,26 @@ __global__ __launch_bounds__(NT) void k_gj_invert(int n, const TI* A, TO* psiM, 
     __syncthreads();
   }
 
+  // ---- from the first NaN pivot on every entry is NaN and the rows left were taken in ascending order;
+  // the sign is that of row exchanges: place k's row is the pivot.  Place k held row k first, and a step
+  // t that took the row of place k put that of its own place t there
+  const int knan = n - __syncthreads_count(own && dv[tid] != dv[tid]);
+  if (knan < n) {
+    used = own && kof[tid] < knan;
+    if (own && !used) kof[tid] = INT_MAX;
+    __syncthreads();
+    for (int k = knan; k < n; ++k) {
+      int p = k;
+      for (int t = kof[p]; t < k; t = kof[p]) p = t;
+      par ^= (unsigned)__popcll(__ballot(own && !used && tid < p)) & 1u;
+      __syncthreads();
+      if (tid == p) {
+        kof[p] = k;
+        used = true;
+      }
+      __syncthreads();
+    }
+  }
   // ---- log|det| and phase: the product of the pivots as mantissa and binary exponent, the parity
   // of the row permutation and of the negative pivots
   {
@@ -967,7 +970,7 @@ __global__ __launch_bounds__(NT) void k_gj_invert(int n, const TI* A, TO* psiM, 
     __syncthreads();
     for (int e = tid; e < n * B; e += NT) {
       const int k = e / B, c = e % B;
-      if (c < jb) out[(size_t)k * n + j0 + c] = knan < n ? (TO)__builtin_nan("") : (TO)P[(size_t)c * (ns + 1) + piv[k]];
+      if (c < jb) out[(size_t)k * n + j0 + c] = (TO)P[(size_t)c * (ns + 1) + piv[k]];
     }
     __syncthreads();
   }

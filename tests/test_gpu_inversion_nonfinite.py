@@ -9,12 +9,12 @@ pytestmark = pytest.mark.gpu
 
 
 def gauss_jordan(a):
-    """(A^-1)^T and the pivots of X = A^T by blocked in-place elimination with row exchanges; a NaN is never
-    the largest candidate, and the row in the pivot's place is the pivot when all candidates are NaN."""
+    """(A^-1)^T, the pivots of X = A^T and the number of row exchanges, by blocked in-place elimination.  A NaN
+    is never the largest candidate; the row in the pivot's place is the pivot when all candidates are NaN."""
     n = len(a)
     width = 32 if n <= 512 else 16
     x = a.T.copy()
-    cols, pivots = np.arange(n), []
+    cols, pivots, exchanges = np.arange(n), [], 0
     for k0 in range(0, n, width):
         b = min(width, n - k0)
         panel, swaps = x[:, k0:k0 + b].copy(), []
@@ -24,6 +24,7 @@ def gauss_jordan(a):
             p = k + int(np.argmax(cand)) if cand.max() >= 0 else k
             panel[[k, p]] = panel[[p, k]]
             swaps.append((k, p))
+            exchanges += p != k
             pivots.append(panel[k, j])
             inv = 1.0 / panel[k, j]
             row, f = panel[k] * inv, panel[:, j].copy()
@@ -42,17 +43,17 @@ def gauss_jordan(a):
             cols[[k, p]] = cols[[p, k]]
     out = np.empty_like(x)
     out[:, cols] = x
-    return out, np.array(pivots)
+    return out, np.array(pivots), exchanges
 
 
 def check(a):
     with np.errstate(all="ignore"):
-        ref, pivots = gauss_jordan(a)
+        ref, pivots, exchanges = gauss_jordan(a)
         log = np.log(np.abs(pivots)).sum()
     # the matrix between two ordinary ones, which it leaves alone
     rng = np.random.default_rng(5)
     other = rng.standard_normal(a.shape)
-    psiM, logdet, _ = qmcx.invert_transpose(np.stack([other, a, other]))
+    psiM, logdet, phase = qmcx.invert_transpose(np.stack([other, a, other]))
     alone, la, _ = qmcx.invert_transpose(other[None])
     for m in (0, 2):
         np.testing.assert_array_equal(psiM[m], alone[0])
@@ -60,6 +61,7 @@ def check(a):
     for test in (np.isnan, np.isinf):
         np.testing.assert_array_equal(test(psiM[1]), test(ref))
         assert test(logdet[1]) == test(log)
+    assert (phase[1] == 0.0) == ((exchanges + (pivots < 0).sum()) % 2 == 0)
 
 
 @pytest.mark.parametrize("value", [np.nan, np.inf])
@@ -75,4 +77,12 @@ def test_nan_and_inf(n, where, value):
         a[:, j] = value
     else:
         a[i] = value
+    check(a)
+
+
+@pytest.mark.parametrize("n", [5, 32, 33, 50, 130, 513])
+def test_zero_last_electron(n):
+    """A singular matrix whose zero pivot comes last, in a panel that is full or not."""
+    a = np.random.default_rng(n).standard_normal((n, n))
+    a[n - 1] = 0.0
     check(a)
