@@ -926,7 +926,7 @@ int moves_det(qmcx_batch_t b, int det, int mode, bool flush) {
 // The delayed rows flex_* moves left pending (state slot 0 of a determinant) reach the inverse
 // (DiracDeterminant::completeUpdates, DiracDeterminant.cpp:294-321), or, with thr > 1, only those of
 // the walkers whose pending rows reached thr; the applied slots are emptied.  The host counts the
-// rows too (the decisions are the caller's), so launches with nothing to apply are left out.
+// rows too (from the move kernel's records), so launches with nothing to apply are left out.
 template <typename T>
 int flush_slot(qmcx_batch_t b, int det, int thr) {
   if (int rc = launch_flush<T>(b, b->stream, det, 0, 1, thr)) return rc;
@@ -945,15 +945,22 @@ int flush_pending(qmcx_batch_t b) {
   b->flex_clear();
   return 0;
 }
-// the rows of determinant det's walkers that reached the delay rank (DelayedUpdate.h:151-152)
+// The rows of determinant det's walkers that reached the delay rank (DelayedUpdate.h:151-152), after an
+// accept launch.  Its decisions are not known yet (a NaN ratio rejects whatever the caller decided), so
+// this counts the caller's, which are no fewer; the kernels look at each walker's own count.
 int flush_full(qmcx_batch_t b, int det) {
-  auto& c = b->flex_cnt[det];
-  if (std::none_of(c.begin(), c.end(), [&](int x) { return x >= b->K; })) return 0;
-  const int rc = b->prec == QMCX_FP32 ? flush_slot<float>(b, det, b->K) : flush_slot<double>(b, det, b->K);
-  if (rc) return rc;
-  for (int& x : c)
-    if (x >= b->K) x = 0;
-  return 0;
+  bool any = false;
+  for (int w = 0; w < b->W; ++w) any = any || b->flex_cnt[det][w] + (b->flex_decide()[w] != 0 ? 1 : 0) >= b->K;
+  if (!any) return 0;
+  return b->prec == QMCX_FP32 ? flush_slot<float>(b, det, b->K) : flush_slot<double>(b, det, b->K);
+}
+// the accept launch's decisions, which it recorded, into the host's counts
+void count_accepted(qmcx_batch_t b, int det) {
+  for (int w = 0; w < b->W; ++w) {
+    int& c = b->flex_cnt[det][w];
+    c += b->flex_record()[9 * (size_t)w + 2] != 0.0 ? 1 : 0;
+    if (c >= b->K) c = 0;   // flush_full's launch applied them
+  }
 }
 
 // FP64 inverse of one determinant of every walker (only: of the walkers whose flag is set) from
@@ -2179,7 +2186,7 @@ static int flex_launch(qmcx_batch_t b, int iel, bool apply) {
   a.mode = QMCX_ACCEPT_METROPOLIS;
   a.slices = 0;
   a.decide = apply ? b->flex_decide() : b->flex_none;
-  a.record = apply ? nullptr : b->flex_record();
+  a.record = b->flex_record();
   // delay rank > 1: the streamed form keeps each walker's accepted rows pending in state slot 0
   // of the determinant (DelayedUpdate::acceptRow, DelayedUpdate.h:124-153) until the walker's
   // count reaches the delay rank (flushed after the accept) or completeUpdates
@@ -2198,10 +2205,8 @@ static int flex_launch(qmcx_batch_t b, int iel, bool apply) {
   if (rc) return rc;
   if (st) {
     b->flex_pending = b->flex_live[det] = true;
-    if (apply) {
-      for (int w = 0; w < b->W; ++w) b->flex_cnt[det][w] += b->flex_decide()[w] != 0 ? 1 : 0;
+    if (apply)
       if (int rc2 = flush_full(b, det)) return rc2;
-    }
   }
   return 0;
 }
@@ -2240,6 +2245,7 @@ int qmcx_flex_accept_restore(qmcx_batch_t b, int iel, const int* accepted) {
   std::memcpy(b->flex_decide(), accepted, sizeof(int) * b->W);
   if (int rc = flex_launch(b, iel, true)) return rc;
   HIPCHK(hipStreamSynchronize(b->stream));
+  if (b->K > 1) count_accepted(b, iel < b->sys->n ? 0 : 1);
   b->flex_iel = -1;
   b->flex_rows = false;
   return 0;
