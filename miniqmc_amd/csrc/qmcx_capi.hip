@@ -270,6 +270,7 @@ struct qmcx_system_s {
   bool has_j3 = false, j3_dirty = false;
   int mw = 0;
   int nbatches = 0;   // live batches of this system
+  unsigned tables = 0;   // counts changes of the device's functors and spline table
   int ng[3] = {0, 0, 0};
   int norb = 0, npad = 0;
   double spoG[9];
@@ -315,6 +316,7 @@ struct qmcx_system_s {
     return S;
   }
   int sync_functors() {
+    if (j3_dirty || fn_dirty) ++tables;
     if (j3_dirty) {
       HIPCHK(hipMemcpy(d_j3d, j3d, sizeof(j3d), hipMemcpyHostToDevice));
       HIPCHK(hipMemcpy(d_j3f, j3f, sizeof(j3f), hipMemcpyHostToDevice));
@@ -369,7 +371,8 @@ struct qmcx_batch_s {
   PinnedBuf flex_io;
   int* flex_none = nullptr;
   int flex_iel = -1;
-  bool flex_rows = false;         // spo and prop hold electron flex_iel's proposal
+  bool flex_rows = false;         // spo and prop hold electron flex_iel's proposal,
+  unsigned flex_tables = 0;       // evaluated with this state of the system's tables
   std::vector<int> flex_cnt[2];   // pending delayed rows of each walker and determinant (state slot 0)
   bool flex_live[2] = {false, false};   // slot 0 of the determinant holds the flex moves' rows
   double* flex_displ() const { return flex_io.as<double>(); }
@@ -1614,6 +1617,7 @@ int qmcx_system_set_spline(qmcx_system_t s, const int* ng, int norb, int npad, c
   if (npad < norb || npad % 4 != 0) return fail(QMCX_ERR_ARG, "npad must be >= norb and a multiple of 4");
   if (ng[0] < 1 || ng[1] < 1 || ng[2] < 1) return fail(QMCX_ERR_ARG, "grid must be positive");
   if ((precision_mask & 3) == 0) return fail(QMCX_ERR_ARG, "precision_mask selects no table");
+  ++s->tables;
   s->ng[0] = ng[0];
   s->ng[1] = ng[1];
   s->ng[2] = ng[2];
@@ -1995,6 +1999,7 @@ int qmcx_evaluate_log(qmcx_batch_t b, double* log_out) {
   int rc = b->prec == QMCX_FP32 ? evaluate_log_impl<float>(b) : evaluate_log_impl<double>(b);
   if (rc) return rc;
   b->flex_clear();   // the inverse is rebuilt from scratch: pending delayed rows are void
+  b->flex_rows = false;
   if (b->cad) {
     hipLaunchKernelGGL(k_cadence_reset, dim3((b->W + 255) / 256), dim3(256), 0, b->stream, b->cad, b->W, -1);
     HIPCHK(hipGetLastError());
@@ -2169,7 +2174,7 @@ static int flex_launch(qmcx_batch_t b, int iel, bool apply) {
   int rc = choose_shape(s, nt);
   if (rc) return rc;
   const int det = iel < s->n ? 0 : 1;
-  if (!b->flex_rows) {
+  if (!b->flex_rows || b->flex_tables != s->tables) {
     rc = f32 ? launch_proposals<float>(b, b->stream, det, iel - det * s->n, 1, 0, 1.0, b->flex_displ())
              : launch_proposals<double>(b, b->stream, det, iel - det * s->n, 1, 0, 1.0, b->flex_displ());
     if (rc) return rc;
@@ -2235,6 +2240,7 @@ int qmcx_flex_ratio_grad(qmcx_batch_t b, int iel, const double* displ, double* r
     }
   }
   b->flex_rows = true;
+  b->flex_tables = b->sys->tables;
   b->flex_iel = iel;
   return 0;
 }
