@@ -2247,7 +2247,7 @@ int qmcx_flex_ratio_grad(qmcx_batch_t b, int iel, const double* displ, double* r
 
 int qmcx_flex_accept_restore(qmcx_batch_t b, int iel, const int* accepted) {
   if (!b || !accepted) return fail(QMCX_ERR_ARG, "null argument");
-  if (iel != b->flex_iel) return fail(QMCX_ERR_STATE, "accept_restore must follow ratio_grad of the same electron");
+  if (iel < 0 || iel != b->flex_iel) return fail(QMCX_ERR_STATE, "accept_restore must follow ratio_grad of the same electron");
   std::memcpy(b->flex_decide(), accepted, sizeof(int) * b->W);
   if (int rc = flex_launch(b, iel, true)) return rc;
   HIPCHK(hipStreamSynchronize(b->stream));

@@ -43,3 +43,24 @@ def test_nan_walker(delay, precision):
     for w in range(W):
         for det in range(2):
             np.testing.assert_array_equal(a.inverse(w, det), b.inverse(w, det))
+
+
+def test_accept_without_a_proposal():
+    """Electron -1, the value that stands for no proposal, is an error before the first ratio_grad and after
+    an accept."""
+    sysd = systems.make_system("nio8-cubic")
+    dev = qmcx.System(sysd, precisions=(qmcx.FP64,))
+    wb = qmcx.WalkerBatch(dev, 2, delay_rank=2, precision=qmcx.FP64)
+    R = systems.initial_positions(sysd, 2)
+    wb.set_positions(R)
+    wb.evaluate_log()
+    yes = np.ones(2, dtype=np.int32)
+    with pytest.raises(qmcx.QmcxError):
+        wb.flex_accept_restore(-1, yes)
+    wb.flex_ratio_grad(3, np.full((2, 3), 0.1))
+    wb.flex_accept_restore(3, yes)
+    after = wb.positions()
+    for iel in (-1, 3):
+        with pytest.raises(qmcx.QmcxError):
+            wb.flex_accept_restore(iel, yes)
+    np.testing.assert_array_equal(wb.positions(), after)
