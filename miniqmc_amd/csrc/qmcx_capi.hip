@@ -718,15 +718,21 @@ int launch_spo_rows(qmcx_batch_t b) {
   const SysP<T> S = s->params<T>();
   const BatchP<T> B = b->params<T>();
   const long long np = (long long)s->N * b->W;
-  if (np > INT_MAX) return fail(QMCX_ERR_ARG, "walkers x electrons too large");
-  if (B.A64 != nullptr || nq > kOrderedThreads || np < kOrderPoints || np * 64 < kOrderReuse * (long long)s->ng[0] * s->ng[1] * s->ng[2]) {
+  bool ordered = B.A64 == nullptr && nq <= kOrderedThreads && np >= kOrderPoints && np <= INT_MAX &&
+                 np * 64 >= kOrderReuse * (long long)s->ng[0] * s->ng[1] * s->ng[2];
+  if (ordered && !b->order) {
+    if (hipMalloc(&b->order, sizeof(int) * (2 * (size_t)np + 2 * (size_t)kBlockKeys)) == hipSuccess) {
+      b->allocs.push_back(b->order);
+    } else {   // no memory for the order: the rows in the electrons' own order are the same
+      (void)hipGetLastError();
+      b->order = nullptr;
+      ordered = false;
+    }
+  }
+  if (!ordered) {
     hipLaunchKernelGGL(k_spo_rows<T>, dim3(s->N, b->W), dim3(nt), lds, b->stream, S, B, slices);
     HIPCHK(hipGetLastError());
     return 0;
-  }
-  if (!b->order) {
-    HIPCHK(hipMalloc(&b->order, sizeof(int) * (2 * (size_t)np + 2 * (size_t)kBlockKeys)));
-    b->allocs.push_back(b->order);
   }
   int *key = b->order + np, *kcnt = key + np, *kcur = kcnt + kBlockKeys;
   const GridBlocks nb = grid_blocks(s);

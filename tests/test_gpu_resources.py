@@ -1,0 +1,17 @@
+"""Runs tests/cpp/check_resources.cpp: failing allocations.
+The binary is built by __graft_entry__.build()."""
+import os
+import subprocess
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+BIN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "check_resources.bin")
+
+
+def test_cpp_resources():
+    assert os.path.exists(BIN), "build first: python -c 'import __graft_entry__ as g; g.build()'"
+    out = subprocess.run([BIN], capture_output=True, text=True, timeout=120)
+    print(out.stdout, out.stderr, flush=True)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert "All checks passed" in out.stdout
