@@ -793,9 +793,10 @@ int evaluate_log_impl(qmcx_batch_t b) {
   hipLaunchKernelGGL(k_jastrow_init<T>, jgrid, jblock, lds, b->aux, s->params<T>(), b->params<T>());
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(b->ev_gl, b->aux));
-  if (int rc = launch_spo_rows<T>(b)) return rc;
-  if (launch_lu_batch<T>(b)) return QMCX_ERR_HIP;
-  HIPCHK(hipStreamWaitEvent(b->stream, b->ev_gl, 0));
+  int rc = launch_spo_rows<T>(b);
+  if (!rc && launch_lu_batch<T>(b)) rc = QMCX_ERR_HIP;
+  HIPCHK(hipStreamWaitEvent(b->stream, b->ev_gl, 0));   // after an error too: later work may write what the sums read
+  if (rc) return rc;
   HIPCHK(hipMemsetAsync(b->ndelay, 0, sizeof(int) * b->W * 2 * b->nch, b->stream));
   return launch_gl<T>(b, false);
 }

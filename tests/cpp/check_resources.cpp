@@ -1,17 +1,20 @@
-// The library's use of HIP resources: what it does when an allocation fails.  The program
-// defines some HIP entry points itself; the library's calls reach these first, which fail the one that a check
-// asks for and pass the others on to the runtime.
+// The library's use of HIP resources: what it does when an allocation or a launch fails.  The
+// program defines some HIP entry points itself; the library's calls reach these first, which fail the one that a
+// check asks for and pass the others on to the runtime.
 #include <dlfcn.h>
 
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <random>
 #include <vector>
 
 #include "qmcx.h"
 
-static int fail_malloc = 0;   // the n-th call from now fails (0: none)
+typedef void* handle;   // hipStream_t, hipEvent_t
+static int fail_malloc = 0, fail_launch = 0;   // the n-th call from now fails (0: none)
+static std::map<handle, handle> recorded;      // event -> stream of its latest record that no other stream waited for
 static const int kOutOfMemory = 2;
 
 template <typename F>
@@ -25,6 +28,23 @@ int hipMalloc(void** p, size_t bytes) {
   static auto f = next<int (*)(void**, size_t)>("hipMalloc");
   if (fail_malloc > 0 && --fail_malloc == 0) return kOutOfMemory;
   return f(p, bytes);
+}
+int hipGetLastError() {
+  static auto f = next<int (*)()>("hipGetLastError");
+  const int e = f();
+  if (fail_launch > 0 && --fail_launch == 0) return kOutOfMemory;
+  return e;
+}
+int hipEventRecord(handle ev, handle st) {
+  static auto f = next<int (*)(handle, handle)>("hipEventRecord");
+  recorded[ev] = st;
+  return f(ev, st);
+}
+int hipStreamWaitEvent(handle st, handle ev, unsigned flags) {
+  static auto f = next<int (*)(handle, handle, unsigned)>("hipStreamWaitEvent");
+  auto it = recorded.find(ev);
+  if (it != recorded.end() && it->second != st) recorded.erase(it);
+  return f(st, ev, flags);
 }
 }
 
@@ -72,7 +92,7 @@ struct Model {
 };
 
 // evaluateLog of enough electrons for them to be ordered by place: without the memory for that it evaluates
-// them in their own order
+// them in their own order, and an error leaves no work of the side stream behind
 static void evaluate_log() {
   Model m(48, 10);
   const int W = 91;
@@ -90,6 +110,21 @@ static void evaluate_log() {
     check(fail_malloc == 0, "evaluateLog asks for memory to order its electrons");
     fail_malloc = 0;
     check(rc == 0 && la == lb, "evaluateLog without that memory gives the same log|Psi|");
+    int errors = 0;
+    for (int k = 2; k < 12; ++k) {
+      recorded.clear();
+      fail_launch = k;
+      if (qmcx_evaluate_log(a, la.data()) != 0) {
+        ++errors;
+        // ev_start, recorded on the batch's stream, was waited for by the side stream; the side
+        // stream's own event must have been waited for by the batch's
+        check(recorded.empty(), "a failed evaluateLog has joined the side stream");
+      }
+      fail_launch = 0;
+    }
+    check(errors > 0, "launches failed");
+    must(qmcx_evaluate_log(a, la.data()), "qmcx_evaluate_log");
+    check(la == lb, "evaluateLog after the errors");
     qmcx_batch_destroy(a);
     qmcx_batch_destroy(b);
   }

@@ -1,4 +1,4 @@
-"""Runs tests/cpp/check_resources.cpp: failing allocations.
+"""Runs tests/cpp/check_resources.cpp: failing allocations and launches.
 The binary is built by __graft_entry__.build()."""
 import os
 import subprocess
