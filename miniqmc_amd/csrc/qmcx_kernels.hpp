@@ -1686,7 +1686,14 @@ __global__ __launch_bounds__(256) void k_nlpp_ratios(SysP<T> S, BatchP<T> B, con
 #pragma unroll
       for (int q = 0; q < Q; ++q)
 #pragma unroll
-        for (int v = 0; v < VW; ++v) s += (double)acc[q][v] * (double)av[q][v];
+        for (int v = 0; v < VW; ++v) {
+          // the table's columns past n may hold anything: they enter as zeros, like av.  (The sum is pinned
+          // first, or the compiler computes it, loads and all, in a branch of its own: twice the time)
+          T x = acc[q][v];
+          asm volatile("" : "+v"(x));
+          x = (lk + LK * q) * VW + v < n ? x : T(0);
+          s += (double)x * (double)av[q][v];
+        }
       s = dpp_add<0xB1, 0xf>(s);   // the lane's row of 16
       s = dpp_add<0x4E, 0xf>(s);
       s = dpp_add<0x141, 0xf>(s);
