@@ -1390,13 +1390,15 @@ static int launch_nlpp(qmcx_batch_t b, double rmax, int maxp) {
                      b->nl_items, b->nl_cnt, cnt);
   // about eight workgroups per CU over the walkers, a wave for at least four electrons
   const int parts = std::max(1, std::min((s->N + 15) / 16, 2048 / b->W));
-  const size_t jlds = nlpp_jastrow_lds<T>(s->N, s->nions);
-  if (b->j3)
-    hipLaunchKernelGGL((k_nlpp_jastrow<T, true>), dim3(parts, b->W), dim3(256), jlds, b->stream, S, B, b->nl_sph, maxp,
-                       b->nl_near, b->nl_cnt, b->nl_jexp);
-  else
-    hipLaunchKernelGGL((k_nlpp_jastrow<T, false>), dim3(parts, b->W), dim3(256), jlds, b->stream, S, B, b->nl_sph, maxp,
-                       b->nl_near, b->nl_cnt, b->nl_jexp);
+  const bool il = nlpp_jastrow_lds<T>(s->N, s->nions) <= kMoveLdsMax;
+  const size_t jlds = nlpp_jastrow_lds<T>(s->N, il ? s->nions : 0);
+  auto jastrow = [&](auto kj3, auto kil) {
+    hipLaunchKernelGGL((k_nlpp_jastrow<T, decltype(kj3)::value, decltype(kil)::value>), dim3(parts, b->W), dim3(256),
+                       jlds, b->stream, S, B, b->nl_sph, maxp, b->nl_near, b->nl_cnt, b->nl_jexp);
+  };
+  if (b->j3) jastrow(std::true_type{}, std::true_type{});   // at most 256 ions
+  else if (il) jastrow(std::false_type{}, std::true_type{});
+  else jastrow(std::false_type{}, std::false_type{});
   const int kgrid = (int)std::min<size_t>((cap * kNlppKnots + 255) / 256, 1024);
   hipLaunchKernelGGL(k_nlpp_keys<T>, dim3(kgrid), dim3(256), 0, b->stream, S, B, b->nl_sph, maxp, b->nl_near,
                      b->nl_items, cnt, nb, ukey, kcnt);

@@ -1519,8 +1519,8 @@ __global__ __launch_bounds__(256) void k_key_scatter(const int* cnt, int per, co
 
 // J1, J2 (and J3) exponents of every listed pair's knots: sums at the electron's position (kept by the
 // moves) less those at the knot (OneBodyJastrow.h:136-140, TwoBodyJastrow.h:103-107,
-// ThreeBodyJastrow.h:262-273).  grid (parts, W): a workgroup stages its walker's positions, the ions,
-// functors and cell in LDS; its waves take electrons part * 4 + wave, + 4 parts, ...; a wave takes
+// ThreeBodyJastrow.h:262-273).  grid (parts, W): a workgroup stages its walker's positions, functors, cell
+// and (IL: when they fit) the ions in LDS; its waves take electrons part * 4 + wave, + 4 parts, ...; a wave takes
 // four of a pair's knots at a time, so a position is read once for the four.
 // Bound: vector arithmetic, (N + M) image distances per knot.  NiO-64, 128 walkers, 396k knots: 0.92 ms
 // in FP32 (it was part of the ratio kernel, where it waited for global loads of positions and
@@ -1530,7 +1530,7 @@ template <typename T>
 __host__ __device__ inline size_t nlpp_jastrow_lds(int N, int M) {
   return sizeof(double) * 3 * (size_t)(N + M) + sizeof(Functor<T>) * (kMaxSpecies + 2) + sizeof(Cell<T>) + 64;
 }
-template <typename T, bool J3>
+template <typename T, bool J3, bool IL>
 __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, const double* spheres, int maxp,
                                                       const double* near, const int* npairs, double* jexp) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -1538,10 +1538,11 @@ __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, co
   const int lane = tid & 63, wid = tid >> 6, nw = nt >> 6;
   double* sR = (double*)smem;
   double* sI = sR + 3 * N;
-  Functor<T>* sFn = (Functor<T>*)(smem + ((sizeof(double) * 3 * (size_t)(N + M) + 15) & ~(size_t)15));
+  Functor<T>* sFn = (Functor<T>*)(smem + ((sizeof(double) * 3 * (size_t)(N + (IL ? M : 0)) + 15) & ~(size_t)15));
   Cell<T>* sCell = (Cell<T>*)(sFn + kMaxSpecies + 2);
   for (int i = tid; i < 3 * N; i += nt) sR[i] = B.R[(size_t)w * 3 * N + i];
-  for (int i = tid; i < 3 * M; i += nt) sI[i] = S.ions[i];
+  if constexpr (IL)
+    for (int i = tid; i < 3 * M; i += nt) sI[i] = S.ions[i];
   for (int i = tid; i < (int)(sizeof(Functor<T>) * (kMaxSpecies + 2) / 4); i += nt) ((int*)sFn)[i] = ((const int*)S.fn)[i];
   for (int i = tid; i < (int)(sizeof(Cell<T>) / 4); i += nt) ((int*)sCell)[i] = ((const int*)S.cell)[i];
   __syncthreads();
@@ -1578,7 +1579,9 @@ __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, co
         for (int ci = lane; ci < M; ci += 64) {
           const Functor<T>& f = sFn[S.species[ci]];
           if (f.ncoef == 0) continue;
-          const double x = sI[ci], y = sI[M + ci], z = sI[2 * M + ci];
+          double x, y, z;
+          if constexpr (IL) x = sI[ci], y = sI[M + ci], z = sI[2 * M + ci];
+          else x = S.ions[ci], y = S.ions[M + ci], z = S.ions[2 * M + ci];
 #pragma unroll
           for (int k = 0; k < kNlppTake; ++k) v[k] += value(f, (T)(x - px[k]), (T)(y - py[k]), (T)(z - pz[k]));
         }

@@ -1,4 +1,5 @@
-"""NonLocalPP at the edges of what the calls accept: spline tables whose padding holds NaN."""
+"""NonLocalPP at the edges of what the calls accept: spline tables whose padding holds NaN, and
+more ions than fit a workgroup's LDS beside the walker."""
 import dataclasses
 
 import numpy as np
@@ -32,3 +33,44 @@ def test_padding_does_not_enter(n, precision):
         ratios.append(r)
     assert np.isfinite(ratios[0]).all()
     np.testing.assert_array_equal(ratios[0], ratios[1])
+
+
+@pytest.mark.parametrize("precision", [qmcx.FP64, qmcx.FP32])
+@pytest.mark.parametrize("nions", [6400, 9000])
+def test_many_ions(nions, precision):
+    """Against the virtual-move ratios at the same points."""
+    rng = np.random.default_rng(nions)
+    n, a, W, rmax = 24, 40.0, 2, 1.3
+    base = orbital_system(n)
+    lattice = np.diag([a, a, a])
+    species = (np.arange(nions) >= nions // 2).astype(np.int32)
+    sysd = dataclasses.replace(base, lattice=lattice, spo_lattice=lattice.copy(), ion_pos=rng.random((nions, 3)) * a,
+                               ion_species=species)
+    dev = qmcx.System(sysd, precisions=(precision,))
+    wb = qmcx.WalkerBatch(dev, W, delay_rank=1, precision=precision)
+    R = rng.random((W, 2 * n, 3)) * a
+    wb.set_positions(R)
+    wb.evaluate_log()
+    spheres = nlpp.NonLocalPP(sysd, rmax=rmax, seed=3).randomize_walkers(W)
+    ratios, pairs = wb.nlpp_evaluate(rmax, spheres, max_pairs=12)
+    assert pairs.sum() > 0
+    eps = 2.0 ** -53 if precision == qmcx.FP64 else 2.0 ** -24
+    for e in range(0, 2 * n, 5):
+        for w in range(W):
+            disp, dist = nlpp.electron_ion_displacements(lattice, sysd.ion_pos, R[w, e])
+            c = np.nonzero(dist < rmax)[0]
+            assert pairs[w, e] == len(c)
+            if len(c) == 0:
+                continue
+            pts = np.broadcast_to(R[:, e, None], (W, 12 * len(c), 3)).copy()
+            pts[w] = np.concatenate([dist[i] * spheres[w] + disp[i] + R[w, e] for i in c])
+            ref = wb.flex_evaluate_ratios(e, pts)[w]
+            inv = wb.inverse(w, e // n)[e % n]
+            psi = dev.spline_vgh(pts[w], precision)[:, 0]
+            # value rows (64 terms an orbital, the points' own rounding times 10 cells of a/10), the sum over
+            # the orbitals, and the exponents' sums over the ions in reach and 2n electrons
+            terms = (np.abs(psi) + 1) * np.abs(inv)
+            jastrow = np.abs(ref / (psi @ inv))
+            tol = (256 + 2 * n) * eps * terms.sum(1) * jastrow + 256 * eps * np.abs(ref)
+            got = ratios[w, e, :len(c)].reshape(-1)
+            assert (np.abs(got - ref) <= tol).all(), (e, w, (np.abs(got - ref) / tol).max())
