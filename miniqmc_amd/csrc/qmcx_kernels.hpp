@@ -17,6 +17,7 @@
 
 #include "qmcx_device.hpp"
 #include "qmcx_j3.hpp"
+#include "qmcx_walk.hpp"
 
 namespace qmcx {
 
@@ -1010,7 +1011,7 @@ __device__ inline int block_key(const SysP<T>& S, const GridBlocks& nb, double x
 template <typename T>
 __global__ __launch_bounds__(256) void k_electron_keys(SysP<T> S, BatchP<T> B, GridBlocks nb, int* key, int* kcnt) {
   const int N = S.N, np = B.W * N;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < np; i += gridDim.x * blockDim.x) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < np; i = walk_next(i, gridDim.x * blockDim.x, np)) {
     const int w = i / N, e = i - w * N;
     const double* R = B.R + (size_t)w * 3 * N;
     const int k = block_key(S, nb, R[e], R[N + e], R[2 * N + e]);
@@ -1476,7 +1477,7 @@ __global__ __launch_bounds__(256) void k_nlpp_keys(SysP<T> S, BatchP<T> B, const
                                                    const double* near, const int* items, const int* cnt,
                                                    GridBlocks nb, int* ukey, int* kcnt) {
   const int nu = cnt[0] * kNlppKnots;
-  for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nu; u += gridDim.x * blockDim.x) {
+  for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nu; u = walk_next(u, gridDim.x * blockDim.x, nu)) {
     int w, e;
     double p[3];
     nlpp_point(S, B, spheres, maxp, near, items, u, w, e, p);
@@ -1513,7 +1514,7 @@ __global__ __launch_bounds__(1024) void k_key_offsets(const int* kcnt, int* kcur
 // points u (cnt[0] * per of them) to their places in the order of their keys
 __global__ __launch_bounds__(256) void k_key_scatter(const int* cnt, int per, const int* ukey, int* kcur, int* units) {
   const int nu = (cnt != nullptr ? cnt[0] : 1) * per;
-  for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nu; u += gridDim.x * blockDim.x)
+  for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nu; u = walk_next(u, gridDim.x * blockDim.x, nu))
     units[atomicAdd(kcur + ukey[u], 1)] = u;
 }
 
@@ -1630,13 +1631,13 @@ __global__ __launch_bounds__(256) void k_nlpp_ratios(SysP<T> S, BatchP<T> B, con
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const int lk = lane & (LK - 1), slot = lane / LK;
   // workgroup b runs on XCD b % 8, and XCD x takes the x-th eighth of the list (gridDim.x % 8 == 0)
-  const int nu = cnt[0] * kNlppKnots, run = KW * take, nruns = (nu + run - 1) / run;
+  const int nu = cnt[0] * kNlppKnots, run = KW * take, nruns = ceil_div(nu, run);
   const int xcd = blockIdx.x & 7, per = (gridDim.x >> 3) * nw;
   const int lo = (int)((long long)nruns * xcd / 8), hi = (int)((long long)nruns * (xcd + 1) / 8);
-  for (int rn = lo + (int)(blockIdx.x >> 3) * nw + wid; rn < hi; rn += per)
+  for (int rn = lo + (int)(blockIdx.x >> 3) * nw + wid; rn < hi; rn = walk_next(rn, per, hi))
     for (int t = 0; t < take; ++t) {
-      const int at = rn * run + t * KW + slot;
-      const int u = units[min(at, nu - 1)];   // past the end: the last knot again, not stored
+      const unsigned at = (unsigned)(rn * run) + (unsigned)(t * KW + slot);   // past INT_MAX at a full list's end
+      const int u = units[min(at, (unsigned)nu - 1u)];   // past the end: the last knot again, not stored
       int w, e;
       double pt[3];
       nlpp_point(S, B, spheres, maxp, near, items, u, w, e, pt);
@@ -1711,7 +1712,7 @@ __global__ __launch_bounds__(256) void k_nlpp_ratios(SysP<T> S, BatchP<T> B, con
         swap_halves(x, y);
         s = x + y;
       }
-      if (lk == 0 && at < nu)
+      if (lk == 0 && at < (unsigned)nu)
         ratios[u] = s * exp(jexp[(size_t)items[u / kNlppKnots] * kNlppKnots + u % kNlppKnots]);
     }
 }
