@@ -387,10 +387,9 @@ struct qmcx_batch_s {
   double* vr_pos = nullptr;       // [W][vr_cap][3] virtual positions of qmcx_flex_evaluate_ratios
   double* vr_out = nullptr;       // [W][vr_cap] their ratios
   int vr_cap = 0;
-  double* nl_out = nullptr;       // [W][N][nl_cap][12] NonLocalPP ratios
-  int* nl_cnt = nullptr;          // [W][N] electron-ion pairs inside rmax
+  double* nl_out = nullptr;       // [W*N*nl_cap][12] NonLocalPP ratios of the listed pairs (before: their knots' keys)
+  int* nl_cnt = nullptr;          // [W][N] electron-ion pairs inside rmax, then [W][N] places of the first in the list
   double* nl_near = nullptr;      // [W][N][nl_cap][4] listed pairs: distance, displacement
-  double* nl_jexp = nullptr;      // [W][N][nl_cap][12] Jastrow exponents of their knots
   int* nl_items = nullptr;        // [W*N*nl_cap] work list of listed pairs, then its length
   int nl_cap = 0;
   double* nl_sph = nullptr;       // [W][12][3] each walker's rotated quadrature knots
@@ -1358,7 +1357,7 @@ static int launch_nlpp_ratios(qmcx_batch_t b, int maxp, int take, const int* uni
   const qmcx_system_s* s = b->sys;
   const int grid = kNlppWorkgroups;   // they walk the ordered knots; their number is only known on the device
   hipLaunchKernelGGL((k_nlpp_ratios<T, LK, Q>), dim3(grid), dim3(256), 0, b->stream, s->params<T>(), b->params<T>(),
-                     b->nl_sph, maxp, b->nl_near, b->nl_items, units, cnt, b->nl_jexp, take, b->nl_out);
+                     b->nl_sph, maxp, b->nl_near, b->nl_items, units, cnt, take, b->nl_out);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -1373,37 +1372,36 @@ static int launch_nlpp(qmcx_batch_t b, double rmax, int maxp) {
     return fail(QMCX_ERR_ARG, unit > 0 ? "NonLocalPP work unit of " + std::to_string(unit) + " knots does not fit a workgroup"
                                        : "spline row does not fit a workgroup");
   const int WN = b->W * s->N;
-  // nl_items: pair list [WN*maxp], its length, per-key counts and cursors, the knots' keys and the
-  // ordered knots [WN*maxp*12 each]
+  // nl_items: pair list [WN*maxp], its length, per-key counts and cursors, the ordered knots [WN*maxp*12]
   const GridBlocks nb = grid_blocks(s);
   const int nkeys = nb.keys();
   const size_t cap = (size_t)WN * maxp;
   int* cnt = b->nl_items + cap;
   int* kcnt = cnt + 1;
   int* kcur = kcnt + nkeys;
-  int* ukey = kcur + nkeys;
-  int* units = ukey + cap * kNlppKnots;
+  int* units = kcur + nkeys;
+  int* ukey = (int*)b->nl_out;   // the knots' keys, until the exponents take their place
   const SysP<T> S = s->params<T>();
   const BatchP<T> B = b->params<T>();
   hipLaunchKernelGGL(k_zero_ints, dim3(16), dim3(256), 0, b->stream, cnt, 1 + nkeys);
   hipLaunchKernelGGL(k_nlpp_pairs<T>, dim3((WN + 255) / 256), dim3(256), 0, b->stream, S, B, rmax, maxp, b->nl_near,
-                     b->nl_items, b->nl_cnt, cnt);
+                     b->nl_items, b->nl_cnt, b->nl_cnt + WN, cnt);
+  const int kgrid = (int)std::min<size_t>((cap * kNlppKnots + 255) / 256, 1024);
+  hipLaunchKernelGGL(k_nlpp_keys<T>, dim3(kgrid), dim3(256), 0, b->stream, S, B, b->nl_sph, maxp, b->nl_near,
+                     b->nl_items, cnt, nb, ukey, kcnt);
+  hipLaunchKernelGGL(k_key_offsets, dim3(1), dim3(1024), 0, b->stream, kcnt, kcur, nkeys);
+  hipLaunchKernelGGL(k_key_scatter, dim3(kgrid), dim3(256), 0, b->stream, cnt, kNlppKnots, ukey, kcur, units);
   // about eight workgroups per CU over the walkers, a wave for at least four electrons
   const int parts = std::max(1, std::min((s->N + 15) / 16, 2048 / b->W));
   const bool il = nlpp_jastrow_lds<T>(s->N, s->nions) <= kMoveLdsMax;
   const size_t jlds = nlpp_jastrow_lds<T>(s->N, il ? s->nions : 0);
   auto jastrow = [&](auto kj3, auto kil) {
     hipLaunchKernelGGL((k_nlpp_jastrow<T, decltype(kj3)::value, decltype(kil)::value>), dim3(parts, b->W), dim3(256),
-                       jlds, b->stream, S, B, b->nl_sph, maxp, b->nl_near, b->nl_cnt, b->nl_jexp);
+                       jlds, b->stream, S, B, b->nl_sph, maxp, b->nl_near, b->nl_cnt, b->nl_cnt + WN, b->nl_out);
   };
   if (b->j3) jastrow(std::true_type{}, std::true_type{});   // at most 256 ions
   else if (il) jastrow(std::false_type{}, std::true_type{});
   else jastrow(std::false_type{}, std::false_type{});
-  const int kgrid = (int)std::min<size_t>((cap * kNlppKnots + 255) / 256, 1024);
-  hipLaunchKernelGGL(k_nlpp_keys<T>, dim3(kgrid), dim3(256), 0, b->stream, S, B, b->nl_sph, maxp, b->nl_near,
-                     b->nl_items, cnt, nb, ukey, kcnt);
-  hipLaunchKernelGGL(k_key_offsets, dim3(1), dim3(1024), 0, b->stream, kcnt, kcur, nkeys);
-  hipLaunchKernelGGL(k_key_scatter, dim3(kgrid), dim3(256), 0, b->stream, cnt, kNlppKnots, ukey, kcur, units);
   HIPCHK(hipGetLastError());
   // the fewest lanes per knot that hold its orbitals in at most three groups each (four past 192
   // groups): a wave then works on several knots of a small system, and no lane idles at NiO-64
@@ -1903,7 +1901,6 @@ int qmcx_batch_destroy(qmcx_batch_t b) {
   if (b->nl_out) hipFree(b->nl_out);
   if (b->nl_cnt) hipFree(b->nl_cnt);
   if (b->nl_near) hipFree(b->nl_near);
-  if (b->nl_jexp) hipFree(b->nl_jexp);
   if (b->nl_items) hipFree(b->nl_items);
   if (b->nl_sph) hipFree(b->nl_sph);
   // the streams are the device's shared ones and stay
@@ -2345,16 +2342,14 @@ int qmcx_nlpp_evaluate(qmcx_batch_t b, double rmax, const double* spheres, int m
     b->nl_cnt = nullptr;
     b->nl_cap = 0;
     if (b->nl_near) hipFree(b->nl_near);
-    if (b->nl_jexp) hipFree(b->nl_jexp);
     if (b->nl_items) hipFree(b->nl_items);
-    b->nl_near = b->nl_jexp = nullptr;
+    b->nl_near = nullptr;
     b->nl_items = nullptr;
     HIPCHK(hipMalloc(&b->nl_out, sizeof(double) * WN * max_pairs * kNlppKnots));
-    HIPCHK(hipMalloc(&b->nl_cnt, sizeof(int) * WN));
+    HIPCHK(hipMalloc(&b->nl_cnt, sizeof(int) * 2 * WN));
     HIPCHK(hipMalloc(&b->nl_near, sizeof(double) * 4 * WN * max_pairs));
-    HIPCHK(hipMalloc(&b->nl_jexp, sizeof(double) * WN * max_pairs * kNlppKnots));
     HIPCHK(hipMalloc(&b->nl_items,
-                     sizeof(int) * (WN * max_pairs * (1 + 2 * kNlppKnots) + 1 + 2 * (size_t)kBlockKeys)));
+                     sizeof(int) * (WN * max_pairs * (1 + kNlppKnots) + 1 + 2 * (size_t)kBlockKeys)));
     b->nl_cap = max_pairs;
   }
   if (!b->nl_sph) HIPCHK(hipMalloc(&b->nl_sph, sizeof(double) * 3 * kNlppKnots * (size_t)b->W));

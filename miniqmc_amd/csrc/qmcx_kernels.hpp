@@ -1393,17 +1393,19 @@ __global__ __launch_bounds__(1024) void k_virtual_ratios(SysP<T> S, BatchP<T> B,
 // k_nlpp_pairs: one lane per (walker, electron) finds the ions within rmax in ion order (minimum
 // image, ion - electron as the BA table's displacement), counts them in npairs[w][e] (the full
 // count, also beyond maxp) and lists the first maxp: near[item][4] = distance, displacement of item =
-// (w*N + e)*maxp + p, items[pos] = item in the order of arrival, cnt[0] = listed pairs.  Knot k of a
-// pair sits at dist * spheres[w][k] + displ + r_e (NonLocalPP.hpp:133; every walker has its own
+// (w*N + e)*maxp + p, items[pos] = item in the order of arrival (an electron's pairs from first[w][e] on),
+// cnt[0] = listed pairs.  Knot k of a pair sits at dist * spheres[w][k] + displ + r_e (NonLocalPP.hpp:133; every walker has its own
 // randomly rotated knots, one rotation per walker and evaluation as the reference's per-mover
 // NonLocalPP::randomize, NonLocalPP.hpp:100-113, miniqmc.cpp:470).
-// k_nlpp_jastrow: the Jastrow exponents of the listed pairs' knots, jexp[item][12], walker by walker
-// (its positions and the functors in LDS, a wave per pair, lanes over the electrons).
 // k_nlpp_keys, k_key_offsets and k_key_scatter order all the knots (unit = pos * 12 + knot) by the
-// block of spline grid cells they fall in, and k_nlpp_ratios walks that order, each XCD over a
+// block of spline grid cells they fall in.
+// k_nlpp_jastrow: the Jastrow exponents of the listed pairs' knots into ratios[pos][12], walker by walker
+// (its positions and the functors in LDS, a wave per pair, lanes over the electrons); the knots' keys,
+// which lay there, are done with.
+// k_nlpp_ratios walks the ordered knots, each XCD over a
 // contiguous eighth of it: knots whose stencils overlap run at the same time on CUs that share an
 // L2, so the orbital table is read from HBM about once instead of once per knot.  ratios[pos][12] =
-// (value row . inverse row) exp(jexp).
+// (value row . inverse row) exp(exponent), in the exponent's place.
 constexpr int kNlppKnots = 12;
 
 __global__ void k_zero_ints(int* p, int n) {
@@ -1412,7 +1414,7 @@ __global__ void k_zero_ints(int* p, int n) {
 
 template <typename T>
 __global__ __launch_bounds__(256) void k_nlpp_pairs(SysP<T> S, BatchP<T> B, double rmax, int maxp, double* near,
-                                                    int* items, int* npairs, int* cnt) {
+                                                    int* items, int* npairs, int* first, int* cnt) {
   const int at = blockIdx.x * blockDim.x + threadIdx.x, N = S.N;
   const bool live = at < B.W * N;
   const int idx = live ? at : 0, M = live ? S.M : 0;
@@ -1452,6 +1454,7 @@ __global__ __launch_bounds__(256) void k_nlpp_pairs(SysP<T> S, BatchP<T> B, doub
   __syncthreads();
   int pos = base + inc - m;
   for (int q = 0; q < wid; ++q) pos += tot[q];
+  if (live) first[idx] = pos;
   for (int p = 0; p < m; ++p) items[pos + p] = idx * maxp + p;
 }
 
@@ -1533,7 +1536,8 @@ __host__ __device__ inline size_t nlpp_jastrow_lds(int N, int M) {
 }
 template <typename T, bool J3, bool IL>
 __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, const double* spheres, int maxp,
-                                                      const double* near, const int* npairs, double* jexp) {
+                                                      const double* near, const int* npairs, const int* first,
+                                                      double* ratios) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int w = blockIdx.y, N = S.N, n = S.n, M = S.M, tid = threadIdx.x, nt = blockDim.x;
   const int lane = tid & 63, wid = tid >> 6, nw = nt >> 6;
@@ -1605,7 +1609,7 @@ __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, co
         // sums in rows 2 and 3; lanes 0 and 16 take their knots' J2 sums from lanes 32 and 48
         const double b0 = __shfl(v[0], (lane & 31) + 32), b1 = __shfl(v[1], (lane & 31) + 32);
         if ((lane & 15) == 0 && lane < 32) {
-          double* out = jexp + item * kNlppKnots + k0 + (lane >> 4) * 2;
+          double* out = ratios + ((size_t)first[idx] + p) * kNlppKnots + k0 + (lane >> 4) * 2;
           out[0] = (j1o - v[0]) + (j2o - b0);
           out[1] = (j1o - v[1]) + (j2o - b1);
         }
@@ -1624,7 +1628,7 @@ __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, co
 template <typename T, int LK, int Q>
 __global__ __launch_bounds__(256) void k_nlpp_ratios(SysP<T> S, BatchP<T> B, const double* spheres, int maxp,
                                                      const double* near, const int* items, const int* units,
-                                                     const int* cnt, const double* jexp, int take, double* ratios) {
+                                                     const int* cnt, int take, double* ratios) {
   using VT = typename V16<T>::type;
   constexpr int VW = V16<T>::n, KW = 64 / LK;
   const int N = S.N, n = S.n, nq = S.npad / VW;
@@ -1713,7 +1717,7 @@ __global__ __launch_bounds__(256) void k_nlpp_ratios(SysP<T> S, BatchP<T> B, con
         s = x + y;
       }
       if (lk == 0 && at < (unsigned)nu)
-        ratios[u] = s * exp(jexp[(size_t)items[u / kNlppKnots] * kNlppKnots + u % kNlppKnots]);
+        ratios[u] = s * exp(ratios[u]);
     }
 }
 

@@ -1,6 +1,6 @@
-// The library's use of HIP resources: what it does when an allocation or a launch fails.  The
-// program defines some HIP entry points itself; the library's calls reach these first, which fail the one that a
-// check asks for and pass the others on to the runtime.
+// The library's use of HIP resources: what it does when an allocation or a launch fails, and how much it
+// allocates.  The program defines some HIP entry points itself; the library's calls reach these first, which
+// count them, fail the one that a check asks for, and pass the others on to the runtime.
 #include <dlfcn.h>
 
 #include <cmath>
@@ -15,6 +15,7 @@
 typedef void* handle;   // hipStream_t, hipEvent_t
 static int fail_malloc = 0, fail_launch = 0;   // the n-th call from now fails (0: none)
 static std::map<handle, handle> recorded;      // event -> stream of its latest record that no other stream waited for
+static size_t device_bytes = 0;   // allocated since it was last set to zero
 static const int kOutOfMemory = 2;
 
 template <typename F>
@@ -27,6 +28,7 @@ extern "C" {
 int hipMalloc(void** p, size_t bytes) {
   static auto f = next<int (*)(void**, size_t)>("hipMalloc");
   if (fail_malloc > 0 && --fail_malloc == 0) return kOutOfMemory;
+  device_bytes += bytes;
   return f(p, bytes);
 }
 int hipGetLastError() {
@@ -130,8 +132,28 @@ static void evaluate_log() {
   }
 }
 
+// device memory of a NonLocalPP evaluation: per slot of a walker's electrons' lists, the slot's index, its
+// pair's distance and displacement, and for each of its twelve knots a ratio and a place in the order
+static void nlpp_device_memory() {
+  Model m(48, 10);
+  const int W = 64, slots = 64;
+  const std::vector<double> R = m.positions(W), spheres((size_t)W * 12 * 3, 0.5);
+  qmcx_batch_t b;
+  must(qmcx_batch_create(&b, m.sys, W, 1, QMCX_FP32), "qmcx_batch_create");
+  must(qmcx_batch_set_positions(b, R.data()), "qmcx_batch_set_positions");
+  must(qmcx_evaluate_log(b, nullptr), "qmcx_evaluate_log");
+  std::vector<int> pairs((size_t)W * 2 * m.n);
+  device_bytes = 0;
+  must(qmcx_nlpp_evaluate(b, 2.0, spheres.data(), slots, nullptr, pairs.data()), "qmcx_nlpp_evaluate");
+  const double per_slot = (double)device_bytes / ((double)W * 2 * m.n * slots);
+  std::printf("%.1f bytes per slot\n", per_slot);
+  check(per_slot <= 4 + 32 + 12 * (8 + 4) + 4, "device memory of a NonLocalPP evaluation");
+  qmcx_batch_destroy(b);
+}
+
 int main() {
   evaluate_log();
+  nlpp_device_memory();
   std::printf(failures == 0 ? "All checks passed\n" : "%d checks failed\n", failures);
   return failures == 0 ? 0 : 1;
 }

@@ -1,4 +1,5 @@
-"""Runs tests/cpp/check_resources.cpp: failing allocations and launches.
+"""Runs tests/cpp/check_resources.cpp: failing allocations and launches, and the memory
+that calls take.
 The binary is built by __graft_entry__.build()."""
 import os
 import subprocess
