@@ -54,11 +54,12 @@ struct PinnedPool {
   std::mutex mu;
   std::vector<std::pair<size_t, void*>> free;   // bytes, block
   size_t bytes = 0;
-  void* take(size_t want, size_t* cap) {   // the smallest block that holds `want`, or null
+  void* take(size_t want, size_t* cap) {   // the smallest block that holds `want` and is not far larger, or null
+    const size_t most = 4 * want + (size_t(64) << 10);   // a small request does not keep a large block for itself
     std::lock_guard<std::mutex> lock(mu);
     int best = -1;
     for (int i = 0; i < (int)free.size(); ++i)
-      if (free[i].first >= want && (best < 0 || free[i].first < free[best].first)) best = i;
+      if (free[i].first >= want && free[i].first <= most && (best < 0 || free[i].first < free[best].first)) best = i;
     if (best < 0) return nullptr;
     void* p = free[best].second;
     *cap = free[best].first;
@@ -627,6 +628,9 @@ constexpr int kPropWorkgroups = 1024;
 constexpr size_t kVirtualInPlace = 2048;
 // virtual positions per walker in one qmcx_flex_evaluate_ratios call (grid x dimension)
 constexpr int kMaxVirtualPoints = 1 << 16;
+// pairs whose ratios a NonLocalPP evaluation has in pinned memory at a time, in each of two buffers (6.5 MB):
+// the host scatters one while the next is copied
+constexpr size_t kNlppCopyPairs = 1 << 16;
 // electron-ion pairs per electron held by qmcx_nlpp_evaluate
 constexpr int kMaxNlppPairs = 64;
 // workgroups of the NonLocalPP ratio launch (they walk the ordered knots), a multiple of the XCDs
@@ -2368,15 +2372,30 @@ int qmcx_nlpp_evaluate(qmcx_batch_t b, double rmax, const double* spheres, int m
   bool over = false;
   for (size_t i = 0; i < WN; ++i) over = over || cnt[i] > max_pairs;
   if (ratios && listed > 0) {
-    // the listed pairs' ratios to their places; the other slots stay as they were
-    if (int rc2 = b->nl_io.need((sizeof(double) * kNlppKnots + sizeof(int)) * listed)) return rc2;
-    double* rat = b->nl_io.as<double>();
-    int* items = (int*)(rat + listed * kNlppKnots);
-    HIPCHK(hipMemcpyAsync(items, b->nl_items, sizeof(int) * listed, hipMemcpyDeviceToHost, b->stream));
-    HIPCHK(hipMemcpyAsync(rat, b->nl_out, sizeof(double) * listed * kNlppKnots, hipMemcpyDeviceToHost, b->stream));
-    HIPCHK(hipStreamSynchronize(b->stream));
-    for (size_t i = 0; i < listed; ++i)
-      std::memcpy(ratios + (size_t)items[i] * kNlppKnots, rat + i * kNlppKnots, sizeof(double) * kNlppKnots);
+    // the listed pairs' ratios to their places; the other slots stay as they were.  The buffers hold a power
+    // of two of pairs, so that evaluations whose lists grow little by little seldom need larger ones
+    size_t chunk = 1024;
+    while (chunk < std::min(listed, kNlppCopyPairs)) chunk *= 2;
+    const size_t bytes = (sizeof(double) * kNlppKnots + sizeof(int)) * chunk;
+    if (int rc2 = b->nl_io.need(bytes * (listed > chunk ? 2 : 1))) return rc2;
+    auto rat = [&](size_t o) { return (double*)(b->nl_io.as<char>() + (o / chunk % 2) * bytes); };
+    auto fetch = [&](size_t o) -> int {
+      const size_t m = std::min(chunk, listed - o);
+      HIPCHK(hipMemcpyAsync(rat(o) + chunk * kNlppKnots, b->nl_items + o, sizeof(int) * m, hipMemcpyDeviceToHost, b->stream));
+      HIPCHK(hipMemcpyAsync(rat(o), b->nl_out + o * kNlppKnots, sizeof(double) * m * kNlppKnots, hipMemcpyDeviceToHost,
+                            b->stream));
+      return 0;
+    };
+    if (int rc2 = fetch(0)) return rc2;
+    for (size_t o = 0; o < listed; o += chunk) {
+      HIPCHK(hipStreamSynchronize(b->stream));
+      if (o + chunk < listed)
+        if (int rc2 = fetch(o + chunk)) return rc2;
+      const double* r = rat(o);
+      const int* items = (const int*)(r + chunk * kNlppKnots);
+      for (size_t i = 0; i < std::min(chunk, listed - o); ++i)
+        std::memcpy(ratios + (size_t)items[i] * kNlppKnots, r + i * kNlppKnots, sizeof(double) * kNlppKnots);
+    }
   }
   if (over) return fail(QMCX_ERR_ARG, "more ions within rmax of an electron than max_pairs");
   return 0;

@@ -16,6 +16,8 @@ typedef void* handle;   // hipStream_t, hipEvent_t
 static int fail_malloc = 0, fail_launch = 0;   // the n-th call from now fails (0: none)
 static std::map<handle, handle> recorded;      // event -> stream of its latest record that no other stream waited for
 static size_t device_bytes = 0;   // allocated since it was last set to zero
+static int pinned_calls = 0;      // pinned allocations since it was last set to zero
+static size_t pinned_largest = 0; // the largest of them
 static const int kOutOfMemory = 2;
 
 template <typename F>
@@ -30,6 +32,12 @@ int hipMalloc(void** p, size_t bytes) {
   if (fail_malloc > 0 && --fail_malloc == 0) return kOutOfMemory;
   device_bytes += bytes;
   return f(p, bytes);
+}
+int hipHostMalloc(void** p, size_t bytes, unsigned flags) {
+  static auto f = next<int (*)(void**, size_t, unsigned)>("hipHostMalloc");
+  ++pinned_calls;
+  pinned_largest = bytes > pinned_largest ? bytes : pinned_largest;
+  return f(p, bytes, flags);
 }
 int hipGetLastError() {
   static auto f = next<int (*)()>("hipGetLastError");
@@ -151,9 +159,63 @@ static void nlpp_device_memory() {
   qmcx_batch_destroy(b);
 }
 
+// pinned host memory of NonLocalPP evaluations and virtual ratios
+static void nlpp_pinned_memory() {
+  const int slots = 64, N = 96;
+  Model m(N / 2, 60);
+  const int W = 64, part = 8;
+  const std::vector<double> R = m.positions(W);
+  std::vector<double> spheres((size_t)W * 12 * 3);
+  for (double& x : spheres) x = m.uniform(-0.5, 0.5);
+  auto batch = [&](int first, int walkers) {
+    qmcx_batch_t b;
+    must(qmcx_batch_create(&b, m.sys, walkers, 1, QMCX_FP32), "qmcx_batch_create");
+    must(qmcx_batch_set_positions(b, R.data() + (size_t)first * N * 3), "qmcx_batch_set_positions");
+    must(qmcx_evaluate_log(b, nullptr), "qmcx_evaluate_log");
+    return b;
+  };
+  std::vector<double> ratios((size_t)W * N * slots * 12), parts(ratios);
+  std::vector<int> pairs((size_t)W * N);
+  auto evaluate = [&](qmcx_batch_t b, double rmax, double* out) {
+    must(qmcx_nlpp_evaluate(b, rmax, spheres.data(), slots, out, pairs.data()), "qmcx_nlpp_evaluate");
+  };
+  // lists that grow from call to call
+  qmcx_batch_t b = batch(0, W);
+  pinned_calls = 0;
+  for (int i = 0; i < 20; ++i) evaluate(b, 1.5 + 0.05 * i, ratios.data());
+  std::printf("%d pinned allocations in 20 evaluations\n", pinned_calls);
+  check(pinned_calls <= 6, "lists that grow seldom need larger pinned buffers");
+  qmcx_batch_destroy(b);
+  // a small request leaves a large block to the next batch that needs it
+  b = batch(0, W);
+  const double point[3] = {1.0, 2.0, 3.0};
+  double ratio = 0;
+  qmcx_batch_t one = batch(0, 1);
+  must(qmcx_flex_evaluate_ratios(one, 0, 1, point, &ratio), "qmcx_flex_evaluate_ratios");
+  pinned_calls = 0;
+  evaluate(b, 2.4, ratios.data());
+  check(pinned_calls == 0, "a batch takes the blocks that one like it gave back");
+  qmcx_batch_destroy(one);
+  // every ion is in reach: the list is longer than the buffers, which stay as they are
+  pinned_largest = 0;
+  evaluate(b, 9.0, ratios.data());
+  std::printf("pinned allocation of %.1f MB for %.1f MB of ratios\n", 1e-6 * pinned_largest, 96e-6 * W * N * 60);
+  check(pinned_largest <= size_t(14) << 20, "the pinned buffers do not grow with the list");
+  qmcx_batch_destroy(b);
+  const std::vector<double> all = spheres;
+  for (int w = 0; w < W; w += part) {
+    b = batch(w, part);
+    std::copy(all.begin() + w * 36, all.begin() + (w + part) * 36, spheres.begin());
+    evaluate(b, 9.0, parts.data() + (size_t)w * N * slots * 12);
+    qmcx_batch_destroy(b);
+  }
+  check(ratios == parts, "the ratios of a long list are those of its parts");
+}
+
 int main() {
   evaluate_log();
   nlpp_device_memory();
+  nlpp_pinned_memory();
   std::printf(failures == 0 ? "All checks passed\n" : "%d checks failed\n", failures);
   return failures == 0 ? 0 : 1;
 }
