@@ -9,6 +9,7 @@
 #include <cstring>
 #include <limits>
 #include <mutex>
+#include <new>
 #include <string>
 #include <utility>
 #include <vector>
@@ -67,10 +68,14 @@ struct PinnedPool {
     free.erase(free.begin() + best);
     return p;
   }
-  bool give(void* p, size_t cap) {
+  bool give(void* p, size_t cap) noexcept {   // false: the block stays the caller's
     std::lock_guard<std::mutex> lock(mu);
     if (bytes + cap > kPinnedPool) return false;
-    free.emplace_back(cap, p);
+    try {
+      free.emplace_back(cap, p);
+    } catch (const std::bad_alloc&) {
+      return false;
+    }
     bytes += cap;
     return true;
   }

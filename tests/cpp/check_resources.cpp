@@ -1,12 +1,14 @@
-// The library's use of HIP resources: what it does when an allocation or a launch fails, and how much it
-// allocates.  The program defines some HIP entry points itself; the library's calls reach these first, which
+// The library's use of HIP resources and host memory: what it does when an allocation or a launch fails, and how
+// much it allocates.  The program defines some HIP entry points itself; the library's calls reach these first, which
 // count them, fail the one that a check asks for, and pass the others on to the runtime.
 #include <dlfcn.h>
 
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <map>
+#include <new>
 #include <random>
 #include <vector>
 
@@ -19,6 +21,21 @@ static size_t device_bytes = 0;   // allocated since it was last set to zero
 static int pinned_calls = 0;      // pinned allocations since it was last set to zero
 static size_t pinned_largest = 0; // the largest of them
 static const int kOutOfMemory = 2;
+
+static bool no_memory = false;    // operator new fails where the library itself calls it
+static int refused = 0;
+__attribute__((noinline)) void* operator new(std::size_t n) {
+  Dl_info at;
+  if (no_memory && dladdr(__builtin_return_address(0), &at) && std::strstr(at.dli_fname, "libqmcx")) {
+    ++refused;
+    throw std::bad_alloc();
+  }
+  void* p = std::malloc(n);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+__attribute__((noinline)) void operator delete(void* p) noexcept { std::free(p); }
+__attribute__((noinline)) void operator delete(void* p, std::size_t) noexcept { std::free(p); }
 
 template <typename F>
 static F next(const char* name) {
@@ -212,10 +229,31 @@ static void nlpp_pinned_memory() {
   check(ratios == parts, "the ratios of a long list are those of its parts");
 }
 
+// a batch given back when the host has no memory for the list of free pinned blocks
+static void destroy_without_memory() {
+  Model m(48, 10);
+  const double point[3] = {1.0, 2.0, 3.0};
+  std::vector<qmcx_batch_t> batches(40);
+  const std::vector<double> R = m.positions(1);
+  for (qmcx_batch_t& b : batches) {
+    must(qmcx_batch_create(&b, m.sys, 1, 1, QMCX_FP64), "qmcx_batch_create");
+    must(qmcx_batch_set_positions(b, R.data()), "qmcx_batch_set_positions");
+    must(qmcx_evaluate_log(b, nullptr), "qmcx_evaluate_log");
+    double ratio;
+    must(qmcx_flex_evaluate_ratios(b, 0, 1, point, &ratio), "qmcx_flex_evaluate_ratios");
+  }
+  int rc = 0;
+  no_memory = true;   // the list of the blocks has to grow for some of them
+  for (qmcx_batch_t b : batches) rc |= qmcx_batch_destroy(b);
+  no_memory = false;
+  check(rc == 0 && refused > 0, "batches destroyed without host memory");
+}
+
 int main() {
   evaluate_log();
   nlpp_device_memory();
   nlpp_pinned_memory();
+  destroy_without_memory();
   std::printf(failures == 0 ? "All checks passed\n" : "%d checks failed\n", failures);
   return failures == 0 ? 0 : 1;
 }
