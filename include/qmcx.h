@@ -203,7 +203,7 @@ int qmcx_flex_evaluate_ratios(qmcx_batch_t b, int iel, int nvp, const double* vp
 int qmcx_nlpp_evaluate(qmcx_batch_t b, double rmax, const double* spheres, int max_pairs, double* ratios,
                        int* npairs);
 /* Tuning knob of qmcx_nlpp_evaluate: runs of knots a wave takes from the ordered knot list at a time (1, 2, 4 or 6;
- * 0 = 1).  QMCX_ERR_ARG at evaluation when that many value rows do not fit a workgroup of 768 lanes. */
+ * 0 = 1).  QMCX_ERR_ARG at evaluation when that many rows of npad orbitals are more than 768 groups of 16 bytes. */
 int qmcx_batch_set_nlpp_unit(qmcx_batch_t b, int knots_per_unit);
 
 /* Per-move record of the most recent sweep, [nw][N][9]:

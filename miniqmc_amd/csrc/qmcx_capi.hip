@@ -615,9 +615,11 @@ int launch_moves(qmcx_batch_t b, int nt, size_t lds, const MoveArgs& a, bool st)
 //   * None when the move, refresh and proposals workgroups together are no more than the CUs: no
 //     move workgroup can then be kept out.  One walker of the cubic cell (n = 48) waited out the
 //     second determinant's 500 us in every sweep, whose two move launches take 340 us.
-//   * Else up to a share of the move launch, which lasts about 9 us per electron: 0.3 n and 1.3 n us
-//     (at n = 384 the constants 100 and 500 us, which measured best there; 37 walkers at n = 96
-//     lost 60 us per sweep to the full 500).
+//   * Else up to a share of the move launch, which lasts about 8 us per electron: 0.3 n and 1.3 n us
+//     (at n = 384 the constants 100 and 500 us, which measured best there).  Three FP32 sweeps with no
+//     holds / these / the constants: n = 48, 256 walkers 2.44 / 2.34 / 2.71 ms; n = 96, 128 walkers 3.49 /
+//     3.31 / 3.63, 256 walkers 5.1 / 4.76 / 4.66; n = 192, 128 walkers 9.5 / 8.76 / 8.77, 256 walkers 13.7 /
+//     11.7 / 11.5; n = 384, 128 walkers 26.2 / 22.3 / 22.4, 256 walkers 45.0 / 43.7 / 43.7.
 constexpr int kHoldRefreshUs = 30, kHoldProp0Us = 100, kHoldProp1Us = 500;
 struct Holds {
   int refresh, prop[2];
@@ -629,7 +631,10 @@ Holds side_holds(int W, int n, int prop_workgroups, int cus) {
 
 // SPO rows at the proposals of electrons det*n + [e0, e0 + ne) of every walker
 constexpr int kPropWorkgroups = 1024;
-// points of a qmcx_flex_evaluate_ratios call up to which the kernel works on pinned host memory in place
+// points of a qmcx_flex_evaluate_ratios call up to which the kernel works on pinned host memory in place:
+// for one walker of NiO-8 24 us against 37 with device buffers and copies at 16 points, 34 against 68 at
+// this many, 49 against 99 at 4096, and the same from 16384 on (NiO-32, 64 walkers: 27 against 39, 42 against 54, 62
+// against 67).  The bound keeps a batch's pinned block at 64 KB.
 constexpr size_t kVirtualInPlace = 2048;
 // virtual positions per walker in one qmcx_flex_evaluate_ratios call (grid x dimension)
 constexpr int kMaxVirtualPoints = 1 << 16;
@@ -640,7 +645,9 @@ constexpr size_t kNlppCopyPairs = 1 << 16;
 constexpr int kMaxNlppPairs = 64;
 // workgroups of the NonLocalPP ratio launch (they walk the ordered knots), a multiple of the XCDs
 constexpr int kNlppWorkgroups = 2048;
-constexpr int kNlppThreads = 768;
+// 16-byte orbital groups (of a row, times the knots of a set unit) up to which an evaluation is accepted: the
+// most that the ratio kernel's widest layout holds (64 lanes x 12)
+constexpr int kNlppGroups = 768;
 
 // proposals workgroups per walker for ne electrons
 int prop_grid(int W, int ne) { return std::max(1, std::min(ne, kPropWorkgroups / W)); }
@@ -1375,9 +1382,8 @@ template <typename T>
 static int launch_nlpp(qmcx_batch_t b, double rmax, int maxp) {
   const qmcx_system_s* s = b->sys;
   const int nq = s->npad / (16 / (int)sizeof(T));
-  // `unit` (qmcx_batch_set_nlpp_unit) is limited to the value rows of a workgroup of kNlppThreads lanes
   const int unit = b->nl_unit;
-  if ((unit > 0 ? unit : 1) * nq > kNlppThreads)
+  if ((unit > 0 ? unit : 1) * nq > kNlppGroups)
     return fail(QMCX_ERR_ARG, unit > 0 ? "NonLocalPP work unit of " + std::to_string(unit) + " knots does not fit a workgroup"
                                        : "spline row does not fit a workgroup");
   const int WN = b->W * s->N;

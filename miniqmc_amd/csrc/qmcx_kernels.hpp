@@ -675,7 +675,7 @@ __global__ __launch_bounds__(64 * kFlushWaves) void k_flush_mfma(SysP<float> S, 
 //
 // Bound: latency of the pivot steps (about 1 us each: two barriers, the pivot search, one division)
 // and of a wave's tile; with as many matrices as CUs at n = 384 the passes over X, whose working
-// set (302 MB) exceeds the last-level cache.  n = 384: one matrix 1.17 ms, 128 at once 1.39, 256 at
+// set (302 MB) exceeds the last-level cache.  n = 384: one matrix 1.19 ms, 128 at once 1.40, 256 at
 // once 2.1 (the form that exchanged rows and streamed X in 64-column chunks through LDS between
 // barriers: 2.32, 2.51 and 2.97); n = 192, 256 at once: 0.41 (0.66) ms.  Sub-panels of 16 columns
 // with a rank-16 update between them take 1.10, 1.30 and 2.0 ms but round differently: an element of
@@ -1623,7 +1623,7 @@ __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, co
 // A wave takes `take` runs of 64 / LK consecutive knots at a time.  The stencil rows come from L2 and
 // the CU's cache (cached loads: neighbouring knots want them).
 // Bound: L2 and L1 bandwidth of the stencils, 64 rows per knot.  NiO-64, 128 walkers, 396k knots:
-// 1.64 ms in FP32 (28 TB/s of stencil bytes); the whole evaluation's kernels 2.7 ms against 7.4 for a
+// 1.59 ms in FP32 (24 TB/s of stencil bytes, 2.3 GB from HBM); the whole evaluation's kernels 2.7 ms against 7.4 for a
 // workgroup per knot in the order of ions, whose stencils came from HBM (38 GB at 5.2 TB/s).
 template <typename T, int LK, int Q>
 __global__ __launch_bounds__(256) void k_nlpp_ratios(SysP<T> S, BatchP<T> B, const double* spheres, int maxp,
