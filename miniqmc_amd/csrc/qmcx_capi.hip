@@ -631,11 +631,12 @@ Holds side_holds(int W, int n, int prop_workgroups, int cus) {
 
 // SPO rows at the proposals of electrons det*n + [e0, e0 + ne) of every walker
 constexpr int kPropWorkgroups = 1024;
-// points of a qmcx_flex_evaluate_ratios call up to which the kernel works on pinned host memory in place:
-// for one walker of NiO-8 24 us against 37 with device buffers and copies at 16 points, 34 against 68 at
-// this many, 49 against 99 at 4096, and the same from 16384 on (NiO-32, 64 walkers: 27 against 39, 42 against 54, 62
-// against 67).  The bound keeps a batch's pinned block at 64 KB.
-constexpr size_t kVirtualInPlace = 2048;
+// points of a qmcx_flex_evaluate_ratios call up to which the kernel works on pinned host memory in place,
+// against device buffers and pageable copies.  NiO-8 FP32, 64 walkers: 33 us against 44 at 2112 points, 51
+// against 53 at 5120, 61 against 64 at 7680, 97 against 97 at 16384, 184 against 150 at 32768; one walker of NiO-8
+// in FP64: 24 against 37 at 16 points.  (A process's first couple of hundred pageable copies take 20 to 120 us
+// longer.)  A batch's pinned block is 512 KB at most.
+constexpr size_t kVirtualInPlace = 16384;
 // virtual positions per walker in one qmcx_flex_evaluate_ratios call (grid x dimension)
 constexpr int kMaxVirtualPoints = 1 << 16;
 // pairs whose ratios a NonLocalPP evaluation has in pinned memory at a time, in each of two buffers (6.5 MB):
@@ -2307,9 +2308,11 @@ int qmcx_flex_evaluate_ratios(qmcx_batch_t b, int iel, int nvp, const double* vp
   };
   if (np <= kVirtualInPlace) {
     // a small call: the kernel reads the points and writes the ratios in pinned host memory
-    if (int rc = b->vr_io.need(sizeof(double) * 4 * kVirtualInPlace)) return rc;
+    size_t most = 2048;   // 64 KB, more when a call needs it
+    while (most < np) most *= 2;
+    if (int rc = b->vr_io.need(sizeof(double) * 4 * most)) return rc;
     double* pos = b->vr_io.as<double>();
-    double* out = pos + 3 * kVirtualInPlace;
+    double* out = pos + 3 * most;
     std::memcpy(pos, vpos, sizeof(double) * 3 * np);
     if (int rc = launch(pos, out)) return rc;
     HIPCHK(hipStreamSynchronize(b->stream));

@@ -1,7 +1,7 @@
 """Shapes that the prepared systems do not have, on the paths that are chosen by size: SPO rows ordered by
-place (orbital counts that are not whole 16-byte vectors, a skewed cell, grids coarser than four cells a block,
-the largest orbital count of the path) and the flush inside the move kernel (tile counts below those its
-forms hold)."""
+place (orbital counts that are not whole 16-byte vectors, a skewed cell, the largest orbital count of the path),
+the flush inside the move kernel (tile counts below those its forms hold), and virtual ratios at the sizes where
+the pinned block grows and where the call leaves it."""
 import numpy as np
 import pytest
 
@@ -60,3 +60,20 @@ def test_flush_tiles(n, delay):
     for a, b in zip(*out):
         assert np.isfinite(a).all()
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("walkers,points", [(1, 2047), (1, 2049), (1, 16384), (1, 16385), (7, 300), (7, 2340),
+                                            (7, 2341), (64, 256), (64, 257)])
+def test_virtual_ratio_sizes(walkers, points):
+    """A call's ratios are those of its points in small calls, whatever the sizes before it."""
+    sysd = orbital_system(33)
+    dev = qmcx.System(sysd, precisions=(qmcx.FP64,))
+    rng = np.random.default_rng(points)
+    wb = qmcx.WalkerBatch(dev, walkers, delay_rank=1, precision=qmcx.FP64)
+    wb.set_positions(rng.random((walkers, 66, 3)) @ sysd.lattice)
+    wb.evaluate_log()
+    pts = rng.random((walkers, points, 3)) @ sysd.lattice
+    whole = wb.flex_evaluate_ratios(5, pts)
+    part = max(1, 2000 // walkers)
+    for o in range(0, points, part):
+        np.testing.assert_array_equal(whole[:, o:o + part], wb.flex_evaluate_ratios(5, pts[:, o:o + part]))
