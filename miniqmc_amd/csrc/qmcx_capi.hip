@@ -1379,6 +1379,31 @@ static int launch_nlpp_ratios(qmcx_batch_t b, int maxp, int take, const int* uni
   return 0;
 }
 
+// Whether the knots of an evaluation are ordered by grid cell, by the bytes of stencils that it is likely to read
+// (ions at their mean density, every electron's list at most maxp long) and those of the spline table.  Ordering
+// takes three launches, about 17 us, and 1 ns per knot.
+//   * Tables past 24 MB: from 256 MB of stencils on.  One walker of NiO-64 FP32 (462 MB; 0.3 GB of stencils) takes
+//     138 us ordered and 142 in the order of the pairs, eight 280 and 458; NiO-32 FP32 (110 MB) 97 and 94 us
+//     with two walkers (0.16 GB), 110 and 118 with four; NiO-16 FP64 (33 MB) 119 and 117 with 16 (0.6 GB), 188 and 201
+//     with 32.
+//   * Smaller ones, which stay in the last-level cache, from 8 GB on: NiO-16 FP32 (16 MB) 562 and 494 us at 4.9 GB,
+//     805 and 838 at 7.9 GB, 5505 and 6640 at 63 GB.
+//   * Never up to 8 MB, which L2 holds most of: NiO-8 FP64 (7.6 MB) 3607 and 2262 us at 31 GB.
+template <typename T>
+static bool nlpp_ordered(const qmcx_batch_t b, double rmax, int maxp) {
+  const qmcx_system_s* s = b->sys;
+  double inv[9];
+  inv3(s->lattice, inv);
+  const double volume = std::fabs(1.0 / (inv[0] * (inv[4] * inv[8] - inv[5] * inv[7]) -
+                                         inv[1] * (inv[3] * inv[8] - inv[5] * inv[6]) +
+                                         inv[2] * (inv[3] * inv[7] - inv[4] * inv[6])));
+  const double pairs = std::min((double)maxp, s->nions * 4.18879 * rmax * rmax * rmax / volume);
+  const double row = (double)s->npad * sizeof(T);
+  const double stencils = pairs * b->W * s->N * kNlppKnots * 64 * row;
+  const double table = (s->ng[0] + 3.0) * (s->ng[1] + 3.0) * (s->ng[2] + 3.0) * row;
+  return table > 8e6 && stencils >= (table > 24e6 ? 256e6 : 8e9);
+}
+
 template <typename T>
 static int launch_nlpp(qmcx_batch_t b, double rmax, int maxp) {
   const qmcx_system_s* s = b->sys;
@@ -1399,16 +1424,21 @@ static int launch_nlpp(qmcx_batch_t b, double rmax, int maxp) {
   int* ukey = (int*)b->nl_out;   // the knots' keys, until the exponents take their place
   const SysP<T> S = s->params<T>();
   const BatchP<T> B = b->params<T>();
-  hipLaunchKernelGGL(k_zero_ints, dim3(16), dim3(256), 0, b->stream, cnt, 1 + nkeys);
+  const bool ordered = nlpp_ordered<T>(b, rmax, maxp);
+  hipLaunchKernelGGL(k_zero_ints, dim3(ordered ? 16 : 1), dim3(256), 0, b->stream, cnt, ordered ? 1 + nkeys : 1);
   hipLaunchKernelGGL(k_nlpp_pairs<T>, dim3((WN + 255) / 256), dim3(256), 0, b->stream, S, B, rmax, maxp, b->nl_near,
                      b->nl_items, b->nl_cnt, b->nl_cnt + WN, cnt);
   const int kgrid = (int)std::min<size_t>((cap * kNlppKnots + 255) / 256, 1024);
-  hipLaunchKernelGGL(k_nlpp_keys<T>, dim3(kgrid), dim3(256), 0, b->stream, S, B, b->nl_sph, maxp, b->nl_near,
-                     b->nl_items, cnt, nb, ukey, kcnt);
-  hipLaunchKernelGGL(k_key_offsets, dim3(1), dim3(1024), 0, b->stream, kcnt, kcur, nkeys);
-  hipLaunchKernelGGL(k_key_scatter, dim3(kgrid), dim3(256), 0, b->stream, cnt, kNlppKnots, ukey, kcur, units);
-  // about eight workgroups per CU over the walkers, a wave for at least four electrons
-  const int parts = std::max(1, std::min((s->N + 15) / 16, 2048 / b->W));
+  if (ordered) {
+    hipLaunchKernelGGL(k_nlpp_keys<T>, dim3(kgrid), dim3(256), 0, b->stream, S, B, b->nl_sph, maxp, b->nl_near,
+                       b->nl_items, cnt, nb, ukey, kcnt);
+    hipLaunchKernelGGL(k_key_offsets, dim3(1), dim3(1024), 0, b->stream, kcnt, kcur, nkeys);
+    hipLaunchKernelGGL(k_key_scatter, dim3(kgrid), dim3(256), 0, b->stream, cnt, kNlppKnots, ukey, kcur, units);
+  } else {
+    units = nullptr;
+  }
+  // about eight workgroups per CU over the walkers
+  const int parts = std::max(1, std::min(s->N, 2048 / b->W));
   const bool il = nlpp_jastrow_lds<T>(s->N, s->nions) <= kMoveLdsMax;
   const size_t jlds = nlpp_jastrow_lds<T>(s->N, il ? s->nions : 0);
   auto jastrow = [&](auto kj3, auto kil) {

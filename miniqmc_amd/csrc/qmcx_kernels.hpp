@@ -1398,7 +1398,7 @@ __global__ __launch_bounds__(1024) void k_virtual_ratios(SysP<T> S, BatchP<T> B,
 // randomly rotated knots, one rotation per walker and evaluation as the reference's per-mover
 // NonLocalPP::randomize, NonLocalPP.hpp:100-113, miniqmc.cpp:470).
 // k_nlpp_keys, k_key_offsets and k_key_scatter order all the knots (unit = pos * 12 + knot) by the
-// block of spline grid cells they fall in.
+// block of spline grid cells they fall in (left out when there are few, or the table is small).
 // k_nlpp_jastrow: the Jastrow exponents of the listed pairs' knots into ratios[pos][12], walker by walker
 // (its positions and the functors in LDS, a wave per pair, lanes over the electrons); the knots' keys,
 // which lay there, are done with.
@@ -1524,15 +1524,17 @@ __global__ __launch_bounds__(256) void k_key_scatter(const int* cnt, int per, co
 // J1, J2 (and J3) exponents of every listed pair's knots: sums at the electron's position (kept by the
 // moves) less those at the knot (OneBodyJastrow.h:136-140, TwoBodyJastrow.h:103-107,
 // ThreeBodyJastrow.h:262-273).  grid (parts, W): a workgroup stages its walker's positions, functors, cell
-// and (IL: when they fit) the ions in LDS; its waves take electrons part * 4 + wave, + 4 parts, ...; a wave takes
-// four of a pair's knots at a time, so a position is read once for the four.
-// Bound: vector arithmetic, (N + M) image distances per knot.  NiO-64, 128 walkers, 396k knots: 0.92 ms
-// in FP32 (it was part of the ratio kernel, where it waited for global loads of positions and
-// functors).
+// and (IL: when they fit) the ions in LDS and takes electrons part, part + parts, ...; a wave takes four of a
+// pair's knots at a time, so a position is read once for the four, and the workgroup's waves deal these
+// fours out among themselves, whatever electrons have the pairs.
+// Bound: vector arithmetic, (N + M) image distances per knot; with few walkers the latency of a wave's
+// fours (13 us each at NiO-64).  NiO-64 FP32, 128 walkers, 396k knots: 0.68 ms; one walker, 3k knots: 26 us
+// (0.91 ms and 163 us with an electron's pairs on one wave and workgroups of 16 electrons).
 constexpr int kNlppTake = 4;
 template <typename T>
 __host__ __device__ inline size_t nlpp_jastrow_lds(int N, int M) {
-  return sizeof(double) * 3 * (size_t)(N + M) + sizeof(Functor<T>) * (kMaxSpecies + 2) + sizeof(Cell<T>) + 64;
+  return sizeof(double) * 3 * (size_t)(N + M) + sizeof(Functor<T>) * (kMaxSpecies + 2) + sizeof(Cell<T>) +
+         sizeof(int) * (size_t)N + 64;
 }
 template <typename T, bool J3, bool IL>
 __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, const double* spheres, int maxp,
@@ -1545,6 +1547,14 @@ __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, co
   double* sI = sR + 3 * N;
   Functor<T>* sFn = (Functor<T>*)(smem + ((sizeof(double) * 3 * (size_t)(N + (IL ? M : 0)) + 15) & ~(size_t)15));
   Cell<T>* sCell = (Cell<T>*)(sFn + kMaxSpecies + 2);
+  int* sNp = (int*)(sCell + 1);   // listed pairs of the workgroup's electrons
+  const int ne = (N - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
+  bool any = false;
+  for (int i = tid; i < ne; i += nt) {
+    sNp[i] = min(npairs[(size_t)w * N + blockIdx.x + (size_t)i * gridDim.x], maxp);
+    any = any || sNp[i] > 0;
+  }
+  if (!__syncthreads_or(any)) return;
   for (int i = tid; i < 3 * N; i += nt) sR[i] = B.R[(size_t)w * 3 * N + i];
   if constexpr (IL)
     for (int i = tid; i < 3 * M; i += nt) sI[i] = S.ions[i];
@@ -1560,67 +1570,72 @@ __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, co
     const T u = functor_v(f, in ? r : f.rcut * T(0.5));
     return in ? (double)u : 0.0;
   };
-  for (int e = blockIdx.x * nw + wid; e < N; e += gridDim.x * nw) {
+  constexpr int kFours = kNlppKnots / kNlppTake;
+  int turn = __builtin_amdgcn_readfirstlane(wid);   // fours to the wave's next one
+  for (int i = 0; i < ne; ++i) {
+    const int nf = __builtin_amdgcn_readfirstlane(sNp[i]) * kFours;   // the same on every lane
+    if (turn >= nf) {
+      turn -= nf;
+      continue;
+    }
+    const int e = blockIdx.x + i * gridDim.x;
     const size_t idx = (size_t)w * N + e;
-    const int np = min(npairs[idx], maxp);
-    if (np == 0) continue;
     const size_t o = (size_t)w * 5 * N + e;
     const double j1o = (double)B.J1[o], j2o = (double)B.J2[o] + (J3 ? (double)B.J3[o] : 0.0);
     const bool up = e < n;
-    for (int p = 0; p < np; ++p) {
-      const size_t item = idx * maxp + p;
-      const double* q = near + item * 4;
+    for (; turn < nf; turn += nw) {
+      const int p = turn / kFours, k0 = (turn - p * kFours) * kNlppTake;
+      const double* q = near + (idx * maxp + p) * 4;
       const double d = q[0], ox = sR[e] + q[1], oy = sR[N + e] + q[2], oz = sR[2 * N + e] + q[3];
-      for (int k0 = 0; k0 < kNlppKnots; k0 += kNlppTake) {
-        const double* sp = spheres + ((size_t)w * kNlppKnots + k0) * 3;
-        double px[kNlppTake], py[kNlppTake], pz[kNlppTake], v[2 * kNlppTake];
+      const double* sp = spheres + ((size_t)w * kNlppKnots + k0) * 3;
+      double px[kNlppTake], py[kNlppTake], pz[kNlppTake], v[2 * kNlppTake];
+#pragma unroll
+      for (int k = 0; k < kNlppTake; ++k) {
+        px[k] = d * sp[3 * k] + ox;
+        py[k] = d * sp[3 * k + 1] + oy;
+        pz[k] = d * sp[3 * k + 2] + oz;
+        v[k] = v[kNlppTake + k] = 0.0;
+      }
+      for (int ci = lane; ci < M; ci += 64) {
+        const Functor<T>& f = sFn[S.species[ci]];
+        if (f.ncoef == 0) continue;
+        double x, y, z;
+        if constexpr (IL) x = sI[ci], y = sI[M + ci], z = sI[2 * M + ci];
+        else x = S.ions[ci], y = S.ions[M + ci], z = S.ions[2 * M + ci];
+#pragma unroll
+        for (int k = 0; k < kNlppTake; ++k) v[k] += value(f, (T)(x - px[k]), (T)(y - py[k]), (T)(z - pz[k]));
+      }
+      for (int j = lane; j < N; j += 64) {
+        const Functor<T>& f = sFn[kMaxSpecies + (((j < n) == up) ? 0 : 1)];
+        const double x = sR[j], y = sR[N + j], z = sR[2 * N + j];
+        const bool self = j == e;
 #pragma unroll
         for (int k = 0; k < kNlppTake; ++k) {
-          px[k] = d * sp[3 * k] + ox;
-          py[k] = d * sp[3 * k + 1] + oy;
-          pz[k] = d * sp[3 * k + 2] + oz;
-          v[k] = v[kNlppTake + k] = 0.0;
-        }
-        for (int ci = lane; ci < M; ci += 64) {
-          const Functor<T>& f = sFn[S.species[ci]];
-          if (f.ncoef == 0) continue;
-          double x, y, z;
-          if constexpr (IL) x = sI[ci], y = sI[M + ci], z = sI[2 * M + ci];
-          else x = S.ions[ci], y = S.ions[M + ci], z = S.ions[2 * M + ci];
-#pragma unroll
-          for (int k = 0; k < kNlppTake; ++k) v[k] += value(f, (T)(x - px[k]), (T)(y - py[k]), (T)(z - pz[k]));
-        }
-        for (int j = lane; j < N; j += 64) {
-          const Functor<T>& f = sFn[kMaxSpecies + (((j < n) == up) ? 0 : 1)];
-          const double x = sR[j], y = sR[N + j], z = sR[2 * N + j];
-          const bool self = j == e;
-#pragma unroll
-          for (int k = 0; k < kNlppTake; ++k) {
-            const double u = value(f, (T)(x - px[k]), (T)(y - py[k]), (T)(z - pz[k]));
-            v[kNlppTake + k] += self ? 0.0 : u;
-          }
-        }
-        if constexpr (J3)
-#pragma unroll
-          for (int k = 0; k < kNlppTake; ++k)
-            v[kNlppTake + k] += j3_value_partial<T>(S, B, C, w, e, px[k], py[k], pz[k], lane, 64);
-        wave_sums_rows<2 * kNlppTake>(v);
-        // row r (lanes 16r ..) holds sums 2r and 2r + 1: the J1 sums of knots k in rows 0 and 1, the J2
-        // sums in rows 2 and 3; lanes 0 and 16 take their knots' J2 sums from lanes 32 and 48
-        const double b0 = __shfl(v[0], (lane & 31) + 32), b1 = __shfl(v[1], (lane & 31) + 32);
-        if ((lane & 15) == 0 && lane < 32) {
-          double* out = ratios + ((size_t)first[idx] + p) * kNlppKnots + k0 + (lane >> 4) * 2;
-          out[0] = (j1o - v[0]) + (j2o - b0);
-          out[1] = (j1o - v[1]) + (j2o - b1);
+          const double u = value(f, (T)(x - px[k]), (T)(y - py[k]), (T)(z - pz[k]));
+          v[kNlppTake + k] += self ? 0.0 : u;
         }
       }
+      if constexpr (J3)
+#pragma unroll
+        for (int k = 0; k < kNlppTake; ++k)
+          v[kNlppTake + k] += j3_value_partial<T>(S, B, C, w, e, px[k], py[k], pz[k], lane, 64);
+      wave_sums_rows<2 * kNlppTake>(v);
+      // row r (lanes 16r ..) holds sums 2r and 2r + 1: the J1 sums of knots k in rows 0 and 1, the J2
+      // sums in rows 2 and 3; lanes 0 and 16 take their knots' J2 sums from lanes 32 and 48
+      const double b0 = __shfl(v[0], (lane & 31) + 32), b1 = __shfl(v[1], (lane & 31) + 32);
+      if ((lane & 15) == 0 && lane < 32) {
+        double* out = ratios + ((size_t)first[idx] + p) * kNlppKnots + k0 + (lane >> 4) * 2;
+        out[0] = (j1o - v[0]) + (j2o - b0);
+        out[1] = (j1o - v[1]) + (j2o - b1);
+      }
     }
+    turn -= nf;
   }
 }
 
 // Determinant part and the ratios, in the order of the knot list: LK lanes of a wave take a knot and
 // hold all of its 64 stencil points' sums for Q 16-byte orbital groups each (no LDS, no barriers).
-// A wave takes `take` runs of 64 / LK consecutive knots at a time.  The stencil rows come from L2 and
+// A wave takes `take` runs of 64 / LK consecutive knots at a time (units null: in the order of the pairs).  The stencil rows come from L2 and
 // the CU's cache (cached loads: neighbouring knots want them).
 // Bound: L2 and L1 bandwidth of the stencils, 64 rows per knot.  NiO-64, 128 walkers, 396k knots:
 // 1.59 ms in FP32 (24 TB/s of stencil bytes, 2.3 GB from HBM); the whole evaluation's kernels 2.7 ms against 7.4 for a
@@ -1641,7 +1656,8 @@ __global__ __launch_bounds__(256) void k_nlpp_ratios(SysP<T> S, BatchP<T> B, con
   for (int rn = lo + (int)(blockIdx.x >> 3) * nw + wid; rn < hi; rn = walk_next(rn, per, hi))
     for (int t = 0; t < take; ++t) {
       const unsigned at = (unsigned)(rn * run) + (unsigned)(t * KW + slot);   // past INT_MAX at a full list's end
-      const int u = units[min(at, (unsigned)nu - 1u)];   // past the end: the last knot again, not stored
+      const int last = (int)min(at, (unsigned)nu - 1u);   // past the end: the last knot again, not stored
+      const int u = units != nullptr ? units[last] : last;
       int w, e;
       double pt[3];
       nlpp_point(S, B, spheres, maxp, near, items, u, w, e, pt);

@@ -1,11 +1,13 @@
 """Shapes that the prepared systems do not have, on the paths that are chosen by size: SPO rows ordered by
 place (orbital counts that are not whole 16-byte vectors, a skewed cell, the largest orbital count of the path),
-the flush inside the move kernel (tile counts below those its forms hold), and virtual ratios at the sizes where
-the pinned block grows and where the call leaves it."""
+the flush inside the move kernel (tile counts below those its forms hold), virtual ratios at the sizes where the
+pinned block grows and where the call leaves it, and NonLocalPP's knots ordered by place and not."""
+import dataclasses
+
 import numpy as np
 import pytest
 
-from miniqmc_amd import qmcx
+from miniqmc_amd import nlpp, qmcx, systems
 from test_gpu_sm_update import orbital_system
 
 pytestmark = pytest.mark.gpu
@@ -77,3 +79,39 @@ def test_virtual_ratio_sizes(walkers, points):
     part = max(1, 2000 // walkers)
     for o in range(0, points, part):
         np.testing.assert_array_equal(whole[:, o:o + part], wb.flex_evaluate_ratios(5, pts[:, o:o + part]))
+
+
+def fine_grid_system(n, ng):
+    """orbital_system with a spline table of the given grid."""
+    base = orbital_system(n)
+    return dataclasses.replace(base, ng=ng, coefs=systems.spline_coefficients(ng, n, base.npad, n))
+
+
+@pytest.mark.parametrize("precision", [qmcx.FP64, qmcx.FP32])
+@pytest.mark.parametrize("n,ng", [(33, (60, 61, 59)), (100, (40, 41, 42))])
+def test_nlpp_order(n, ng, precision):
+    """NonLocalPP of walkers enough for their knots to be ordered by grid cell, in a table past 24 MB, against
+    the same walkers one at a time, whose knots are not: the same ratios."""
+    sysd = fine_grid_system(n, ng)
+    dev = qmcx.System(sysd, precisions=(precision,))
+    row = sysd.npad * (4 if precision == qmcx.FP32 else 8)
+    assert np.prod(np.array(ng) + 3) * row > 24e6
+    rmax = 1.1
+    per_walker = 2 * 4 * np.pi / 3 * rmax**3 / abs(np.linalg.det(sysd.lattice)) * 2 * n * 12 * 64 * row
+    walkers = int(512e6 / per_walker) + 1
+    assert per_walker < 256e6 < walkers * per_walker   # the call's own rule
+    R = np.random.default_rng(n).random((walkers, 2 * n, 3)) @ sysd.lattice
+    spheres = nlpp.NonLocalPP(sysd, rmax=rmax, seed=n).randomize_walkers(walkers)
+
+    def evaluate(lo, hi):
+        wb = qmcx.WalkerBatch(dev, hi - lo, delay_rank=1, precision=precision)
+        wb.set_positions(R[lo:hi])
+        wb.evaluate_log()
+        return wb.nlpp_evaluate(rmax, spheres[lo:hi], max_pairs=4)
+
+    ratios, pairs = evaluate(0, walkers)
+    assert pairs.sum() > 0
+    for w in range(0, walkers, max(1, walkers // 12)):
+        one, count = evaluate(w, w + 1)
+        np.testing.assert_array_equal(count[0], pairs[w])
+        np.testing.assert_array_equal(one[0], ratios[w])
