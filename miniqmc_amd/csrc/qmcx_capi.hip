@@ -717,9 +717,15 @@ GridBlocks grid_blocks(const qmcx_system_s* s) {
 }
 
 // evaluateLog's electrons are ordered by place when there are this many (the four ordering launches take
-// about 30 us, as long as the rows of a few thousand electrons), and their stencils cover the grid
-// this many times over (else there is little to share).  Batches that keep FP64 Slater rows are not: their
-// FP32 rows would round differently.
+// about 30 us, as long as the rows of a few thousand electrons), their stencils cover the grid this many
+// times over (else there is little to share), and rows are long enough: the ordered kernel gives an
+// electron's row of 16-byte groups the lanes of one wave or more.
+//   * From 40 groups on: 200 orbitals FP32 (52 groups, a table of 2.3 MB), 24 walkers 601 us ordered and 758 not;
+//     NiO-16 FP64 (48 groups) 326 and 377 at 48 walkers.
+//   * From 24 groups on with tables past 8 MB: NiO-16 FP32 (24 groups, 16 MB) 293 and 311 us at 48 walkers; but
+//     NiO-8 FP64 (24 groups, 7.6 MB) 237 and 228 at 91, and 50 orbitals in FP64 (32 groups, 1.4 MB) 272 and 243 at 100.
+//   * Not below: NiO-8 FP32 (12 groups) 680 and 566 us at 512 walkers, 7 orbitals (4 groups) 283 and 185 at 700.
+// Batches that keep FP64 Slater rows are not ordered: their FP32 rows would round differently.
 constexpr long long kOrderPoints = 8192, kOrderReuse = 4;
 
 template <typename T>
@@ -734,7 +740,9 @@ int launch_spo_rows(qmcx_batch_t b) {
   const SysP<T> S = s->params<T>();
   const BatchP<T> B = b->params<T>();
   const long long np = (long long)s->N * b->W;
-  bool ordered = B.A64 == nullptr && nq <= kOrderedThreads && np >= kOrderPoints && np <= INT_MAX &&
+  const double table = (s->ng[0] + 3.0) * (s->ng[1] + 3.0) * (s->ng[2] + 3.0) * s->npad * sizeof(T);
+  bool ordered = B.A64 == nullptr && nq <= kOrderedThreads && (nq >= 40 || (nq >= 24 && table > 8e6)) &&
+                 np >= kOrderPoints && np <= INT_MAX &&
                  np * 64 >= kOrderReuse * (long long)s->ng[0] * s->ng[1] * s->ng[2];
   if (ordered && !b->order) {
     if (hipMalloc(&b->order, sizeof(int) * (2 * (size_t)np + 2 * (size_t)kBlockKeys)) == hipSuccess) {
@@ -798,20 +806,27 @@ int launch_gl(qmcx_batch_t b, bool record) {
 template <typename T>
 int evaluate_log_impl(qmcx_batch_t b) {
   const qmcx_system_s* s = b->sys;
-  // the Jastrow sums need the positions only: they run on the recompute stream beside the SPO rows.
+  // the Jastrow sums need the positions only: they run on the recompute stream beside the SPO rows (with 24
+  // electrons or more; the events cost up to 20 us: 14 electrons take 88 us so and 70 on one stream, 28 take 90 and
+  // 90, 96 take 142 and 182).
   // Without a three-body Jastrow (whose sums read every electron's ion mask) a walker's electrons are
   // split over workgroups of 128: at NiO-64 with 128 walkers 0.70 ms by a workgroup per walker
-  HIPCHK(hipEventRecord(b->ev_start, b->stream));
-  HIPCHK(hipStreamWaitEvent(b->aux, b->ev_start, 0));
+  const bool beside = s->N >= 24;
+  const hipStream_t jst = beside ? b->aux : b->stream;
+  if (beside) {
+    HIPCHK(hipEventRecord(b->ev_start, b->stream));
+    HIPCHK(hipStreamWaitEvent(b->aux, b->ev_start, 0));
+  }
   // positions, reduction scratch, functors, the minimum-image cell and the J3 ion masks
   const size_t lds = jastrow_init_lds<T>(s->N, s->has_j3 ? s->mw : 0);
   const dim3 jgrid(b->W, b->j3 ? 1 : (s->N + 127) / 128), jblock(b->j3 ? 1024 : 128);
-  hipLaunchKernelGGL(k_jastrow_init<T>, jgrid, jblock, lds, b->aux, s->params<T>(), b->params<T>());
+  hipLaunchKernelGGL(k_jastrow_init<T>, jgrid, jblock, lds, jst, s->params<T>(), b->params<T>());
   HIPCHK(hipGetLastError());
-  HIPCHK(hipEventRecord(b->ev_gl, b->aux));
+  if (beside) HIPCHK(hipEventRecord(b->ev_gl, b->aux));
   int rc = launch_spo_rows<T>(b);
   if (!rc && launch_lu_batch<T>(b)) rc = QMCX_ERR_HIP;
-  HIPCHK(hipStreamWaitEvent(b->stream, b->ev_gl, 0));   // after an error too: later work may write what the sums read
+  // after an error too: later work may write what the sums read
+  if (beside) HIPCHK(hipStreamWaitEvent(b->stream, b->ev_gl, 0));
   if (rc) return rc;
   HIPCHK(hipMemsetAsync(b->ndelay, 0, sizeof(int) * b->W * 2 * b->nch, b->stream));
   return launch_gl<T>(b, false);
@@ -2425,7 +2440,8 @@ int qmcx_nlpp_evaluate(qmcx_batch_t b, double rmax, const double* spheres, int m
     auto rat = [&](size_t o) { return (double*)(b->nl_io.as<char>() + (o / chunk % 2) * bytes); };
     auto fetch = [&](size_t o) -> int {
       const size_t m = std::min(chunk, listed - o);
-      HIPCHK(hipMemcpyAsync(rat(o) + chunk * kNlppKnots, b->nl_items + o, sizeof(int) * m, hipMemcpyDeviceToHost, b->stream));
+      HIPCHK(hipMemcpyAsync(rat(o) + chunk * kNlppKnots, b->nl_items + o, sizeof(int) * m, hipMemcpyDeviceToHost,
+                            b->stream));
       HIPCHK(hipMemcpyAsync(rat(o), b->nl_out + o * kNlppKnots, sizeof(double) * m * kNlppKnots, hipMemcpyDeviceToHost,
                             b->stream));
       return 0;

@@ -1638,8 +1638,8 @@ __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, co
 // A wave takes `take` runs of 64 / LK consecutive knots at a time (units null: in the order of the pairs).  The stencil rows come from L2 and
 // the CU's cache (cached loads: neighbouring knots want them).
 // Bound: L2 and L1 bandwidth of the stencils, 64 rows per knot.  NiO-64, 128 walkers, 396k knots:
-// 1.59 ms in FP32 (24 TB/s of stencil bytes, 2.3 GB from HBM); the whole evaluation's kernels 2.7 ms against 7.4 for a
-// workgroup per knot in the order of ions, whose stencils came from HBM (38 GB at 5.2 TB/s).
+// 1.52 ms in FP32 (26 TB/s of stencil bytes, 2.3 GB from HBM); the whole evaluation's kernels 2.4 ms against
+// 7.4 for a workgroup per knot in the order of ions, whose stencils came from HBM (38 GB at 5.2 TB/s).
 template <typename T, int LK, int Q>
 __global__ __launch_bounds__(256) void k_nlpp_ratios(SysP<T> S, BatchP<T> B, const double* spheres, int maxp,
                                                      const double* near, const int* items, const int* units,

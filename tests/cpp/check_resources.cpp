@@ -121,8 +121,8 @@ struct Model {
 // evaluateLog of enough electrons for them to be ordered by place: without the memory for that it evaluates
 // them in their own order, and an error leaves no work of the side stream behind
 static void evaluate_log() {
-  Model m(48, 10);
-  const int W = 91;
+  Model m(160, 10);
+  const int W = 26;
   const std::vector<double> R = m.positions(W);
   for (int precision : {QMCX_FP64, QMCX_FP32}) {
     qmcx_batch_t a, b;

@@ -13,16 +13,25 @@ from test_gpu_sm_update import orbital_system
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("precision,n,walkers", [(qmcx.FP32, 33, 130), (qmcx.FP32, 50, 90), (qmcx.FP32, 7, 600),
-                                                 (qmcx.FP32, 384, 12), (qmcx.FP64, 33, 130), (qmcx.FP64, 129, 40),
-                                                 (qmcx.FP64, 512, 9)])
-def test_ordered_rows(precision, n, walkers):
+def fine_grid_system(n, ng):
+    """orbital_system with a spline table of the given grid."""
+    base = orbital_system(n)
+    return dataclasses.replace(base, ng=ng, coefs=systems.spline_coefficients(ng, n, base.npad, n))
+
+
+@pytest.mark.parametrize("precision,n,walkers,ng", [
+    (qmcx.FP32, 161, 30, None), (qmcx.FP32, 250, 18, None), (qmcx.FP32, 384, 12, None), (qmcx.FP32, 97, 50, (28, 29, 30)),
+    (qmcx.FP64, 83, 60, None), (qmcx.FP64, 129, 40, None), (qmcx.FP64, 512, 9, None), (qmcx.FP64, 50, 110, (32, 30, 31))])
+def test_ordered_rows(precision, n, walkers, ng):
     """A batch whose electrons are ordered against the same walkers in batches of fewer than 8192 electrons."""
-    sysd = orbital_system(n)
+    sysd = orbital_system(n) if ng is None else fine_grid_system(n, ng)
     dev = qmcx.System(sysd, precisions=(precision,))
     R = np.random.default_rng(n).random((walkers, 2 * n, 3)) @ sysd.lattice
-    # the call's own rule: 8192 electrons or more whose 64-point stencils cover the grid four times
+    # the call's own rule: 8192 electrons or more whose 64-point stencils cover the grid four times, and rows
+    # of 40 groups of 16 bytes (24 with a table past 8 MB)
+    row = sysd.npad * (4 if precision == qmcx.FP32 else 8)
     assert walkers * 2 * n >= 8192 and 64 * walkers * 2 * n >= 4 * np.prod(sysd.ng)
+    assert row >= 40 * 16 or (row >= 24 * 16 and np.prod(np.array(sysd.ng) + 3) * row > 8e6)
     part = 8191 // (2 * n)
 
     def evaluate(r):
@@ -79,12 +88,6 @@ def test_virtual_ratio_sizes(walkers, points):
     part = max(1, 2000 // walkers)
     for o in range(0, points, part):
         np.testing.assert_array_equal(whole[:, o:o + part], wb.flex_evaluate_ratios(5, pts[:, o:o + part]))
-
-
-def fine_grid_system(n, ng):
-    """orbital_system with a spline table of the given grid."""
-    base = orbital_system(n)
-    return dataclasses.replace(base, ng=ng, coefs=systems.spline_coefficients(ng, n, base.npad, n))
 
 
 @pytest.mark.parametrize("precision", [qmcx.FP64, qmcx.FP32])
