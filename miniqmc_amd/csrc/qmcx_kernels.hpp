@@ -1394,9 +1394,9 @@ __global__ __launch_bounds__(1024) void k_virtual_ratios(SysP<T> S, BatchP<T> B,
 // image, ion - electron as the BA table's displacement), counts them in npairs[w][e] (the full
 // count, also beyond maxp) and lists the first maxp: near[item][4] = distance, displacement of item =
 // (w*N + e)*maxp + p, items[pos] = item in the order of arrival (an electron's pairs from first[w][e] on),
-// cnt[0] = listed pairs.  Knot k of a pair sits at dist * spheres[w][k] + displ + r_e (NonLocalPP.hpp:133; every walker has its own
-// randomly rotated knots, one rotation per walker and evaluation as the reference's per-mover
-// NonLocalPP::randomize, NonLocalPP.hpp:100-113, miniqmc.cpp:470).
+// cnt[0] = listed pairs.  Knot k of a pair sits at dist * spheres[w][k] + displ + r_e (NonLocalPP.hpp:133;
+// every walker has its own randomly rotated knots, one rotation per walker and evaluation as the reference's
+// per-mover NonLocalPP::randomize, NonLocalPP.hpp:100-113, miniqmc.cpp:470).
 // k_nlpp_keys, k_key_offsets and k_key_scatter order all the knots (unit = pos * 12 + knot) by the
 // block of spline grid cells they fall in (left out when there are few, or the table is small).
 // k_nlpp_jastrow: the Jastrow exponents of the listed pairs' knots into ratios[pos][12], walker by walker
@@ -1521,6 +1521,39 @@ __global__ __launch_bounds__(256) void k_key_scatter(const int* cnt, int per, co
     units[atomicAdd(kcur + ukey[u], 1)] = u;
 }
 
+// j3_value_partial of the lanes of one wave, with the walker's positions and the ions in LDS: the lanes look
+// for the ions in reach of the point, then sum over the electrons ion by ion, in the same order.  NiO-16, 32
+// walkers, FP32: 129 us the whole Jastrow kernel, 277 with every ion looked at by all lanes from memory.
+template <typename T>
+__device__ inline double j3_value_wave(const SysP<T>& S, const BatchP<T>& B, const Cell<T>& C, int w, int e, double x,
+                                       double y, double z, const double* sR, const double* sI, int lane) {
+  const int N = S.N, n = S.n, M = S.M, mw = S.mw;
+  const unsigned long long* mk = B.j3mask + (size_t)w * N * mw;
+  const bool up = e < n;
+  T dx, dy, dz;
+  double acc = 0.0;
+  for (int I0 = 0; I0 < M; I0 += 64) {
+    const int Il = min(I0 + lane, M - 1);
+    const T Ll = S.j3[2 * S.species[Il]].L;
+    const T rl = min_image(C, (T)(sI[Il] - x), (T)(sI[M + Il] - y), (T)(sI[2 * M + Il] - z), T(-1), dx, dy, dz);
+    unsigned long long near = __ballot(I0 + lane < M && Ll > T(0) && rl < Ll);
+    for (; near != 0; near &= near - 1) {
+      const int I = I0 + __ffsll((long long)near) - 1, sp = S.species[I], wd = I >> 6;
+      const unsigned long long bit = 1ull << (I & 63);
+      const double ix = sI[I], iy = sI[M + I], iz = sI[2 * M + I];
+      const T rxI = min_image(C, (T)(ix - x), (T)(iy - y), (T)(iz - z), T(-1), dx, dy, dz);
+      for (int k = lane; k < N; k += 64) {
+        if (k == e || !(mk[(size_t)k * mw + wd] & bit)) continue;
+        const double kx = sR[k], ky = sR[N + k], kz = sR[2 * N + k];
+        const T rkI = min_image(C, (T)(ix - kx), (T)(iy - ky), (T)(iz - kz), T(-1), dx, dy, dz);
+        const T rxk = min_image(C, (T)(kx - x), (T)(ky - y), (T)(kz - z), T(-1), dx, dy, dz);
+        acc += (double)poly3_v(S.j3[2 * sp + (((k < n) == up) ? 0 : 1)], rxk, rxI, rkI);
+      }
+    }
+  }
+  return acc;
+}
+
 // J1, J2 (and J3) exponents of every listed pair's knots: sums at the electron's position (kept by the
 // moves) less those at the knot (OneBodyJastrow.h:136-140, TwoBodyJastrow.h:103-107,
 // ThreeBodyJastrow.h:262-273).  grid (parts, W): a workgroup stages its walker's positions, functors, cell
@@ -1618,7 +1651,7 @@ __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, co
       if constexpr (J3)
 #pragma unroll
         for (int k = 0; k < kNlppTake; ++k)
-          v[kNlppTake + k] += j3_value_partial<T>(S, B, C, w, e, px[k], py[k], pz[k], lane, 64);
+          v[kNlppTake + k] += j3_value_wave<T>(S, B, C, w, e, px[k], py[k], pz[k], sR, sI, lane);
       wave_sums_rows<2 * kNlppTake>(v);
       // row r (lanes 16r ..) holds sums 2r and 2r + 1: the J1 sums of knots k in rows 0 and 1, the J2
       // sums in rows 2 and 3; lanes 0 and 16 take their knots' J2 sums from lanes 32 and 48
@@ -1635,8 +1668,8 @@ __global__ __launch_bounds__(256) void k_nlpp_jastrow(SysP<T> S, BatchP<T> B, co
 
 // Determinant part and the ratios, in the order of the knot list: LK lanes of a wave take a knot and
 // hold all of its 64 stencil points' sums for Q 16-byte orbital groups each (no LDS, no barriers).
-// A wave takes `take` runs of 64 / LK consecutive knots at a time (units null: in the order of the pairs).  The stencil rows come from L2 and
-// the CU's cache (cached loads: neighbouring knots want them).
+// A wave takes `take` runs of 64 / LK consecutive knots at a time (units null: in the order of the pairs).  The
+// stencil rows come from L2 and the CU's cache (cached loads: neighbouring knots want them).
 // Bound: L2 and L1 bandwidth of the stencils, 64 rows per knot.  NiO-64, 128 walkers, 396k knots:
 // 1.52 ms in FP32 (26 TB/s of stencil bytes, 2.3 GB from HBM); the whole evaluation's kernels 2.4 ms against
 // 7.4 for a workgroup per knot in the order of ions, whose stencils came from HBM (38 GB at 5.2 TB/s).
