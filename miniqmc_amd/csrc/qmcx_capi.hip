@@ -635,8 +635,12 @@ constexpr int kPropWorkgroups = 1024;
 // against device buffers and pageable copies.  NiO-8 FP32, 64 walkers: 33 us against 44 at 2112 points, 51
 // against 53 at 5120, 61 against 64 at 7680, 97 against 97 at 16384, 184 against 150 at 32768; one walker of NiO-8
 // in FP64: 24 against 37 at 16 points.  (A process's first couple of hundred pageable copies take 20 to 120 us
-// longer.)  A batch's pinned block is 512 KB at most.
+// longer.)
 constexpr size_t kVirtualInPlace = 16384;
+// points up to which a larger call's copies go through pinned memory (2 MB): 93 us against 99 with pageable ones at
+// 17280 points, 145 against 146 at 32768, 268 against 268 at 65536, 408 against 393 at 96000; but 534 against 186 at 30720
+// while the runtime's pageable copies are slow
+constexpr size_t kVirtualPinned = 65536;
 // virtual positions per walker in one qmcx_flex_evaluate_ratios call (grid x dimension)
 constexpr int kMaxVirtualPoints = 1 << 16;
 // pairs whose ratios a NonLocalPP evaluation has in pinned memory at a time, in each of two buffers (6.5 MB):
@@ -2351,14 +2355,18 @@ int qmcx_flex_evaluate_ratios(qmcx_batch_t b, int iel, int nvp, const double* vp
     return b->prec == QMCX_FP32 ? launch_virtual_ratios<float>(b, iel, nvp, pos, out)
                                 : launch_virtual_ratios<double>(b, iel, nvp, pos, out);
   };
-  if (np <= kVirtualInPlace) {
-    // a small call: the kernel reads the points and writes the ratios in pinned host memory
+  double* pos = nullptr;   // the points and ratios in pinned host memory
+  double* out = nullptr;
+  if (np <= kVirtualPinned) {
     size_t most = 2048;   // 64 KB, more when a call needs it
     while (most < np) most *= 2;
     if (int rc = b->vr_io.need(sizeof(double) * 4 * most)) return rc;
-    double* pos = b->vr_io.as<double>();
-    double* out = pos + 3 * most;
+    pos = b->vr_io.as<double>();
+    out = pos + 3 * most;
     std::memcpy(pos, vpos, sizeof(double) * 3 * np);
+  }
+  if (np <= kVirtualInPlace) {
+    // a small call: the kernel reads the points and writes the ratios there
     if (int rc = launch(pos, out)) return rc;
     HIPCHK(hipStreamSynchronize(b->stream));
     std::memcpy(ratios, out, sizeof(double) * np);
@@ -2374,10 +2382,11 @@ int qmcx_flex_evaluate_ratios(qmcx_batch_t b, int iel, int nvp, const double* vp
     HIPCHK(hipMalloc(&b->vr_out, sizeof(double) * (size_t)nvp * b->W));
     b->vr_cap = nvp;
   }
-  HIPCHK(hipMemcpyAsync(b->vr_pos, vpos, sizeof(double) * 3 * np, hipMemcpyHostToDevice, b->stream));
+  HIPCHK(hipMemcpyAsync(b->vr_pos, pos ? pos : vpos, sizeof(double) * 3 * np, hipMemcpyHostToDevice, b->stream));
   if (int rc = launch(b->vr_pos, b->vr_out)) return rc;
-  HIPCHK(hipMemcpyAsync(ratios, b->vr_out, sizeof(double) * np, hipMemcpyDeviceToHost, b->stream));
+  HIPCHK(hipMemcpyAsync(out ? out : ratios, b->vr_out, sizeof(double) * np, hipMemcpyDeviceToHost, b->stream));
   HIPCHK(hipStreamSynchronize(b->stream));
+  if (out) std::memcpy(ratios, out, sizeof(double) * np);
   return 0;
 }
 

@@ -74,7 +74,7 @@ def test_flush_tiles(n, delay):
 
 
 @pytest.mark.parametrize("walkers,points", [(1, 2047), (1, 2049), (1, 16384), (1, 16385), (7, 300), (7, 2340),
-                                            (7, 2341), (64, 256), (64, 257)])
+                                            (7, 2341), (64, 256), (64, 257), (64, 1024), (64, 1025)])
 def test_virtual_ratio_sizes(walkers, points):
     """A call's ratios are those of its points in small calls, whatever the sizes before it."""
     sysd = orbital_system(33)
