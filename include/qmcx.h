@@ -175,7 +175,8 @@ int qmcx_batch_set_graph(qmcx_batch_t b, int enable);
  *   + WaveFunction::flex_ratioGrad (src/Particle/ParticleSet.cpp:296-346, src/QMCWaveFunctions/WaveFunction.cpp:343-417):
  *   displ[nw][3] -> ratio[nw], grad_now[nw][3], grad_new[nw][3] (outputs may be NULL); no state changes.
  * qmcx_flex_accept_restore: WaveFunction::flex_acceptrestoreMove + ParticleSet::acceptMove/rejectMove
- *   (WaveFunction.cpp:418-485, miniqmc_sync_move.cpp:496-505) for the same electron, accepted[nw] != 0.
+ *   (WaveFunction.cpp:418-485, miniqmc_sync_move.cpp:496-505) for the same electron, accepted[nw] != 0.  A move
+ *   whose ratio is NaN is rejected in any case.  QMCX_ERR_STATE when ratio_grad of that electron did not come before.
  * qmcx_flex_complete_updates: WaveFunction::flex_completeUpdates (WaveFunction.cpp:486-499): the delayed rows
  *   that flex moves left pending reach the inverse (DiracDeterminant.cpp:294-321).  With delay rank k > 1 an
  *   accepted flex move is a pending delayed row of its walker until the walker has k of them, as in

@@ -637,9 +637,9 @@ constexpr int kPropWorkgroups = 1024;
 // in FP64: 24 against 37 at 16 points.  (A process's first couple of hundred pageable copies take 20 to 120 us
 // longer.)
 constexpr size_t kVirtualInPlace = 16384;
-// points up to which a larger call's copies go through pinned memory (2 MB): 93 us against 99 with pageable ones at
-// 17280 points, 145 against 146 at 32768, 268 against 268 at 65536, 408 against 393 at 96000; but 534 against 186 at 30720
-// while the runtime's pageable copies are slow
+// points up to which a larger call's copies go through pinned memory (2 MB): 93 us against 99 with pageable ones
+// at 17280 points, 145 against 146 at 32768, 268 against 268 at 65536, 408 against 393 at 96000; while the runtime's
+// pageable copies are slow they take 534 at 30720
 constexpr size_t kVirtualPinned = 65536;
 // virtual positions per walker in one qmcx_flex_evaluate_ratios call (grid x dimension)
 constexpr int kMaxVirtualPoints = 1 << 16;
@@ -1411,11 +1411,9 @@ static int launch_nlpp_ratios(qmcx_batch_t b, int maxp, int take, const int* uni
 template <typename T>
 static bool nlpp_ordered(const qmcx_batch_t b, double rmax, int maxp) {
   const qmcx_system_s* s = b->sys;
-  double inv[9];
-  inv3(s->lattice, inv);
-  const double volume = std::fabs(1.0 / (inv[0] * (inv[4] * inv[8] - inv[5] * inv[7]) -
-                                         inv[1] * (inv[3] * inv[8] - inv[5] * inv[6]) +
-                                         inv[2] * (inv[3] * inv[7] - inv[4] * inv[6])));
+  const double* a = s->lattice;
+  const double volume = std::fabs(a[0] * (a[4] * a[8] - a[5] * a[7]) - a[1] * (a[3] * a[8] - a[5] * a[6]) +
+                                  a[2] * (a[3] * a[7] - a[4] * a[6]));
   const double pairs = std::min((double)maxp, s->nions * 4.18879 * rmax * rmax * rmax / volume);
   const double row = (double)s->npad * sizeof(T);
   const double stencils = pairs * b->W * s->N * kNlppKnots * 64 * row;
